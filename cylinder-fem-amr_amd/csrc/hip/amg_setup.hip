@@ -496,6 +496,80 @@ __global__ void k_prolongator_rows(int n, const int* __restrict__ ap_rp, const i
     if (pass == 0) cnt[i] = out;
 }
 
+// y = X - omega D^-1 y on y's pattern (which contains X's), one thread per row merging the two
+// sorted rows
+__global__ void k_smooth_product(int n, const int* __restrict__ x_rp, const int* __restrict__ x_ci,
+                                 const double* __restrict__ x_v, const int* __restrict__ y_rp,
+                                 const int* __restrict__ y_ci, double* __restrict__ y_v,
+                                 const double* __restrict__ dinv, double omega) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double f = omega * dinv[i];
+    int a = x_rp[i];
+    const int a1 = x_rp[i + 1];
+    for (int k = y_rp[i]; k < y_rp[i + 1]; ++k) {
+        const int j = y_ci[k];
+        while (a < a1 && x_ci[a] < j) ++a;
+        const double x = a < a1 && x_ci[a] == j ? x_v[a] : 0.0;
+        y_v[k] = x - f * y_v[k];
+    }
+}
+
+// ---- The cycle of a small level as a dense matrix ------------------------------------------------
+// Row i of the operator of two steps from zero: 2 omega d_i on the diagonal minus omega d_i a_ij
+// omega d_j
+__global__ void __launch_bounds__(BLOCK)
+k_dense_two_steps(int n, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ v,
+                  const double* __restrict__ dinv, double omega, double* __restrict__ out) {
+    const int i = blockIdx.x;
+    double* row = out + (size_t)i * n;
+    const double di = omega * dinv[i];
+    for (int j = threadIdx.x; j < n; j += BLOCK) row[j] = j == i ? di + di : 0.0;
+    __syncthreads();
+    for (int k = rp[i] + threadIdx.x; k < rp[i + 1]; k += BLOCK) {
+        const int j = ci[k];
+        const double y = -v[k] * (omega * dinv[j]);
+        row[j] = j == i ? di + di * (1.0 + y) : di * y;
+    }
+}
+
+// f[j, i] = sum_l coarse[j, l] w[i, l]: the coarse row j in LDS, one thread per fine row i
+__global__ void __launch_bounds__(BLOCK)
+k_dense_coarse_wt(int rows, int cols, const int* __restrict__ w_rp, const int* __restrict__ w_ci,
+                  const double* __restrict__ w_v, const double* __restrict__ coarse, double* __restrict__ f) {
+    extern __shared__ double crow[];
+    const int j = blockIdx.y;
+    for (int l = threadIdx.x; l < cols; l += BLOCK) crow[l] = coarse[(size_t)j * cols + l];
+    __syncthreads();
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= rows) return;
+    double s = 0.0;
+    for (int k = w_rp[i]; k < w_rp[i + 1]; ++k) s += w_v[k] * crow[w_ci[k]];
+    f[(size_t)j * rows + i] = s;
+}
+
+// y[i, :] = x[i, :] + omega d_i (e_i - sum_j a_ij x[j, :]) (+ sum_l w_il f[l, :]): one smoothing step
+// on every column of the identity, a workgroup per row and 256 columns, the row's entries uniform
+__global__ void __launch_bounds__(BLOCK)
+k_dense_sweep(int n, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ v,
+              const double* __restrict__ dinv, double omega, const double* __restrict__ x,
+              const int* __restrict__ w_rp, const int* __restrict__ w_ci, const double* __restrict__ w_v,
+              const double* __restrict__ f, double* __restrict__ y) {
+    const int i = blockIdx.y, c = blockIdx.x * BLOCK + threadIdx.x;
+    if (c >= n) return;
+    double s = 0.0;
+#pragma unroll 4
+    for (int k = rp[i]; k < rp[i + 1]; ++k) s += v[k] * x[(size_t)ci[k] * n + c];
+    double t = x[(size_t)i * n + c] + omega * dinv[i] * ((c == i ? 1.0 : 0.0) - s);
+    if (f) {
+        double u = 0.0;
+#pragma unroll 4
+        for (int k = w_rp[i]; k < w_rp[i + 1]; ++k) u += w_v[k] * f[(size_t)w_ci[k] * n + c];
+        t += u;
+    }
+    y[(size_t)i * n + c] = t;
+}
+
 // ---- R = P^T (csr_transpose: entries of each column in ascending row order) ----------------------
 // ---- transpose (host csr_transpose: the entries of a column in ascending row order) ----------------
 // A stable radix sort of the entries by column, from their CSR order (rows ascending), lists
@@ -776,6 +850,36 @@ int cfa_amg_prolongator(int n, const int* ap_rp, const int* ap_ci, const double*
     if ((pass == 0 && !cnt) || (pass == 1 && (!p_rp || !p_ci || !p_v))) return CFA_E_ARG;
     hipLaunchKernelGGL(k_prolongator_rows, dim3(blocks(n)), dim3(BLOCK), 0, as_stream(stream), n, ap_rp, ap_ci, ap_v,
                        agg, p0v, dinv, omega, pass, cnt, p_rp, p_ci, p_v);
+    return launch_status();
+}
+
+int cfa_amg_smooth_product(int n, const int* x_rp, const int* x_ci, const double* x_v, const int* y_rp,
+                           const int* y_ci, double* y_v, const double* dinv, double omega, cfa_stream_t stream) {
+    if (n < 0) return CFA_E_ARG;
+    if (n == 0) return CFA_OK;
+    if (!x_rp || !x_ci || !x_v || !y_rp || !y_ci || !y_v || !dinv) return CFA_E_ARG;
+    hipLaunchKernelGGL(k_smooth_product, dim3(blocks(n)), dim3(BLOCK), 0, as_stream(stream), n, x_rp, x_ci, x_v, y_rp,
+                       y_ci, y_v, dinv, omega);
+    return launch_status();
+}
+
+int cfa_amg_dense_level(int rows, const int* a_rp, const int* a_ci, const double* a_v, const double* dinv,
+                        double omega, const int* w_rp, const int* w_ci, const double* w_v, int cols,
+                        const double* coarse, double* f, double* tmp, double* out, cfa_stream_t stream) {
+    if (rows < 0 || cols < 0 || rows > CFA_AMG_DENSE_MAX || cols > CFA_AMG_DENSE_MAX) return CFA_E_ARG;
+    if (rows == 0) return CFA_OK;
+    if (!a_rp || !a_ci || !a_v || !dinv || !tmp || !out) return CFA_E_ARG;
+    if (cols > 0 && (!w_rp || !w_ci || !w_v || !coarse || !f)) return CFA_E_ARG;
+    const hipStream_t s = as_stream(stream);
+    const unsigned cb = (unsigned)blocks(rows);
+    hipLaunchKernelGGL(k_dense_two_steps, dim3(rows), dim3(BLOCK), 0, s, rows, a_rp, a_ci, a_v, dinv, omega, out);
+    if (cols > 0)
+        hipLaunchKernelGGL(k_dense_coarse_wt, dim3(cb, cols), dim3(BLOCK), (size_t)cols * sizeof(double), s, rows, cols,
+                           w_rp, w_ci, w_v, coarse, f);
+    hipLaunchKernelGGL(k_dense_sweep, dim3(cb, rows), dim3(BLOCK), 0, s, rows, a_rp, a_ci, a_v, dinv, omega, out,
+                       nullptr, nullptr, nullptr, nullptr, tmp);
+    hipLaunchKernelGGL(k_dense_sweep, dim3(cb, rows), dim3(BLOCK), 0, s, rows, a_rp, a_ci, a_v, dinv, omega, tmp, w_rp,
+                       w_ci, w_v, cols > 0 ? f : nullptr, out);
     return launch_status();
 }
 

@@ -108,6 +108,15 @@ __global__ void k_jacobi_init(int n, T omega, const T* __restrict__ dinv, const 
     if (i < n) x[i] = omega * dinv[i] * b[i];
 }
 
+// The lane's share of one row of a dense product, its loads eight at a time ahead of their uses
+template <typename T>
+__device__ __forceinline__ double dense_row(int n, const double* __restrict__ a, const T* __restrict__ x, int lane) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int j = lane; j < n; j += WAVE) s += a[j] * (double)x[j];
+    return s;
+}
+
 // y = Ainv x with the dense coarse inverse, one wavefront per row (src/cfa/linalg.cuh:929-937);
 // FP64 arithmetic also when x and y are FP32 (the coarse solve stays FP64 in the mixed cycle)
 template <typename T = double>
@@ -116,10 +125,7 @@ k_dense_matvec(int n, const double* __restrict__ A, const T* __restrict__ x, T* 
                const int* __restrict__ state) {
     if (halted(state)) return;
     const int i = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
-    double s = 0.0;
-    if (i < n)
-        for (int j = lane; j < n; j += WAVE) s += A[(size_t)i * n + j] * (double)x[j];
-    s = wave_sum(s);
+    const double s = i < n ? wave_sum(dense_row(n, A + (size_t)i * n, x, lane)) : 0.0;
     if (i < n && lane == 0) y[i] = (T)s;
 }
 
@@ -131,6 +137,8 @@ template <> struct Lv<double> {
     __host__ __device__ static const double* r(const cfa_amg_level_t& L) { return L.r_v; }
     __host__ __device__ static const double* dinv(const cfa_amg_level_t& L) { return L.dinv; }
     __host__ __device__ static const double* sv(const cfa_amg_level_t& L) { return L.s_v; }
+    static const double* w(const cfa_amg_level_t& L) { return L.w_v; }
+    static const double* q(const cfa_amg_level_t& L) { return L.q_v; }
     __host__ __device__ static double* x(const cfa_amg_level_t& L) { return L.x; }
     __host__ __device__ static double* b(const cfa_amg_level_t& L) { return L.b; }
     __host__ __device__ static double* res(const cfa_amg_level_t& L) { return L.r; }
@@ -144,6 +152,8 @@ template <> struct Lv<float> {
     __host__ __device__ static const float* r(const cfa_amg_level_t& L) { return L.r_v32; }
     __host__ __device__ static const float* dinv(const cfa_amg_level_t& L) { return L.dinv32; }
     __host__ __device__ static const float* sv(const cfa_amg_level_t& L) { return L.s_v32; }
+    static const float* w(const cfa_amg_level_t& L) { return L.w_v32; }
+    static const float* q(const cfa_amg_level_t& L) { return L.q_v32; }
     __host__ __device__ static float* x(const cfa_amg_level_t& L) { return L.x32; }
     __host__ __device__ static float* b(const cfa_amg_level_t& L) { return L.b32; }
     __host__ __device__ static float* res(const cfa_amg_level_t& L) { return L.r32; }
@@ -766,6 +776,256 @@ k_sell_from_zero_check(int positions, const int* __restrict__ sp, const int* __r
     if (row < 0) return;
     const double x0 = omega * dinv[row] * b[row];
     y[row] = x0 + omega * dinv[row] * (b[row] - s);
+}
+
+// ---- The coupled V(2,2) cycle --------------------------------------------------------------------
+// With G = I - omega D^-1 A and W = G^2 P (set up once per hierarchy), a level's cycle is
+//   x1 = two steps from zero on b,   b_coarse = W^T b,   x = two steps from x1 on b + W e_coarse:
+// the restricted residual P^T (b - A x1) is P^T (G^T)^2 b for a symmetric A, and the two steps after
+// the correction x1 + P e are linear, so they give two steps from x1 plus G^2 P e. Nothing the level
+// smooths is then on the way down or up: its smoothing runs in the launches that carry the coarser
+// levels, and a level costs two launches (one down, one up) instead of six. A cycle on the adaptive
+// meshes is bound by its launches (3-4 us each below level 0, whatever their size), not by bytes;
+// W has about as many entries per row as A, so the bytes moved are those of the residual,
+// restriction and prolongation it replaces.
+//
+// One launch of the descent (stage l): from-zero steps of level l, the coarse right-hand side of
+// level l + 1 (or the dense bottom product), and the first step of level l - 1, each on its own
+// range of workgroups. RowSet: CSR rows with 2^shift lanes per row.
+template <typename T, typename B>
+struct RowSet {
+    int blocks, rows, shift;
+    const int* rp; const int* ci; const T* v;
+    const T* x; const B* b; const T* dinv; T omega; T* y;
+};
+template <typename T, typename B, typename B2>
+struct CoupledStage {
+    RowSet<T, B> zero;     // y = two steps from zero on b
+    RowSet<T, B> mul;      // y = v b, or the dense product
+    RowSet<T, B2> step;    // y = x + omega dinv (b - A x)
+    const double* dense;   // mul is this dense matrix (rows x rows) times x
+    int sell;              // which of the two level-0 slots runs on the sliced-ELL copy: 0 zero, 2 step
+    const int* s_sp; const int* s_row; const int* s_ci; const T* s_v;
+    const double* prr; int nb_rr; double* sc; int* st; int* status;   // the residual test (prr set)
+};
+
+// row_entries and group_sum with 2^shift lanes per row: the same entries in the same order
+template <typename T, typename F>
+__device__ __forceinline__ T lanes_row_sum(const int* __restrict__ ci, const T* __restrict__ v, int k0, int k1, int lane,
+                                           int shift, F xv) {
+    const int tpr = 1 << shift;
+    T s = 0;
+    for (int k = k0 + lane; k < k1; k += ROW_UNROLL * tpr) {
+        int c[ROW_UNROLL];
+        T a[ROW_UNROLL];
+#pragma unroll
+        for (int u = 0; u < ROW_UNROLL; ++u) {
+            const int idx = k + u * tpr;
+            const bool ok = idx < k1;
+            c[u] = ok ? ci[idx] : 0;
+            a[u] = ok ? v[idx] : T(0);
+        }
+#pragma unroll
+        for (int u = 0; u < ROW_UNROLL; ++u) s += a[u] * xv(c[u]);
+    }
+    for (int o = tpr >> 1; o > 0; o >>= 1) s += __shfl_down(s, o, tpr);
+    return s;
+}
+
+// The iteration's residual test as fp_residual_test, with the state word read beside the partials:
+// one pair of barriers. True (in every thread of every block) when the solve goes on.
+__device__ __forceinline__ bool residual_test_running(const double* prr, int nb_rr, double* sc, int* st, int* status,
+                                                      double* lds, int* lds_state) {
+    double v = 0.0;
+    for (int k = threadIdx.x; k < nb_rr; k += BLOCK) v += prr[k];
+    if (threadIdx.x == 0) *lds_state = st[0];
+    v = wave_sum(v);
+    if ((threadIdx.x & (WAVE - 1)) == 0) lds[threadIdx.x / WAVE] = v;
+    __syncthreads();
+    double rr = 0.0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / WAVE; ++w) rr += lds[w];
+    if (*lds_state != ST_RUNNING) return false;
+    const double r_norm = sqrt(rr);
+    const bool done = r_norm < sc[S_TOL] * sc[S_BNORM];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc[S_RNORM] = r_norm;
+        sc[S_REL] = r_norm / sc[S_BNORM];
+        const int it = st[2];
+        if (done) {
+            st[0] = ST_CONVERGED;
+            st[1] = it;
+        }
+        publish(status, it, done ? ST_CONVERGED : ST_RUNNING);
+    }
+    return !done;
+}
+
+// MAXL, G: the sliced-ELL copy of level 0 (MAXL 0: none in this stage). Every value is computed
+// before the residual test's barrier, so the test's reduction runs beside the row loads.
+template <int MAXL, int G, typename T, typename B, typename B2>
+__global__ void __launch_bounds__(BLOCK)
+k_coupled_stage(CoupledStage<T, B, B2> a) {
+    __shared__ double lds[BLOCK / WAVE];
+    __shared__ int lds_state;
+    int blk = blockIdx.x;
+    T out = 0;
+    T* dst = nullptr;
+    int row = -1;
+    const int sv = a.st ? a.st[0] : ST_RUNNING;
+    if (blk < a.mul.blocks) {
+        const RowSet<T, B>& r = a.mul;
+        if (a.dense) {
+            const int i = (blk * BLOCK + threadIdx.x) / WAVE, lane = threadIdx.x & (WAVE - 1);
+            if (i < r.rows) {
+                const double s = wave_sum(dense_row(r.rows, a.dense + (size_t)i * r.rows, r.x, lane));
+                if (lane == 0) { out = (T)s; row = i; }
+            }
+        } else {
+            const int g = blk * BLOCK + threadIdx.x, i = g >> r.shift, lane = g & ((1 << r.shift) - 1);
+            const int k0 = i < r.rows ? r.rp[i] : 0, k1 = i < r.rows ? r.rp[i + 1] : 0;
+            const B* __restrict__ b = r.b;
+            out = lanes_row_sum(r.ci, r.v, k0, k1, lane, r.shift, [&](int j) { return (T)b[j]; });
+            if (i < r.rows && lane == 0) row = i;
+        }
+        dst = r.y;
+    } else if ((blk -= a.mul.blocks) < a.zero.blocks) {
+        const RowSet<T, B>& r = a.zero;
+        const B* __restrict__ b = r.b;
+        const T* __restrict__ dinv = r.dinv;
+        const T omega = r.omega;
+        const auto x0 = [&](int j) { return omega * dinv[j] * (T)b[j]; };
+        T s = 0;
+        bool done = false;
+        if constexpr (MAXL > 0) {
+            if (a.sell == 0) {
+                const int p = blk * BLOCK + threadIdx.x;
+                if (p < sell_positions(r.rows)) {
+                    int base, len;
+                    (void)sell_slot(a.s_sp, a.s_row, p, nullptr, row, base, len);
+                    s = sell_row_sum<MAXL, G, false>(a.s_ci, a.s_v, base, len, x0);
+                }
+                done = true;
+            }
+        }
+        if (!done) {
+            const int g = blk * BLOCK + threadIdx.x, i = g >> r.shift, lane = g & ((1 << r.shift) - 1);
+            const int k0 = i < r.rows ? r.rp[i] : 0, k1 = i < r.rows ? r.rp[i + 1] : 0;
+            s = lanes_row_sum(r.ci, r.v, k0, k1, lane, r.shift, x0);
+            if (i < r.rows && lane == 0) row = i;
+        }
+        if (row >= 0) {
+            const T bi = (T)b[row];
+            const T xi = omega * dinv[row] * bi;
+            out = xi + omega * dinv[row] * (bi - s);
+        }
+        dst = r.y;
+    } else {
+        blk -= a.zero.blocks;
+        const RowSet<T, B2>& r = a.step;
+        const T* __restrict__ x = r.x;
+        T s = 0;
+        bool done = false;
+        if constexpr (MAXL > 0) {
+            if (a.sell == 2) {
+                const int p = blk * BLOCK + threadIdx.x;
+                if (p < sell_positions(r.rows)) {
+                    int base, len;
+                    (void)sell_slot(a.s_sp, a.s_row, p, nullptr, row, base, len);
+                    s = sell_row_sum<MAXL, G, false>(a.s_ci, a.s_v, base, len, [&](int j) { return x[j]; });
+                }
+                done = true;
+            }
+        }
+        if (!done) {
+            const int g = blk * BLOCK + threadIdx.x, i = g >> r.shift, lane = g & ((1 << r.shift) - 1);
+            const int k0 = i < r.rows ? r.rp[i] : 0, k1 = i < r.rows ? r.rp[i + 1] : 0;
+            s = lanes_row_sum(r.ci, r.v, k0, k1, lane, r.shift, [&](int j) { return x[j]; });
+            if (i < r.rows && lane == 0) row = i;
+        }
+        if (row >= 0) out = x[row] + r.omega * r.dinv[row] * ((T)r.b[row] - s);
+        dst = r.y;
+    }
+    bool running = sv == ST_RUNNING;
+    if (a.prr) running = residual_test_running(a.prr, a.nb_rr, a.sc, a.st, a.status, lds, &lds_state);
+    if (running && row >= 0) dst[row] = out;
+}
+
+// The ascent of a level: second step and coarse correction, y = x + omega dinv (b - A x) + W e
+template <typename T, typename B>
+__global__ void __launch_bounds__(BLOCK)
+k_coupled_up(RowSet<T, B> r, const int* __restrict__ w_rp, const int* __restrict__ w_ci, const T* __restrict__ w_v,
+             const T* __restrict__ e, const int* __restrict__ state) {
+    const int g = blockIdx.x * BLOCK + threadIdx.x, i = g >> r.shift, lane = g & ((1 << r.shift) - 1);
+    const int sv = state ? state[0] : ST_RUNNING;
+    const bool in = i < r.rows;
+    const int a0 = in ? r.rp[i] : 0, a1 = in ? r.rp[i + 1] : 0, w0 = in ? w_rp[i] : 0, w1 = in ? w_rp[i + 1] : 0;
+    if (sv != ST_RUNNING) return;
+    const T* __restrict__ x = r.x;
+    const T s = lanes_row_sum(r.ci, r.v, a0, a1, lane, r.shift, [&](int j) { return x[j]; });
+    const T c = lanes_row_sum(w_ci, w_v, w0, w1, lane, r.shift, [&](int j) { return e[j]; });
+    if (in && lane == 0) r.y[i] = x[i] + r.omega * r.dinv[i] * ((T)r.b[i] - s) + c;
+}
+
+// The ascent of level 0 into the FP64 output with the r.z block partials. The entries of RB
+// consecutive rows are one contiguous run of each CSR matrix: the workgroup loads it coalesced, every
+// lane's entries and gathers in flight together, leaves the products in LDS, and one lane per row
+// adds its row's in CSR order. (With lanes per row the loads of a wavefront scatter over its rows:
+// 2 lanes took 7.3 us for the step alone on 115k rows, 20 us on 460k.) A run longer than the LDS
+// tile takes further passes.
+template <int RB, typename T>
+__global__ void __launch_bounds__(BLOCK)
+k_coupled_up_dot(int rows, const int* __restrict__ a_rp, const int* __restrict__ a_ci, const T* __restrict__ a_v,
+                 const T* __restrict__ x, const double* __restrict__ r, const T* __restrict__ dinv, T omega,
+                 const int* __restrict__ w_rp, const int* __restrict__ w_ci, const T* __restrict__ w_v,
+                 const T* __restrict__ e, double* __restrict__ y, double* __restrict__ part,
+                 const int* __restrict__ state) {
+    constexpr int U = RB / 32, CAP = U * BLOCK;
+    __shared__ T pa[CAP], pw[CAP];
+    __shared__ double lds[BLOCK / WAVE];
+    if (state && state[0] != ST_RUNNING) return;
+    const int tid = threadIdx.x;
+    double contrib = 0.0;
+    for (int r0 = blockIdx.x * RB; r0 < rows; r0 += gridDim.x * RB) {
+        const int r1 = r0 + RB < rows ? r0 + RB : rows, row = r0 + tid;
+        const int a0 = a_rp[r0], a1 = a_rp[r1], w0 = w_rp[r0], w1 = w_rp[r1];
+        const bool own = tid < RB && row < rows;
+        const int ra0 = own ? a_rp[row] : 0, ra1 = own ? a_rp[row + 1] : 0;
+        const int rw0 = own ? w_rp[row] : 0, rw1 = own ? w_rp[row + 1] : 0;
+        const double ri = own ? r[row] : 0.0;
+        const T xi = own ? x[row] : T(0), di = own ? dinv[row] : T(0);
+        T sa = 0, sw = 0;
+        for (int ta = a0, tw = w0; ta < a1 || tw < w1; ta += CAP, tw += CAP) {
+            int ca[U], cw[U];
+            T va[U], vw[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int ka = ta + u * BLOCK + tid, kw = tw + u * BLOCK + tid;
+                ca[u] = ka < a1 ? a_ci[ka] : 0;
+                va[u] = ka < a1 ? a_v[ka] : T(0);
+                cw[u] = kw < w1 ? w_ci[kw] : 0;
+                vw[u] = kw < w1 ? w_v[kw] : T(0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                pa[u * BLOCK + tid] = va[u] * x[ca[u]];
+                pw[u * BLOCK + tid] = vw[u] * e[cw[u]];
+            }
+            __syncthreads();
+            for (int k = max(ra0, ta), k1 = min(ra1, ta + CAP); k < k1; ++k) sa += pa[k - ta];
+            for (int k = max(rw0, tw), k1 = min(rw1, tw + CAP); k < k1; ++k) sw += pw[k - tw];
+            __syncthreads();
+        }
+        if (own) {
+            const double z = (double)(xi + omega * di * ((T)ri - sa) + sw);
+            y[row] = z;
+            contrib += ri * z;
+        }
+    }
+    if (part) {
+        contrib = block_sum(contrib, lds);
+        if (tid == 0) part[blockIdx.x] = contrib;
+    }
 }
 
 // The positions of one window's rows (a workgroup per window of SELL_WINDOW rows): each row's rank
@@ -1530,6 +1790,163 @@ void level_from_zero_check_launch(const cfa_amg_level_t& L, const double* b, dou
     });
 }
 
+// The level index of the cycle's bottom: the dense level when there is one, else past the last level
+int bottom_level(const cfa_amg_t* amg) { return amg->dense ? amg->dense_level : amg->n_levels; }
+
+// Level l and every level above the bottom carry the coupled transfers, for the V(2,2) cycle
+bool coupled_from(const cfa_amg_t* amg, int l) {
+    if (amg->smooth_steps != 2) return false;
+    for (int k = l; k < bottom_level(amg); ++k)
+        if (!amg->levels[k].w_rp) return false;
+    return l < bottom_level(amg);
+}
+
+// right-hand side, result, size and matrix of the dense product at the cycle's bottom
+template <typename T>
+struct Bottom {
+    int n;
+    const double* m;
+    T* b;
+    T* x;
+};
+template <typename T>
+Bottom<T> bottom_of(const cfa_amg_t* amg) {
+    if (amg->dense) {
+        const cfa_amg_level_t& L = amg->levels[amg->dense_level];
+        return {L.rows, amg->dense, Lv<T>::b(L), Lv<T>::x(L)};
+    }
+    return {amg->coarse_n, amg->coarse_inv, Lv<T>::cb(amg), Lv<T>::cx(amg)};
+}
+
+int log2_of(int tpr) {
+    int s = 0;
+    while ((1 << s) < tpr && s < 6) ++s;
+    return s;
+}
+
+// workgroups of rows with 2^shift lanes each
+int row_blocks(int rows, int shift) { return blocks_for((long long)rows << shift); }
+
+template <typename T, typename B, typename B2>
+void coupled_stage_launch(const CoupledStage<T, B, B2>& a, const cfa_amg_level_t* sell, hipStream_t s) {
+    const int grid = a.zero.blocks + a.mul.blocks + a.step.blocks;
+    if (grid == 0) return;
+    auto go = [&](auto m, auto g) {
+        constexpr int M = decltype(m)::value, G = decltype(g)::value;
+        hipLaunchKernelGGL((k_coupled_stage<M, G, T, B, B2>), dim3(grid), dim3(BLOCK), 0, s, a);
+    };
+    if (!sell) {
+        go(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
+        return;
+    }
+    auto with_g = [&](auto m) {
+        if (sell->tpr_a == 1) go(m, std::integral_constant<int, 1>{});
+        else if (sell->tpr_a == 2) go(m, std::integral_constant<int, 2>{});
+        else go(m, std::integral_constant<int, 4>{});
+    };
+    if (sell->s_len <= 8) with_g(std::integral_constant<int, 8>{});
+    else if (sell->s_len <= 12) with_g(std::integral_constant<int, 12>{});
+    else with_g(std::integral_constant<int, 16>{});
+}
+
+// Stage l of the descent, from level l0 (B0: the type of level l0's right-hand side b0, FP64 on level
+// 0): from-zero steps of level l, its coarse right-hand side or the dense product, the first step of
+// level l - 1.
+template <typename T, typename B, typename B2, typename B0>
+void coupled_stage(const cfa_amg_t* amg, int l0, int l, const B0* b0, const int* st, hipStream_t s, PrecHooks* hk) {
+    CoupledStage<T, B, B2> a;
+    std::memset(&a, 0, sizeof(a));
+    const cfa_amg_level_t* sell = nullptr;
+    auto use_sell = [&](const cfa_amg_level_t& L, int slot) {
+        sell = &L;
+        a.sell = slot;
+        a.s_sp = L.s_sp; a.s_row = L.s_row; a.s_ci = L.s_ci; a.s_v = Lv<T>::sv(L);
+        return blocks_for(sell_positions(L.rows));
+    };
+    a.sell = -1;
+    a.st = const_cast<int*>(st);
+    const int bottom = bottom_level(amg);
+    if (l == bottom) {
+        const Bottom<T> e = bottom_of<T>(amg);
+        a.dense = e.m;
+        a.mul.rows = e.n;
+        a.mul.x = e.b;
+        a.mul.y = e.x;
+        a.mul.blocks = blocks_for((long long)e.n * WAVE);
+    } else {
+        const cfa_amg_level_t& L = amg->levels[l];
+        const B* b;
+        if constexpr (std::is_same<B, B0>::value) b = l == l0 ? b0 : (const B*)(const void*)Lv<T>::b(L);
+        else b = (const B*)(const void*)Lv<T>::b(L);
+        const int sh = log2_of(L.tpr_a), shq = log2_of(L.tpr_q);
+        a.zero = {row_blocks(L.rows, sh), L.rows, sh, L.a_rp, L.a_ci, Lv<T>::a(L), nullptr, b, Lv<T>::dinv(L),
+                  (T)L.omega, Lv<T>::x(L)};
+        if (L.s_sp) a.zero.blocks = use_sell(L, 0);
+        T* cb = l + 1 < bottom ? Lv<T>::b(amg->levels[l + 1]) : bottom_of<T>(amg).b;
+        a.mul = {row_blocks(L.cols, shq), L.cols, shq, L.q_rp, L.q_ci, Lv<T>::q(L), nullptr, b, nullptr, T(0), cb};
+        if (l == 0 && hk && hk->prr) {
+            a.prr = hk->prr; a.nb_rr = hk->nb_rr; a.sc = hk->sc; a.st = hk->st_w; a.status = hk->status;
+        }
+    }
+    if (l > l0) {
+        const cfa_amg_level_t& F = amg->levels[l - 1];
+        const B2* b;
+        if constexpr (std::is_same<B2, B0>::value) b = l - 1 == l0 ? b0 : (const B2*)(const void*)Lv<T>::b(F);
+        else b = (const B2*)(const void*)Lv<T>::b(F);
+        const int sh = log2_of(F.tpr_a);
+        a.step = {row_blocks(F.rows, sh), F.rows, sh, F.a_rp, F.a_ci, Lv<T>::a(F), Lv<T>::x(F), b, Lv<T>::dinv(F),
+                  (T)F.omega, Lv<T>::ax(F)};
+        if (F.s_sp) a.step.blocks = use_sell(F, 2);
+    }
+    coupled_stage_launch(a, sell, s);
+}
+
+// The coupled cycle from level l0 with right-hand side b0 (FP64 on level 0, also in the FP32 cycle);
+// the result in level l0's x buffer, or on level 0 in the FP64 `out`, with the r.z partials.
+template <typename T, typename B0>
+T* coupled_vcycle(const cfa_amg_t* amg, int l0, const B0* b0, double* out, const int* st, hipStream_t s,
+                  PrecHooks* hk) {
+    const int bottom = bottom_level(amg);
+    for (int l = l0; l <= bottom; ++l) {
+        if (l == l0) coupled_stage<T, B0, T, B0>(amg, l0, l, b0, st, s, hk);
+        else if (l == l0 + 1) coupled_stage<T, T, B0, B0>(amg, l0, l, b0, st, s, hk);
+        else coupled_stage<T, T, T, B0>(amg, l0, l, b0, st, s, hk);
+    }
+    for (int l = bottom - 1; l >= l0; --l) {
+        const cfa_amg_level_t& L = amg->levels[l];
+        const T* e = l + 1 < bottom ? Lv<T>::x(amg->levels[l + 1]) : bottom_of<T>(amg).x;
+        if constexpr (std::is_same<B0, double>::value) {
+            if (out && l == 0) {
+                // rows per workgroup: one pass of at most RED_BLOCKS workgroups as long as that takes no
+                // more than 256 rows each
+                auto go = [&](auto rb) {
+                    constexpr int RB = decltype(rb)::value;
+                    const int nb = std::min(blocks_for(L.rows, RB), RED_BLOCKS);
+                    hipLaunchKernelGGL((k_coupled_up_dot<RB, T>), dim3(nb), dim3(BLOCK), 0, s, L.rows, L.a_rp, L.a_ci,
+                                       Lv<T>::a(L), Lv<T>::ax(L), b0, Lv<T>::dinv(L), (T)L.omega, L.w_rp, L.w_ci,
+                                       Lv<T>::w(L), e, out, hk ? hk->dot_part : nullptr, st);
+                    if (hk && hk->dot_part) hk->dot_blocks = nb;
+                };
+                if (L.rows <= 64 * RED_BLOCKS) go(std::integral_constant<int, 64>{});
+                else if (L.rows <= 128 * RED_BLOCKS) go(std::integral_constant<int, 128>{});
+                else go(std::integral_constant<int, 256>{});
+                return nullptr;
+            }
+        }
+        const int sh = log2_of(L.tpr_a);
+        auto up = [&](auto* b) {
+            using B = typename std::remove_cv<typename std::remove_pointer<decltype(b)>::type>::type;
+            RowSet<T, B> r = {row_blocks(L.rows, sh), L.rows, sh, L.a_rp, L.a_ci, Lv<T>::a(L), Lv<T>::ax(L), b,
+                              Lv<T>::dinv(L), (T)L.omega, Lv<T>::x(L)};
+            hipLaunchKernelGGL((k_coupled_up<T, B>), dim3(r.blocks), dim3(BLOCK), 0, s, r, L.w_rp, L.w_ci, Lv<T>::w(L),
+                               e, st);
+        };
+        if (l == l0) up(b0);
+        else up((const T*)Lv<T>::b(L));
+    }
+    return Lv<T>::x(amg->levels[l0]);
+}
+
 // One V-cycle (src/cfa/linalg.cuh:1184-1206) for level l with right-hand side b, in FP64 or FP32
 // (T). Each level's x / ax buffers form a ping-pong pair; the function returns the buffer holding
 // the level's iterate. On level 0 the last smoothing step writes straight into the FP64 `out`
@@ -1537,6 +1954,8 @@ void level_from_zero_check_launch(const cfa_amg_level_t& L, const double* b, dou
 template <typename T>
 T* vcycle(const cfa_amg_t* amg, int l, const T* b, double* out, const double* rdot, const int* st, hipStream_t s,
           PrecHooks* hk = nullptr) {
+    if (coupled_from(amg, l) && (l > 0 || std::is_same<T, double>::value))
+        return coupled_vcycle<T, T>(amg, l, b, l == 0 ? out : nullptr, st, s, hk);
     const cfa_amg_level_t& L = amg->levels[l];
     const int n = L.rows;
     const int ss = amg->smooth_steps;
@@ -1564,17 +1983,18 @@ T* vcycle(const cfa_amg_t* amg, int l, const T* b, double* out, const double* rd
         hipLaunchKernelGGL(k_jacobi_init<T>, dim3(blocks_for(n)), dim3(BLOCK), 0, s, n, (T)L.omega, dv, b, xa, st);
     }
     level_op_launch<OP_RESID, T>(L, xa, b, nullptr, Lv<T>::res(L), st, s);
-    const bool deeper = l + 1 < amg->n_levels;
-    T* cb = deeper ? Lv<T>::b(amg->levels[l + 1]) : Lv<T>::cb(amg);
+    const bool deeper = l + 1 < bottom_level(amg);
+    const Bottom<T> bot = bottom_of<T>(amg);
+    T* cb = deeper ? Lv<T>::b(amg->levels[l + 1]) : bot.b;
     csr_op_launch<OP_SPMV, T>(L.tpr_r, L.cols, L.r_rp, L.r_ci, Lv<T>::r(L), Lv<T>::res(L), nullptr, nullptr, 0.0, cb,
                               st, s);
     const T* cx;
     if (deeper) {
         cx = vcycle<T>(amg, l + 1, Lv<T>::b(amg->levels[l + 1]), nullptr, nullptr, st, s);
     } else {
-        hipLaunchKernelGGL(k_dense_matvec<T>, dim3(blocks_for((long long)amg->coarse_n * WAVE)), dim3(BLOCK), 0, s,
-                           amg->coarse_n, amg->coarse_inv, Lv<T>::cb(amg), Lv<T>::cx(amg), st);
-        cx = Lv<T>::cx(amg);
+        hipLaunchKernelGGL(k_dense_matvec<T>, dim3(blocks_for((long long)bot.n * WAVE)), dim3(BLOCK), 0, s, bot.n, bot.m,
+                           bot.b, bot.x, st);
+        cx = bot.x;
     }
     csr_op_launch<OP_ADD, T>(L.tpr_p, n, L.p_rp, L.p_ci, Lv<T>::p(L), cx, nullptr, nullptr, 0.0, xa, st, s);
     for (int k = 0; k < ss; ++k) {
@@ -1606,8 +2026,10 @@ bool amg_valid(const cfa_amg_t* amg) {
     for (int l = 0; l < amg->n_levels; ++l) {
         const cfa_amg_level_t& L = amg->levels[l];
         if (L.s_sp && !sell_usable(L)) return false;
+        if (L.w_rp && (!L.w_ci || !L.w_v || !L.q_rp || !L.q_ci || !L.q_v)) return false;
+        if (L.w_rp && amg->use_f32 && (!L.w_v32 || !L.q_v32)) return false;
     }
-    return true;
+    return !amg->dense || (amg->dense_level >= 1 && amg->dense_level < amg->n_levels);
 }
 
 // z = V-cycle(r); with hooks, the residual test first and the r.z partials last. The FP32 cycle
@@ -1622,6 +2044,9 @@ void amg_apply_enqueue(const cfa_amg_t* amg, const double* r, double* z, const i
             hipLaunchKernelGGL(k_fp_check, dim3(1), dim3(BLOCK), 0, s, hk->prr, hk->nb_rr, hk->sc, hk->st_w, hk->status);
         hipLaunchKernelGGL(k_dense_matvec<double>, dim3(blocks_for((long long)amg->coarse_n * WAVE)), dim3(BLOCK), 0, s,
                            amg->coarse_n, amg->coarse_inv, r, z, st);
+    } else if (f32 && coupled_from(amg, 0)) {   // r is read in FP64 where the level-0 kernels use it
+        (void)coupled_vcycle<float, double>(amg, 0, r, z, st, s, hk);
+        wrote_z = true;
     } else if (f32) {
         float* b32 = amg->levels[0].b32;
         hipLaunchKernelGGL(k_to_f32_check, dim3(red_blocks(n)), dim3(BLOCK), 0, s, n, r, b32,
@@ -2030,7 +2455,8 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
         kb.add(amg != nullptr);
         if (amg) {
             kb.add(amg->n_levels); kb.add(amg->coarse_n); kb.add(amg->coarse_inv); kb.add(amg->cb); kb.add(amg->cx);
-            kb.add(amg->smooth_steps);
+            kb.add(amg->smooth_steps); kb.add(amg->cb32); kb.add(amg->cx32); kb.add(amg->use_f32);
+            kb.add(amg->dense_level); kb.add(amg->dense);
             if (amg->n_levels > 0) kb.add_bytes(amg->levels, sizeof(cfa_amg_level_t) * (size_t)amg->n_levels);
         }
         graph = iteration_graph(ws, internal_of(ws)->pcg, kb.k, two_iterations);

@@ -754,12 +754,13 @@ int AmgPreconditioner::device_level(int n, int nnz, const int* arp, const int* a
         give_back();
         return -1;
     }
+    L->omega = omega;
+    build_coupling(*L, n, na, nnz, arp, aci, av, dev_tmp_, left_max);
     phase_end(PH_GALERKIN);
     // the level's operator: the caller's matrix on level 0, the previous product after that
     if (first) upload_csr_from_device(n, nnz, arp, aci, av, L->A);
     else std::swap(L->A, dev_next_);
     L->A.tpr = csr_lanes_per_row(n, L->A.nnz);
-    L->omega = omega;
     if (first && keep_p0_host) {   // remap() reads the level-0 prolongator on the host
         P0_host.rows = n;
         P0_host.cols = na;
@@ -773,6 +774,59 @@ int AmgPreconditioner::device_level(int n, int nnz, const int* arp, const int* a
     nnz_next = dev_next_.nnz;
     phase_end(PH_DOWNLOAD);
     return 1;
+}
+
+// W = G (G P), G = I - omega D^-1 A: G P lies on the pattern of A P (A has its diagonal), W on that of
+// A (G P); Q = W^T. A level beyond the sparse products' capacity, or whose smoothing is not two steps,
+// keeps the separate residual, restriction and prolongation.
+void AmgPreconditioner::build_coupling(Level& L, int n, int cols, int nnz, const int* arp, const int* aci,
+                                       const double* av, DevCsr& AP, int left_max_row) {
+    L.has_coupling = false;
+    if (smooth_steps != 2 || n > couple_max_rows) return;
+    const cfa_stream_t s = solver_stream();
+    GPU_CHECK(cfa_amg_smooth_product(n, L.P.rp, L.P.ci, L.P.v, AP.rp, AP.ci, AP.v, L.dinv, L.omega, s));
+    const int counted = sorted_products;   // the count is of the hierarchy's own products
+    const bool ok = device_product(n, cols, nnz, arp, aci, av, AP.rp, AP.ci, AP.v, L.W, left_max_row);
+    sorted_products = counted;
+    if (!ok) return;
+    GPU_CHECK(cfa_amg_smooth_product(n, AP.rp, AP.ci, AP.v, L.W.rp, L.W.ci, L.W.v, L.dinv, L.omega, s));
+    const int w_nnz = L.W.nnz;
+    L.Q.rp.reserve(cols + 1);
+    L.Q.ci.reserve(std::max(w_nnz, 1));
+    L.Q.v.reserve(std::max(w_nnz, 1));
+    const size_t tws = cfa_csr_transpose_ws_bytes(n, cols, w_nnz);
+    d_tws_.reserve(std::max<size_t>(tws, 1));
+    GPU_CHECK(cfa_csr_transpose(n, cols, w_nnz, L.W.rp, L.W.ci, L.W.v, d_tws_, tws, L.Q.rp, L.Q.ci, L.Q.v, s));
+    L.Q.rows = cols;
+    L.Q.nnz = w_nnz;
+    L.Q.tpr = csr_lanes_per_row(cols, w_nnz);
+    L.has_coupling = true;
+}
+
+// The cycle below the first level (from level 1) of at most dense_max_rows rows as one dense matrix,
+// from the coarse inverse upwards.
+void AmgPreconditioner::build_dense() {
+    has_dense_ = false;
+    size_t m = 1;
+    while (m < levels.size() && levels[m]->A.rows > dense_max_rows) ++m;
+    if (m >= levels.size() || coarse_n <= 0 || coarse_n > CFA_AMG_DENSE_MAX) return;
+    for (size_t l = m; l < levels.size(); ++l)
+        if (!levels[l]->has_coupling || levels[l]->A.rows > CFA_AMG_DENSE_MAX) return;
+    const cfa_stream_t s = solver_stream();
+    const size_t rows = levels[m]->A.rows;
+    for (auto& d : d_dense_) d.reserve(rows * rows, 0);
+    d_dense_tmp_.reserve(rows * rows, 0);
+    const double* coarse = d_coarse_inv;
+    for (size_t l = levels.size(); l-- > m;) {
+        const Level& L = *levels[l];
+        dense_slot_ ^= 1;
+        d_dense_f_.reserve((size_t)L.Q.rows * L.A.rows, 0);
+        GPU_CHECK(cfa_amg_dense_level(L.A.rows, L.A.rp, L.A.ci, L.A.v, L.dinv, L.omega, L.W.rp, L.W.ci, L.W.v, L.Q.rows,
+                                      coarse, d_dense_f_, d_dense_tmp_, d_dense_[dense_slot_], s));
+        coarse = d_dense_[dense_slot_];
+    }
+    dense_level_ = (int)m;
+    has_dense_ = true;
 }
 
 void AmgPreconditioner::setup(int n, int nnz, const int* d_row_ptr, const int* d_col_ind, const double* d_val) {
@@ -818,6 +872,7 @@ void AmgPreconditioner::setup(int n, int nnz, const int* d_row_ptr, const int* d
     d_coarse_inv.upload(inv);
     d_cx.reserve(std::max(coarse_n, 1), 16);
     d_cb.reserve(std::max(coarse_n, 1), 16);
+    build_dense();
     refresh_view();
     dev_sync();
     phase_end(PH_COARSE);
@@ -884,6 +939,12 @@ void AmgPreconditioner::refresh_view() {
         d.s_ci = L.has_sell ? L.s_ci.ptr : nullptr;
         d.s_v = L.has_sell ? L.s_v.ptr : nullptr;
         d.s_v32 = nullptr;
+        const bool w = L.has_coupling;
+        d.tpr_w = L.W.tpr;
+        d.tpr_q = L.Q.tpr;
+        d.w_rp = w ? L.W.rp.ptr : nullptr; d.w_ci = w ? L.W.ci.ptr : nullptr; d.w_v = w ? L.W.v.ptr : nullptr;
+        d.q_rp = w ? L.Q.rp.ptr : nullptr; d.q_ci = w ? L.Q.ci.ptr : nullptr; d.q_v = w ? L.Q.v.ptr : nullptr;
+        d.w_v32 = d.q_v32 = nullptr;
     }
     if (fp32) {   // FP32 copies of the values and FP32 work vectors
         const cfa_stream_t s = solver_stream();
@@ -906,6 +967,14 @@ void AmgPreconditioner::refresh_view() {
                 GPU_CHECK(cfa_to_f32(L.s_entries, L.s_v, L.s_v32, s));
                 d.s_v32 = L.s_v32;
             }
+            if (L.has_coupling) {
+                L.W32.reserve(std::max(L.W.nnz, 1), 256);
+                L.Q32.reserve(std::max(L.Q.nnz, 1), 256);
+                GPU_CHECK(cfa_to_f32(L.W.nnz, L.W.v, L.W32, s));
+                GPU_CHECK(cfa_to_f32(L.Q.nnz, L.Q.v, L.Q32, s));
+                d.w_v32 = L.W32;
+                d.q_v32 = L.Q32;
+            }
         }
         d_cx32.reserve(std::max(coarse_n, 1), 16);
         d_cb32.reserve(std::max(coarse_n, 1), 16);
@@ -920,6 +989,8 @@ void AmgPreconditioner::refresh_view() {
     view_.cb = d_cb;
     view_.cx = d_cx;
     view_.smooth_steps = smooth_steps;
+    view_.dense_level = has_dense_ ? dense_level_ : 0;
+    view_.dense = has_dense_ ? d_dense_[dense_slot_].ptr : nullptr;
 }
 
 const cfa_amg_t* AmgPreconditioner::second_view() {
@@ -1056,6 +1127,10 @@ void AmgPreconditioner::remap(int n, int nnz, const int* d_row_ptr, const int* d
     GPU_CHECK(cfa_csr_transpose(n, cols, pn, L.P.rp, L.P.ci, L.P.v, d_tws_, tws, L.R.rp, L.R.ci, L.R.v, s));
     ensure_level_vectors(L, n);
     GPU_CHECK(cfa_inv_diag(n, L.A.rp, L.A.ci, L.A.v, 1.0e-300, L.dinv, s));
+    L.has_coupling = false;
+    if (smooth_steps == 2 && n <= couple_max_rows &&
+        device_product(n, cols, nnz, L.A.rp, L.A.ci, L.A.v, L.P.rp, L.P.ci, L.P.v, dev_tmp_, -1))
+        build_coupling(L, n, cols, nnz, L.A.rp, L.A.ci, L.A.v, dev_tmp_, -1);
     P0_host = std::move(P);
     ++remaps;
     refresh_view();

@@ -168,12 +168,20 @@ public:
         DevArray<int> s_sp, s_row, s_ci;
         DevArray<double> s_v;
         DevArray<float> s_v32;
+        // coupled transfers W = (I - omega D^-1 A)^2 P and Q = W^T (cfa_amg_level_t)
+        bool has_coupling = false;
+        DevCsr W, Q;
+        DevArray<float> W32, Q32;
     };
 
     int smooth_steps = 2;
     double theta = 0.08;
     int coarse_target = 300;
     int max_levels = 15;
+    // Levels up to this size carry the coupled transfers, the first one (from level 1) up to
+    // dense_max_rows the dense matrix of the rest of the cycle (0: none).
+    int couple_max_rows = 1 << 20;
+    int dense_max_rows = 1536;
     bool fp32 = false;   // run the cycle in FP32 (coarse solve in FP64); FP32 copies made at set-up
     // The whole set-up runs on the device, level by level (D^-1, spectral radius, aggregation,
     // P smoothing, transpose, Galerkin product); only the coarse operator comes to the host for
@@ -238,6 +246,15 @@ private:
     DevArray<unsigned char> d_tws_, d_sws_, d_aws_, d_gws_;   // transpose, scan, aggregation, sorted product
     DevArray<unsigned char> d_sell_ws_;
     DevArray<int> d_sell_info_;
+    // W and Q of a level (A in arp, aci, av) from AP = A P, which is overwritten
+    void build_coupling(Level& L, int n, int cols, int nnz, const int* arp, const int* aci, const double* av, DevCsr& AP,
+                        int left_max_row);
+    // the dense matrix of the cycle from the first small level down
+    void build_dense();
+    int dense_level_ = 0;
+    bool has_dense_ = false;
+    DevArray<double> d_dense_[2], d_dense_tmp_, d_dense_f_;
+    int dense_slot_ = 0;
     // the sliced-ELL copy of the level's operator when its rows are at most CFA_SELL_MAX_LEN long
     void build_sell(Level& L);
     DevArray<double> d_p0v_, d_x0_, d_pw_;

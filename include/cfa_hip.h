@@ -266,6 +266,14 @@ typedef struct {
      * (use_f32). */
     int s_len;
     const int* s_sp; const int* s_row; const int* s_ci; const double* s_v; const float* s_v32;
+    /* Coupled transfers of the V(2,2) cycle: W = G^2 P (rows x cols; G = I - omega D^-1 A, two
+     * smoothing steps) and Q = W^T, with w_v32, q_v32 their FP32 copies (use_f32). For a symmetric A
+     * the restricted residual after two steps from zero is Q b, and two steps from x + P e are two
+     * steps from x plus W e, so a level needs neither the residual nor its coarse correction before
+     * it smooths. NULL w_rp for none. tpr_w, tpr_q: lanes per row (powers of two up to 64). */
+    int tpr_w, tpr_q;
+    const int* w_rp; const int* w_ci; const double* w_v; const float* w_v32;
+    const int* q_rp; const int* q_ci; const double* q_v; const float* q_v32;
 } cfa_amg_level_t;
 
 /* SA-AMG hierarchy for the V(ss, ss) cycle (src/cfa/linalg.cuh:1161-1206).
@@ -282,6 +290,10 @@ typedef struct {
     int smooth_steps;
     int use_f32;
     float* cb32; float* cx32;
+    /* The cycle from level dense_level (1 <= dense_level < n_levels) down as one dense matrix of that
+     * level's rows (row-major, cfa_amg_dense_level; FP64 also in the FP32 cycle); NULL for none. */
+    int dense_level;
+    const double* dense;
 } cfa_amg_t;
 
 /* z = M^{-1} r, one V-cycle (src/cfa/linalg.cuh:1161-1169 AmgPreconditioner::apply). */
@@ -490,6 +502,19 @@ int cfa_amg_prolongator(int n, const int* ap_rp, const int* ap_ci, const double*
                         const double* p0v, const double* dinv, double omega, int pass, int* cnt, const int* p_rp,
                         int* p_ci, double* p_v, cfa_stream_t stream);
 size_t cfa_csr_transpose_ws_bytes(int rows, int cols, int nnz);
+/* cfa_amg_smooth_product (no counterpart in the reference): y holds A X on its own pattern, which
+ * contains X's (both with sorted columns, n rows); y = X - omega D^-1 y in place. Twice, from P, this
+ * gives the coupled transfer W of cfa_amg_level_t. */
+int cfa_amg_smooth_product(int n, const int* x_rp, const int* x_ci, const double* x_v, const int* y_rp,
+                           const int* y_ci, double* y_v, const double* dinv, double omega, cfa_stream_t stream);
+/* cfa_amg_dense_level (no counterpart in the reference): the V(2,2) cycle of one level as a dense
+ * matrix, out [rows x rows] = two steps from zero, two more steps, + W coarse W^T, where coarse
+ * [cols x cols] (symmetric) is the cycle of the next level or the inverse of the coarsest operator.
+ * tmp [rows x rows] and f [cols x rows] are scratch. At most CFA_AMG_DENSE_MAX rows and columns. */
+#define CFA_AMG_DENSE_MAX 4096
+int cfa_amg_dense_level(int rows, const int* a_rp, const int* a_ci, const double* a_v, const double* dinv,
+                        double omega, const int* w_rp, const int* w_ci, const double* w_v, int cols,
+                        const double* coarse, double* f, double* tmp, double* out, cfa_stream_t stream);
 /* cfa_amg_aggregate: the three-phase greedy aggregation of smoothed_prolongator (linalg.cuh:
  * 1306-1356) for the n x n CSR matrix (rp, ci, val) with inverse diagonal dinv and strength
  * threshold theta: agg [n] (aggregate of each row, numbered as the row-order loop numbers them),

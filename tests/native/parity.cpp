@@ -5,7 +5,7 @@
 // block reductions or other summation orders must match to the stated relative tolerance.
 //
 //   parity <case> [level]    case: momentum pressure correction forces indicator mms oss ilu
-//                                  spmv amg sell pcg bicgstab jacobi mixed topology outlet nvb remap reproject
+//                                  spmv amg sell coupled pcg bicgstab jacobi mixed topology outlet nvb remap reproject
 //                                  all
 //
 // Prints one line per compared quantity and exits 0 when every comparison passes.
@@ -667,6 +667,51 @@ void case_sell(Fixture& f) {
         GPU_CHECK(cfa_amg_apply(&csr_view, d_r, d_z2, f.s()));
         same_bits(f32 ? "FP32 V-cycle: sliced ELL = CSR" : "FP64 V-cycle: sliced ELL = CSR", down(d_z1, n),
                   down(d_z2, n));
+    }
+}
+
+// The coupled V(2,2) cycle (two launches per level through W = G^2 P, the small levels as one dense
+// matrix) against the cycle with separate residual, restriction and prolongation on the same
+// hierarchy: coupled from level 0, from level 1, with and without the dense matrix, FP64 and FP32.
+// FP64: about 4 levels of a few dozen rounded operations per value on operators of norm O(1): 1e-13.
+// FP32: the same count at 6e-8 each: 2e-5 (both cycles against the FP64 one).
+void case_coupled(Fixture& f) {
+    std::printf("[coupled V-cycle]\n");
+    (void)case_pressure(f, false);
+    Vec r(f.n);
+    for (auto& v : r) v = std::uniform_real_distribution<double>(-1, 1)(f.rng);
+    DevArray<double> d_r, d_z;
+    d_r.upload(r);
+    d_z.reserve(f.n);
+    struct Form {
+        const char* name;
+        int couple, dense;
+    };
+    const Form forms[] = {{"from level 0", 1 << 30, 0},
+                          {"from level 0, dense bottom", 1 << 30, 1536},
+                          {"from level 0, dense level 1", 1 << 30, CFA_AMG_DENSE_MAX},
+                          {"from level 1", f.n - 1, 0},
+                          {"from level 1, dense bottom", f.n - 1, 1536}};
+    Vec plain;
+    for (int f32 = 0; f32 < 2; ++f32) {
+        for (int k = -1; k < 5; ++k) {
+            AmgPreconditioner amg;
+            amg.fp32 = f32 == 1;
+            amg.couple_max_rows = k < 0 ? 0 : forms[k].couple;
+            amg.dense_max_rows = k < 0 ? 0 : forms[k].dense;
+            amg.setup(f.n, f.nnz, f.g.d_row_ptr, f.g.d_col_ind, f.g.d_Kp_val);
+            amg.apply(d_r, d_z);
+            const Vec z = down(d_z, f.n);
+            if (k < 0 && !f32) plain = z;
+            else if (k < 0) close_rel("FP32, not coupled", z, plain, 2e-5);
+            else close_rel(forms[k].name, z, plain, f32 ? 2e-5 : 1e-13);
+            if (k >= 0) {
+                int with = 0;
+                for (const auto& L : amg.levels) with += L->has_coupling ? 1 : 0;
+                expect(with == (int)amg.levels.size() - (forms[k].couple < f.n ? 1 : 0), "levels coupled");
+                expect((amg.view()->dense != nullptr) == (forms[k].dense > 0), "dense bottom");
+            }
+        }
     }
 }
 
@@ -1458,6 +1503,7 @@ int main(int argc, char** argv) {
         if (all || what == "spmv") case_spmv(f);
         if (all || what == "amg") case_amg(f);
         if (all || what == "sell") case_sell(f);
+        if (all || what == "coupled") case_coupled(f);
         if (all || what == "pcg") case_pcg(f);
         if (all || what == "bicgstab") case_bicgstab(f);
         if (all || what == "jacobi") case_jacobi(f);

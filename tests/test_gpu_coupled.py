@@ -1,0 +1,19 @@
+"""The coupled V-cycle through the C ABI, on the GPU (tests/native/parity.cpp):
+the cycle against the one with separate residual, restriction and prolongation (uniform levels 1, 3
+and 4: one to four smoothed levels, with the dense bottom at none, the last or the first coarse one)."""
+import subprocess
+from pathlib import Path
+
+import pytest
+
+BIN = Path(__file__).resolve().parent / "native" / "build" / "parity"
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("level", [1, 3, 4])
+def test_coupled_cycle(level):
+    print(f"[case] coupled V-cycle level {level}", flush=True)
+    r = subprocess.run([str(BIN), "coupled", str(level)], capture_output=True, text=True, timeout=120)
+    print(r.stdout)
+    assert r.returncode == 0 and "ALL PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-2000:]
