@@ -376,66 +376,119 @@ __global__ void k_pcg_p(int n, const double* __restrict__ z, const double* __res
     if (i < n) p[i] = z[i] + beta * p[i];
 }
 
-// Fused operator, stage 1: q = Kp p (CSR) and g = M^-1 B p, both on the same row pattern
-template <int TPR>
+// ---- Row runs through LDS ------------------------------------------------------------------------
+// The entries of RB consecutive rows are one contiguous run of a CSR matrix. A workgroup loads such a
+// run coalesced, every lane's column indices, values and gathers in flight together, leaves the
+// products in LDS, and a lane per row and value array adds the row's products in CSR order. With
+// lanes per row instead, one load instruction of a wavefront touches the entries of 32 rows scattered
+// over 1.8 KB, and the operator's kernels (three and two value arrays) ran at 2.2-2.9 TB/s.
+constexpr int RUN_SLOTS(int RB) { return RB / 32; }              // entries per lane and tile
+constexpr int RUN_TILE(int RB) { return RUN_SLOTS(RB) * BLOCK; }   // 8 entries per row
+
+template <int RB, int NV>
+struct RunTile {
+    int c[RUN_SLOTS(RB)];
+    double v[RUN_SLOTS(RB)][NV];
+    __device__ __forceinline__ void load(const int* __restrict__ ci, const RowValues<NV, double>& vals, int t, int end) {
+#pragma unroll
+        for (int u = 0; u < RUN_SLOTS(RB); ++u) {
+            const int k = t + u * BLOCK + (int)threadIdx.x;
+            const bool ok = k < end;
+            c[u] = ok ? ci[k] : 0;
+#pragma unroll
+            for (int m = 0; m < NV; ++m) v[u][m] = ok ? vals.p[m][k] : 0.0;
+        }
+    }
+};
+
+// Adds the tile's products of the lane's row (entries k0..k1 of the run, tile from t) to acc, for the
+// value arrays of the lane's part of the workgroup (BLOCK / RB parts, array m with part m mod parts)
+template <int RB, int NV>
+__device__ __forceinline__ void run_row_sums(const double* __restrict__ prod, int t, int k0, int k1, double (&acc)[NV]) {
+    constexpr int PARTS = BLOCK / RB;
+    const int part = threadIdx.x / RB;
+    const int a = max(k0, t) - t, b = min(k1, t + RUN_TILE(RB)) - t;
+#pragma unroll
+    for (int m = 0; m < NV; ++m) {
+        if (m % PARTS != part) continue;
+        for (int k = a; k < b; ++k) acc[m] += prod[m * RUN_TILE(RB) + k];
+    }
+}
+template <int RB>
+__device__ __forceinline__ bool run_part_has(int m) { return m % (BLOCK / RB) == (int)threadIdx.x / RB; }
+
+// Fused operator, stage 1: q = Kp p (CSR) and g = M^-1 B p, all on the same row pattern
+template <int RB>
 __global__ void __launch_bounds__(BLOCK)
 k_apply_K_B(int n, int nnz, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ val,
             const double* __restrict__ oss, const double* __restrict__ inv_m, const double* __restrict__ in,
             double* __restrict__ q, double* __restrict__ gx, double* __restrict__ gy, const int* __restrict__ st) {
+    __shared__ double prod[3 * RUN_TILE(RB)];
     if (halted(st)) return;
-    const int groups = gridDim.x * (blockDim.x / TPR);
-    const int lane = threadIdx.x % TPR;
     const RowValues<3, double> kb{{val, oss, oss + (size_t)nnz}};
-    for (int row = (blockIdx.x * blockDim.x + threadIdx.x) / TPR; row < n; row += groups) {
-        double s = 0.0, sx = 0.0, sy = 0.0;
-        row_entries_n<TPR>(ci, kb, rp[row], rp[row + 1], lane, [&](const double* v, int j) {
-            const double xj = in[j];
-            s += v[0] * xj;
-            sx += v[1] * xj;
-            sy += v[2] * xj;
-        });
-        s = group_sum<TPR>(s);
-        sx = group_sum<TPR>(sx);
-        sy = group_sum<TPR>(sy);
-        if (lane == 0) {
-            q[row] = s;
-            gx[row] = sx * inv_m[row];
-            gy[row] = sy * inv_m[row];
+    for (int r0 = blockIdx.x * RB; r0 < n; r0 += gridDim.x * RB) {
+        const int row = r0 + (int)threadIdx.x % RB, e0 = rp[r0], e1 = rp[min(r0 + RB, n)];
+        const int k0 = row < n ? rp[row] : e1, k1 = row < n ? rp[row + 1] : e1;
+        double s[3] = {0.0, 0.0, 0.0};
+        for (int t = e0; t < e1; t += RUN_TILE(RB)) {
+            RunTile<RB, 3> tile;
+            tile.load(ci, kb, t, e1);
+#pragma unroll
+            for (int u = 0; u < RUN_SLOTS(RB); ++u) {
+                const double xj = in[tile.c[u]];
+#pragma unroll
+                for (int m = 0; m < 3; ++m) prod[m * RUN_TILE(RB) + u * BLOCK + threadIdx.x] = tile.v[u][m] * xj;
+            }
+            __syncthreads();
+            run_row_sums<RB, 3>(prod, t, k0, k1, s);
+            __syncthreads();
         }
+        if (row >= n) continue;
+        if (run_part_has<RB>(0)) q[row] = s[0];
+        if (run_part_has<RB>(1)) gx[row] = s[1] * inv_m[row];
+        if (run_part_has<RB>(2)) gy[row] = s[2] * inv_m[row];
     }
 }
 
 // Fused operator, stage 2: q -= B^T g on non-Dirichlet rows; partial p.q per block. The grid is
-// capped (grid-stride over rows) so the partials fit the workspace.
-template <int TPR>
+// capped (grid-stride over row runs) so that the consumers' re-summation stays short.
+template <int RB>
 __global__ void __launch_bounds__(BLOCK)
 k_apply_BT_dot(int n, int nnz, const int* __restrict__ rp, const int* __restrict__ ci,
                const double* __restrict__ oss, const int* __restrict__ tag, OutletMode om,
                const double* __restrict__ gx, const double* __restrict__ gy, const double* __restrict__ p,
                double* __restrict__ q, double* __restrict__ part, const int* __restrict__ st) {
+    __shared__ double prod[RUN_TILE(RB)];
     __shared__ double lds[BLOCK / WAVE];
     if (halted(st)) return;
-    const double* BTx = oss + 2 * (size_t)nnz;
-    const double* BTy = oss + 3 * (size_t)nnz;
-    const int groups = gridDim.x * (blockDim.x / TPR);
-    const int lane = threadIdx.x % TPR;
-    const RowValues<2, double> bt{{BTx, BTy}};
+    const RowValues<2, double> bt{{oss + 2 * (size_t)nnz, oss + 3 * (size_t)nnz}};
     double contrib = 0.0;
-    for (int row = (blockIdx.x * blockDim.x + threadIdx.x) / TPR; row < n; row += groups) {
-        const bool active = !pressure_dirichlet(row, tag[row], om);
-        double s = 0.0;
-        if (active)
-            row_entries_n<TPR>(ci, bt, rp[row], rp[row + 1], lane,
-                               [&](const double* v, int c) { s += v[0] * gx[c] + v[1] * gy[c]; });
-        s = group_sum<TPR>(s);
-        if (lane == 0) {
-            double qi = q[row];
-            if (active) {
-                qi -= s;
-                q[row] = qi;
+    for (int r0 = blockIdx.x * RB; r0 < n; r0 += gridDim.x * RB) {
+        const int row = r0 + (int)threadIdx.x, e0 = rp[r0], e1 = rp[min(r0 + RB, n)];
+        const bool own = (int)threadIdx.x < RB && row < n;
+        const int k0 = own ? rp[row] : e1, k1 = own ? rp[row + 1] : e1;
+        const double qi0 = own ? q[row] : 0.0, pi = own ? p[row] : 0.0;
+        const int ti = own ? tag[row] : 0;
+        double s[1] = {0.0};
+        for (int t = e0; t < e1; t += RUN_TILE(RB)) {
+            RunTile<RB, 2> tile;
+            tile.load(ci, bt, t, e1);
+#pragma unroll
+            for (int u = 0; u < RUN_SLOTS(RB); ++u) {
+                const int j = tile.c[u];
+                prod[u * BLOCK + threadIdx.x] = tile.v[u][0] * gx[j] + tile.v[u][1] * gy[j];
             }
-            contrib += p[row] * qi;
+            __syncthreads();
+            if (own) run_row_sums<RB, 1>(prod, t, k0, k1, s);
+            __syncthreads();
         }
+        if (!own) continue;
+        double qi = qi0;
+        if (!pressure_dirichlet(row, ti, om)) {
+            qi -= s[0];
+            q[row] = qi;
+        }
+        contrib += pi * qi;
     }
     contrib = block_sum(contrib, lds);
     if (threadIdx.x == 0) part[blockIdx.x] = contrib;
@@ -477,63 +530,115 @@ __device__ __forceinline__ int block_state(const int* st, int* it_out) {
 
 // Operator of iteration k (parity h): p_k formed on the fly and stored to p[h]; q = Kp p_k, and
 // with OSS g = M^-1 B p_k for the second stage, else the p.q partials here. Iteration cap check.
-template <int TPR, bool OSS>
+// Row runs through LDS; the first run's entries and both gathers are loaded before the barrier of
+// the r.z sums, so the sums and the state word cost no round trip of their own.
+template <int RB, bool OSS>
 __global__ void __launch_bounds__(BLOCK)
 k_fp_operator(PcgArgs a, int h) {
+    constexpr int NV = OSS ? 3 : 1, U = RUN_SLOTS(RB), TILE = RUN_TILE(RB);
+    __shared__ double prod[NV * TILE];
     __shared__ double lds[2 * BLOCK / WAVE];
-    int it;
-    if (block_state(a.st, &it) != ST_RUNNING) return;
-    if (it >= a.max_iter) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) { a.st[0] = ST_CAPPED; publish(a.status, it, ST_CAPPED); }
-        return;
-    }
-    const bool first = it == 0;
-    double beta = 0.0;
-    if (!first) {
-        double rz[2];
-        sum_partials_k<2>({a.prz[h], a.prz[1 - h]}, {a.nb_rz, a.nb_rz}, 1, rz, lds);
-        beta = rz[0] / (rz[1] + 1.0e-30);
-    }
+    __shared__ int lds_st[2];
     const double* __restrict__ z = a.z;
     const double* __restrict__ po = a.p[1 - h];
     double* __restrict__ pn = a.p[h];
     const int* __restrict__ rp = a.rp;
     const int* __restrict__ ci = a.ci;
-    const double* __restrict__ val = a.val;
-    const int groups = gridDim.x * (blockDim.x / TPR);
-    const int lane = threadIdx.x % TPR;
-    const RowValues<3, double> kb{{val, a.oss, a.oss + (size_t)a.nnz}};
+    RowValues<NV, double> kb;
+    kb.p[0] = a.val;
+    if constexpr (OSS) {
+        kb.p[1] = a.oss;
+        kb.p[2] = a.oss + (size_t)a.nnz;
+    }
+    RunTile<RB, NV> tile;
+    double zj[U], pj[U], zi = 0.0, pi = 0.0;
+    int row, e0, e1, k0, k1;
+    auto load_tile = [&](int t) {
+        tile.load(ci, kb, t, e1);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            zj[u] = z[tile.c[u]];
+            pj[u] = po[tile.c[u]];
+        }
+    };
+    auto load_run = [&](int r0) {
+        row = r0 + (int)threadIdx.x % RB;
+        e0 = rp[r0];
+        e1 = rp[min(r0 + RB, a.n)];
+        load_tile(e0);
+        k0 = row < a.n ? rp[row] : e1;
+        k1 = row < a.n ? rp[row + 1] : e1;
+        if (row < a.n) {
+            zi = z[row];
+            pi = po[row];
+        }
+    };
+    int r0 = blockIdx.x * RB;   // the grid has no empty workgroups
+    load_run(r0);
+    // r_k.z_k, r_{k-1}.z_{k-1} and the state
+    double rz[2] = {0.0, 0.0};
+    for (int k = threadIdx.x; k < a.nb_rz; k += BLOCK) {
+        rz[0] += a.prz[h][k];
+        rz[1] += a.prz[1 - h][k];
+    }
+    if (threadIdx.x == 0) { lds_st[0] = a.st[0]; lds_st[1] = a.st[2]; }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        rz[q] = wave_sum(rz[q]);
+        if ((threadIdx.x & (WAVE - 1)) == 0) lds[q * (BLOCK / WAVE) + threadIdx.x / WAVE] = rz[q];
+    }
+    __syncthreads();
+    const int it = lds_st[1];
+    if (lds_st[0] != ST_RUNNING) return;
+    if (it >= a.max_iter) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) { a.st[0] = ST_CAPPED; publish(a.status, it, ST_CAPPED); }
+        return;
+    }
+    const bool first = it == 0;   // p and r_{k-1}.z_{k-1} are not set yet
+    double beta = 0.0;
+    if (!first) {
+        double now = 0.0, before = 0.0;
+#pragma unroll
+        for (int w = 0; w < BLOCK / WAVE; ++w) {
+            now += lds[w];
+            before += lds[BLOCK / WAVE + w];
+        }
+        beta = now / (before + 1.0e-30);
+    }
     double contrib = 0.0;
-    for (int row = (blockIdx.x * blockDim.x + threadIdx.x) / TPR; row < a.n; row += groups) {
-        double s = 0.0, sx = 0.0, sy = 0.0;
-        if (!OSS) {
-            row_entries<TPR>(ci, val, rp[row], rp[row + 1], lane, [&](double av, int j) {
-                s += av * (first ? z[j] : fma(beta, po[j], z[j]));
-            });
-        } else {
-            row_entries_n<TPR>(ci, kb, rp[row], rp[row + 1], lane, [&](const double* v, int j) {
-                const double pj = first ? z[j] : fma(beta, po[j], z[j]);
-                s += v[0] * pj;
-                sx += v[1] * pj;
-                sy += v[2] * pj;
-            });
+    for (;;) {
+        double s[NV];
+#pragma unroll
+        for (int m = 0; m < NV; ++m) s[m] = 0.0;
+        for (int t = e0;;) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const double xj = first ? zj[u] : fma(beta, pj[u], zj[u]);
+#pragma unroll
+                for (int m = 0; m < NV; ++m) prod[m * TILE + u * BLOCK + threadIdx.x] = tile.v[u][m] * xj;
+            }
+            __syncthreads();
+            run_row_sums<RB, NV>(prod, t, k0, k1, s);
+            __syncthreads();
+            t += TILE;
+            if (t >= e1) break;
+            load_tile(t);
         }
-        s = group_sum<TPR>(s);
-        if (OSS) {
-            sx = group_sum<TPR>(sx);
-            sy = group_sum<TPR>(sy);
-        }
-        if (lane == 0) {
-            const double pi = first ? z[row] : fma(beta, po[row], z[row]);
-            pn[row] = pi;
-            a.q[row] = s;
-            if (OSS) {
-                a.gx[row] = sx * a.inv_m[row];
-                a.gy[row] = sy * a.inv_m[row];
-            } else {
-                contrib += pi * s;
+        if (row < a.n) {
+            if (run_part_has<RB>(0)) {
+                const double p = first ? zi : fma(beta, pi, zi);
+                pn[row] = p;
+                a.q[row] = s[0];
+                if (!OSS) contrib += p * s[0];
+            }
+            if constexpr (OSS) {
+                if (run_part_has<RB>(1)) a.gx[row] = s[1] * a.inv_m[row];
+                if (run_part_has<RB>(2)) a.gy[row] = s[2] * a.inv_m[row];
             }
         }
+        r0 += gridDim.x * RB;
+        if (r0 >= a.n) break;
+        load_run(r0);
     }
     if (!OSS) {
         contrib = block_sum(contrib, lds);
@@ -2329,37 +2434,49 @@ namespace {
 // PCG with the reductions folded into the consuming kernels (k_fp_*), two iterations per
 // captured graph (the search direction and the r.z partials alternate between two buffers).
 // Same algorithm, guards and stopping rules as the reference (src/cfa/linalg.cuh:183-256).
-// The operator kernels run with 2 or 4 lanes per row (about four entries per lane).
+// BiCGSTAB2's product runs with 2 or 4 lanes per row (about four entries per lane).
 int operator_lanes(int n, long long nnz) { return nnz <= 12LL * n ? 2 : 4; }
 
-template <int TPR>
-void launch_fp_operator_t(bool oss, int grid, hipStream_t s, const PcgArgs& a, int h) {
-    if (oss) hipLaunchKernelGGL((k_fp_operator<TPR, true>), dim3(grid), dim3(BLOCK), 0, s, a, h);
-    else hipLaunchKernelGGL((k_fp_operator<TPR, false>), dim3(grid), dim3(BLOCK), 0, s, a, h);
+// Rows per workgroup of the operator kernels and their workgroups (at most RED_BLOCKS, so that the
+// consumers re-sum at most that many partials; 1536 and 2048 ran the same). 64 rows split a small mesh
+// over the CUs; 128 leave room for six workgroups' LDS on a CU. Stage 1 with 64 / 128 / 256 rows:
+// 6.0 / 6.3 / 8.9 us on 29k nodes; 64 / 128 rows: 11.3 / 11.2 us on 115k, 118 / 107 us on 1.84 M.
+int run_rows(int n) {
+    return n <= 64 * RED_BLOCKS ? 64 : 128;
 }
-void launch_fp_operator(int tpr, bool oss, int grid, hipStream_t s, const PcgArgs& a, int h) {
-    if (tpr == 2) launch_fp_operator_t<2>(oss, grid, s, a, h);
-    else launch_fp_operator_t<4>(oss, grid, s, a, h);
+int run_blocks(int n) { return std::min(blocks_for(n, run_rows(n)), RED_BLOCKS); }
+template <typename F>
+void run_dispatch(int n, F f) {
+    if (run_rows(n) == 64) f(std::integral_constant<int, 64>{});
+    else f(std::integral_constant<int, 128>{});
 }
-void launch_apply_K_B(int tpr, int grid, hipStream_t s, int n, int nnz, const int* rp, const int* ci,
-                      const double* val, const double* oss, const double* inv_m, const double* in, double* q,
-                      double* gx, double* gy, const int* st) {
-    if (tpr == 2)
-        hipLaunchKernelGGL(k_apply_K_B<2>, dim3(grid), dim3(BLOCK), 0, s, n, nnz, rp, ci, val, oss, inv_m, in, q, gx, gy,
-                           st);
-    else
-        hipLaunchKernelGGL(k_apply_K_B<4>, dim3(grid), dim3(BLOCK), 0, s, n, nnz, rp, ci, val, oss, inv_m, in, q, gx, gy,
-                           st);
+
+void launch_fp_operator(bool oss, hipStream_t s, const PcgArgs& a, int h) {
+    run_dispatch(a.n, [&](auto rb) {
+        constexpr int RB = decltype(rb)::value;
+        if (oss) hipLaunchKernelGGL((k_fp_operator<RB, true>), dim3(run_blocks(a.n)), dim3(BLOCK), 0, s, a, h);
+        else hipLaunchKernelGGL((k_fp_operator<RB, false>), dim3(run_blocks(a.n)), dim3(BLOCK), 0, s, a, h);
+    });
 }
-void launch_apply_BT_dot(int tpr, int grid, hipStream_t s, int n, int nnz, const int* rp, const int* ci,
-                         const double* oss, const int* tag, OutletMode om, const double* gx, const double* gy,
-                         const double* p, double* q, double* part, const int* st) {
-    if (tpr == 2)
-        hipLaunchKernelGGL(k_apply_BT_dot<2>, dim3(grid), dim3(BLOCK), 0, s, n, nnz, rp, ci, oss, tag, om, gx, gy, p,
-                           q, part, st);
-    else
-        hipLaunchKernelGGL(k_apply_BT_dot<4>, dim3(grid), dim3(BLOCK), 0, s, n, nnz, rp, ci, oss, tag, om, gx, gy, p,
-                           q, part, st);
+void launch_apply_K_B(hipStream_t s, int n, int nnz, const int* rp, const int* ci, const double* val,
+                      const double* oss, const double* inv_m, const double* in, double* q, double* gx, double* gy,
+                      const int* st) {
+    run_dispatch(n, [&](auto rb) {
+        constexpr int RB = decltype(rb)::value;
+        hipLaunchKernelGGL(k_apply_K_B<RB>, dim3(run_blocks(n)), dim3(BLOCK), 0, s, n, nnz, rp, ci, val, oss, inv_m, in,
+                           q, gx, gy, st);
+    });
+}
+// returns the number of partials
+int launch_apply_BT_dot(hipStream_t s, int n, int nnz, const int* rp, const int* ci, const double* oss,
+                        const int* tag, OutletMode om, const double* gx, const double* gy, const double* p, double* q,
+                        double* part, const int* st) {
+    run_dispatch(n, [&](auto rb) {
+        constexpr int RB = decltype(rb)::value;
+        hipLaunchKernelGGL(k_apply_BT_dot<RB>, dim3(run_blocks(n)), dim3(BLOCK), 0, s, n, nnz, rp, ci, oss, tag, om, gx,
+                           gy, p, q, part, st);
+    });
+    return run_blocks(n);
 }
 
 // pressure-Dirichlet rows of the operator: node p_pin with the outlet Dirichlet condition, else outlet nodes
@@ -2399,7 +2516,7 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
     ws->status_host[1] = ST_RUNNING;
     const int nb = red_blocks(n);
     const int blocks = blocks_for(n);
-    const int nb_op = std::min(blocks_for((long long)n * TPR), OP_BLOCKS);
+    const int nb_op = run_blocks(n);
     const int* st_r = a.st;
 
     // prologue (linalg.cuh:205-227): ||b||, x = 0 when trivial, r = b - A x, initial test, z = M^-1 r
@@ -2408,8 +2525,8 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
     hipLaunchKernelGGL(k_zero_if_trivial, dim3(blocks), dim3(BLOCK), 0, s, n, x, st_r);
     if (!amg) hipLaunchKernelGGL(k_inv_diag, dim3(blocks), dim3(BLOCK), 0, s, n, rp, ci, val, 1.0e-14, inv_diag);
     if (oss) {
-        launch_apply_K_B(TPR, nb_op, s, n, a.nnz, rp, ci, val, a.oss, a.inv_m, x, a.q, a.gx, a.gy, st_r);
-        launch_apply_BT_dot(TPR, nb_op, s, n, a.nnz, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.q, a.q, scratch, st_r);
+        launch_apply_K_B(s, n, a.nnz, rp, ci, val, a.oss, a.inv_m, x, a.q, a.gx, a.gy, st_r);
+        (void)launch_apply_BT_dot(s, n, a.nnz, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.q, a.q, scratch, st_r);
     } else {
         csr_op_launch<OP_SPMV, double>(TPR, n, rp, ci, val, x, nullptr, nullptr, 0.0, a.q, st_r, s);
     }
@@ -2435,10 +2552,9 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
 
     // iteration k with parity h (linalg.cuh:231-253)
     auto iteration = [&](int h, hipStream_t q_s) {
-        launch_fp_operator(TPR, oss != nullptr, nb_op, q_s, a, h);
+        launch_fp_operator(oss != nullptr, q_s, a, h);
         if (oss)
-            launch_apply_BT_dot(TPR, nb_op, q_s, n, a.nnz, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.p[h], a.q, a.ppq,
-                                st_r);
+            (void)launch_apply_BT_dot(q_s, n, a.nnz, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.p[h], a.q, a.ppq, st_r);
         hipLaunchKernelGGL(k_fp_update, dim3(nb), dim3(BLOCK), 0, q_s, a, h, nb_op);
         (void)apply_prec(1 - h, true, q_s);
     };
@@ -2566,14 +2682,11 @@ int cfa_pcg_operator(int n, const int* rp, const int* ci, const double* val, con
     int nnz = 0;
     CFA_TRY(hipMemcpyAsync(&nnz, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
     CFA_TRY(hipStreamSynchronize(s));
-    const int tpr = operator_lanes(n, nnz);
-    const int blocks_tpr = std::min(blocks_for((long long)n * tpr), OP_BLOCKS);
     if (stage != 2)
-        launch_apply_K_B(tpr, blocks_tpr, s, n, nnz, rp, ci, val, oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy,
-                         nullptr);
+        launch_apply_K_B(s, n, nnz, rp, ci, val, oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy, nullptr);
     if (stage != 1)
-        launch_apply_BT_dot(tpr, blocks_tpr, s, n, nnz, rp, ci, oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx,
-                            oss->gy, in, out, part, nullptr);
+        (void)launch_apply_BT_dot(s, n, nnz, rp, ci, oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx, oss->gy, in,
+                                  out, part, nullptr);
     return launch_status();
 }
 
@@ -2605,7 +2718,6 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
     const int nb = red_blocks(n);
     const int blocks = blocks_for(n);
     constexpr int TPR = 4;
-    const int blocks_tpr = std::min(blocks_for((long long)n * TPR), OP_BLOCKS);
     int nnz = 0;
     if (oss) {
         CFA_TRY(hipMemcpyAsync(&nnz, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -2619,8 +2731,7 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
 
     auto apply_op = [&](const double* in, double* out, hipStream_t q_s) {
         if (oss) {
-            hipLaunchKernelGGL(k_apply_K_B<TPR>, dim3(blocks_tpr), dim3(BLOCK), 0, q_s, n, nnz, rp, ci, val,
-                               oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy, st);
+            launch_apply_K_B(q_s, n, nnz, rp, ci, val, oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy, st);
         } else {
             csr_op_launch<OP_SPMV, double>(TPR, n, rp, ci, val, in, nullptr, nullptr, 0.0, out, st, q_s);
             if (extra_cb) extra_cb(in, out, extra_ctx);
@@ -2629,9 +2740,8 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
     // second stage of the fused operator (q -= B^T g) with the p.q partials, or a plain dot
     auto finish_op_dot = [&](const double* pv, double* qv, hipStream_t q_s) {
         if (oss) {
-            hipLaunchKernelGGL(k_apply_BT_dot<TPR>, dim3(blocks_tpr), dim3(BLOCK), 0, q_s, n, nnz, rp, ci,
-                               oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx, oss->gy, pv, qv, part, st);
-            return blocks_tpr;
+            return launch_apply_BT_dot(q_s, n, nnz, rp, ci, oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx, oss->gy,
+                                       pv, qv, part, st);
         }
         hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(BLOCK), 0, q_s, n, pv, qv, part, st);
         return nb;

@@ -5,7 +5,7 @@
 // block reductions or other summation orders must match to the stated relative tolerance.
 //
 //   parity <case> [level]    case: momentum pressure correction forces indicator mms oss ilu
-//                                  spmv amg sell coupled pcg bicgstab jacobi mixed topology outlet nvb remap reproject
+//                                  spmv amg sell coupled runs pcg bicgstab jacobi mixed topology outlet nvb remap reproject
 //                                  all
 //
 // Prints one line per compared quantity and exits 0 when every comparison passes.
@@ -712,6 +712,70 @@ void case_coupled(Fixture& f) {
                 expect((amg.view()->dense != nullptr) == (forms[k].dense > 0), "dense bottom");
             }
         }
+    }
+}
+
+// The pressure operator's row runs (cfa_pcg_operator) at the edges of their tiles, against FP64 sums
+// in entry order on the host: rows of 0 to 40 entries (more than a tile's 8 per row, so that a run takes
+// several passes, and runs without entries), and sizes around one and two workgroups' rows and past
+// the capped grid (64 x 1024 rows, 128 x 1024 rows). Tolerance: a row's sum of 40 products in another
+// order differs by at most 40 eps of its terms' sum (values and vector in [-1, 1], so 40): 4e-13
+// relative to the largest entry (at least a few tenths).
+void case_runs() {
+    std::printf("[operator row runs]\n");
+    std::mt19937_64 rng(7);
+    std::uniform_real_distribution<double> U(-1.0, 1.0);
+    for (int n : {1, 63, 64, 65, 127, 129, 200, 65535, 65537, 131071, 131073, 300007}) {
+        std::vector<int> rp(n + 1, 0), ci, tag(n);
+        for (int i = 0; i < n; ++i) {
+            const int block = i / 64 % 3, len = block == 0 ? (int)(rng() % 41) : block == 1 ? 0 : 5 + (int)(rng() % 5);
+            for (int k = 0; k < len; ++k) ci.push_back((int)(rng() % n));
+            rp[i + 1] = (int)ci.size();
+            tag[i] = rng() % 7 ? BC_INTERIOR : BC_OUTLET;
+        }
+        const int nnz = rp[n];
+        const size_t cap = std::max(nnz, 1);
+        Vec val(cap), oss(4 * cap), im(n), x(n);
+        for (Vec* v : {&val, &oss, &im, &x})
+            for (double& e : *v) e = U(rng);
+        if (ci.empty()) ci.push_back(0);
+        DevArray<int> d_rp, d_ci, d_tag;
+        DevArray<double> d_val, d_oss, d_im, d_x, d_gx, d_gy, d_out, d_part;
+        d_rp.upload(rp);
+        d_ci.upload(ci);
+        d_tag.upload(tag);
+        d_val.upload(val);
+        d_im.upload(im);
+        d_x.upload(x);
+        for (auto* d : {&d_gx, &d_gy, &d_out}) d->reserve(n);
+        d_part.reserve(4096);
+        Vec packed(4 * cap, 0.0);   // the four value arrays nnz apart
+        for (int m = 0; m < 4; ++m) std::copy_n(oss.begin() + m * cap, nnz, packed.begin() + (size_t)m * nnz);
+        d_oss.upload(packed);
+        const cfa_oss_op_t op = {d_oss, d_im, d_tag, d_gx, d_gy, 0, 0};
+        GPU_CHECK(cfa_pcg_operator(n, d_rp, d_ci, d_val, &op, d_x, d_out, d_part, 0, solver_stream()));
+        Vec gx(n), gy(n), out(n);
+        for (int i = 0; i < n; ++i) {
+            double s = 0.0, sx = 0.0, sy = 0.0;
+            for (int k = rp[i]; k < rp[i + 1]; ++k) {
+                s += val[k] * x[ci[k]];
+                sx += packed[k] * x[ci[k]];
+                sy += packed[(size_t)nnz + k] * x[ci[k]];
+            }
+            out[i] = s;
+            gx[i] = sx * im[i];
+            gy[i] = sy * im[i];
+        }
+        for (int i = 0; i < n; ++i) {
+            double s = 0.0;
+            for (int k = rp[i]; k < rp[i + 1]; ++k)
+                s += packed[2 * (size_t)nnz + k] * gx[ci[k]] + packed[3 * (size_t)nnz + k] * gy[ci[k]];
+            if (tag[i] != BC_OUTLET) out[i] -= s;
+        }
+        std::printf("  n %d, %d entries\n", n, nnz);
+        close_rel("  Kp x - B^T M^-1 B x", down(d_out, n), out, 4e-13);
+        close_rel("  M^-1 Bx x", down(d_gx, n), gx, 4e-13);
+        close_rel("  M^-1 By x", down(d_gy, n), gy, 4e-13);
     }
 }
 
@@ -1504,6 +1568,7 @@ int main(int argc, char** argv) {
         if (all || what == "amg") case_amg(f);
         if (all || what == "sell") case_sell(f);
         if (all || what == "coupled") case_coupled(f);
+        if (all || what == "runs") case_runs();
         if (all || what == "pcg") case_pcg(f);
         if (all || what == "bicgstab") case_bicgstab(f);
         if (all || what == "jacobi") case_jacobi(f);

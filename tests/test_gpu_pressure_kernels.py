@@ -1,6 +1,7 @@
 """The coupled V-cycle through the C ABI, on the GPU (tests/native/parity.cpp):
 the cycle against the one with separate residual, restriction and prolongation (uniform levels 1, 3
-and 4: one to four smoothed levels, with the dense bottom at none, the last or the first coarse one)."""
+and 4: one to four smoothed levels, with the dense bottom at none, the last or the first coarse one);
+and the pressure operator's row runs at the edges of their tiles against sums on the host."""
 import subprocess
 from pathlib import Path
 
@@ -15,5 +16,12 @@ pytestmark = pytest.mark.gpu
 def test_coupled_cycle(level):
     print(f"[case] coupled V-cycle level {level}", flush=True)
     r = subprocess.run([str(BIN), "coupled", str(level)], capture_output=True, text=True, timeout=120)
+    print(r.stdout)
+    assert r.returncode == 0 and "ALL PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-2000:]
+
+
+def test_operator_row_runs():
+    print("[case] operator row runs", flush=True)
+    r = subprocess.run([str(BIN), "runs", "0"], capture_output=True, text=True, timeout=120)
     print(r.stdout)
     assert r.returncode == 0 and "ALL PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-2000:]
