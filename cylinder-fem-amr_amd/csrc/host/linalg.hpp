@@ -178,9 +178,15 @@ public:
     double theta = 0.08;
     int coarse_target = 300;
     int max_levels = 15;
-    // Levels up to this size carry the coupled transfers, the first one (from level 1) up to
-    // dense_max_rows the dense matrix of the rest of the cycle (0: none).
-    int couple_max_rows = 1 << 20;
+    // Levels up to couple_max_rows carry the coupled transfers: below, a cycle is bound by its launches;
+    // beyond, W's 11 entries per row (A has 7, P 2.7) cost more than the launches saved. Two time steps
+    // with limits 60k / 300k / 1M / 3M: level 4 (115k rows) 10.4 / 10.1 / 10.1 / 10.1 ms, level 5 (461k)
+    // 16.2 / 16.0 / 16.8 / 16.8 ms, level 6 (1.84 M) 63.3 / 63.3 / 63.5 / 69.6 ms.
+    int couple_max_rows = 300000;
+    // The first level (from level 1) of at most dense_max_rows rows carries the dense matrix of the rest
+    // of the cycle (0: none). 500 / 1000 / 1536 / 2500: level 3 (639 rows) 3.08 / 2.77 / 2.77 / 2.77 ms a
+    // step, level 5 (1311 rows) 17.4 / 17.4 / 16.7 / 16.8 ms, level 4 (2389 rows) 5.05 / 5.05 / 5.03 / 4.95
+    // ms, where building the matrix takes longer than the 50 steps of a hierarchy gain.
     int dense_max_rows = 1536;
     bool fp32 = false;   // run the cycle in FP32 (coarse solve in FP64); FP32 copies made at set-up
     // The whole set-up runs on the device, level by level (D^-1, spectral radius, aggregation,
