@@ -570,6 +570,108 @@ k_dense_sweep(int n, const int* __restrict__ rp, const int* __restrict__ ci, con
     y[(size_t)i * n + c] = t;
 }
 
+// ---- Dense inverse of the coarsest operator ------------------------------------------------------
+// Block Gauss-Jordan elimination in place, two launches per block of GJ_B columns K: the panels (the
+// inverse D of the pivot block, the row panel R = D A_K: with D in its own columns, a copy C of the
+// column panel), then every tile of the matrix, A - C R outside the block's rows and R inside them.
+// On the host (Cholesky, forward substitution, triangular product) this took 0.5 ms of a set-up at
+// 135 rows, 20 ms at 613 (uniform level 6) and 450 ms at 1340 rows.
+constexpr int GJ_B = 32;
+constexpr int GJ_T = 64;   // tile edge
+
+__global__ void k_csr_to_dense(int n, const int* __restrict__ rp, const int* __restrict__ ci,
+                               const double* __restrict__ v, double* __restrict__ out) {
+    const int i = blockIdx.x;
+    double* row = out + (size_t)i * n;
+    for (int j = threadIdx.x; j < n; j += BLOCK) row[j] = 0.0;
+    __syncthreads();
+    for (int k = rp[i] + threadIdx.x; k < rp[i + 1]; k += BLOCK) row[ci[k]] = v[k];
+}
+
+// GJ_T columns of R and rows of C per workgroup; each workgroup inverts the pivot block itself (32
+// steps in LDS, about 5 us, instead of a launch of its own). A last block shorter than GJ_B is padded
+// with the identity.
+__global__ void __launch_bounds__(BLOCK)
+k_gj_panels(int n, int k0, const double* __restrict__ a, double* __restrict__ r, double* __restrict__ c,
+            double* __restrict__ info) {
+#pragma clang fp contract(fast)
+    __shared__ double d[GJ_B][GJ_B + 1], col[GJ_B], p[GJ_B][GJ_T + 1];
+    const int nb = min(GJ_B, n - k0), j0 = blockIdx.x * GJ_T, t = threadIdx.x;
+    for (int e = t; e < GJ_B * GJ_B; e += BLOCK) {
+        const int i = e / GJ_B, j = e % GJ_B;
+        d[i][j] = i < nb && j < nb ? a[(size_t)(k0 + i) * n + k0 + j] : (i == j ? 1.0 : 0.0);
+    }
+    for (int e = t; e < GJ_B * GJ_T; e += BLOCK) {
+        const int i = e / GJ_T, j = j0 + e % GJ_T;
+        p[i][e % GJ_T] = i < nb && j < n ? a[(size_t)(k0 + i) * n + j] : 0.0;
+    }
+    for (int e = t; e < GJ_B * GJ_T; e += BLOCK) {
+        const int i = j0 + e / GJ_B, l = e % GJ_B;
+        if (i < n) c[(size_t)i * GJ_B + l] = l < nb ? a[(size_t)i * n + k0 + l] : 0.0;
+    }
+    for (int s = 0; s < GJ_B; ++s) {
+        __syncthreads();
+        const double piv = d[s][s];
+        if (t < GJ_B) col[t] = d[t][s];
+        if (blockIdx.x == 0 && t == 0 && !(piv > 0.0) && info[0] == 0.0) {
+            info[0] = 1.0;
+            info[1] = piv;
+        }
+        __syncthreads();
+        const double f = 1.0 / piv;
+        if (t < GJ_B) d[s][t] = (t == s ? 1.0 : d[s][t]) * f;
+        __syncthreads();
+        for (int e = t; e < GJ_B * GJ_B; e += BLOCK) {
+            const int i = e / GJ_B, j = e % GJ_B;
+            if (i != s) d[i][j] = (j == s ? 0.0 : d[i][j]) - col[i] * d[s][j];
+        }
+    }
+    __syncthreads();
+    const int jl = t % GJ_T, j = j0 + jl;
+    if (j >= n) return;
+    const bool own = j >= k0 && j < k0 + nb;
+    for (int i = t / GJ_T; i < nb; i += BLOCK / GJ_T) {
+        double s = 0.0;
+        for (int l = 0; l < GJ_B; ++l) s += d[i][l] * p[l][jl];
+        r[(size_t)i * n + j] = own ? d[i][j - k0] : s;
+    }
+}
+
+// One tile of the elimination step, 4 x 4 entries per thread
+__global__ void __launch_bounds__(BLOCK)
+k_gj_update(int n, int k0, const double* __restrict__ r, const double* __restrict__ c, double* __restrict__ a) {
+#pragma clang fp contract(fast)
+    __shared__ double cs[GJ_T][GJ_B + 1], rs[GJ_B][GJ_T];
+    const int nb = min(GJ_B, n - k0), i0 = blockIdx.y * GJ_T, j0 = blockIdx.x * GJ_T, t = threadIdx.x;
+    for (int e = t; e < GJ_T * GJ_B; e += BLOCK) {
+        const int i = i0 + e / GJ_B, l = e % GJ_B;
+        cs[e / GJ_B][l] = i < n ? c[(size_t)i * GJ_B + l] : 0.0;
+        const int l2 = e / GJ_T, j = j0 + e % GJ_T;
+        rs[l2][e % GJ_T] = l2 < nb && j < n ? r[(size_t)l2 * n + j] : 0.0;
+    }
+    __syncthreads();
+    const int ti = t / 16 * 4, tj = t % 16;
+    double s[4][4] = {};
+#pragma unroll 4
+    for (int l = 0; l < GJ_B; ++l)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) s[x][y] += cs[ti + x][l] * rs[l][tj + 16 * y];
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const int i = i0 + ti + x, j = j0 + tj + 16 * y;
+            if (i >= n || j >= n) continue;
+            double* out = a + (size_t)i * n + j;
+            if (i >= k0 && i < k0 + nb) *out = rs[i - k0][tj + 16 * y];
+            else *out = (j >= k0 && j < k0 + nb ? 0.0 : *out) - s[x][y];
+        }
+}
+
+__global__ void k_gj_info(double* info) { info[threadIdx.x] = 0.0; }
+
 // ---- R = P^T (csr_transpose: entries of each column in ascending row order) ----------------------
 // ---- transpose (host csr_transpose: the entries of a column in ascending row order) ----------------
 // A stable radix sort of the entries by column, from their CSR order (rows ascending), lists
@@ -880,6 +982,26 @@ int cfa_amg_dense_level(int rows, const int* a_rp, const int* a_ci, const double
                        nullptr, nullptr, nullptr, nullptr, tmp);
     hipLaunchKernelGGL(k_dense_sweep, dim3(cb, rows), dim3(BLOCK), 0, s, rows, a_rp, a_ci, a_v, dinv, omega, tmp, w_rp,
                        w_ci, w_v, cols > 0 ? f : nullptr, out);
+    return launch_status();
+}
+
+size_t cfa_amg_coarse_inverse_ws_doubles(int n) { return n > 0 ? 2 * (size_t)GJ_B * n : 1; }
+
+int cfa_amg_coarse_inverse(int n, const int* rp, const int* ci, const double* v, double* ws, double* inv, double* info,
+                           cfa_stream_t stream) {
+    if (n < 0 || !info) return CFA_E_ARG;
+    const hipStream_t s = as_stream(stream);
+    hipLaunchKernelGGL(k_gj_info, dim3(1), dim3(2), 0, s, info);
+    if (n == 0) return launch_status();
+    if (!rp || !ci || !v || !ws || !inv) return CFA_E_ARG;
+    double* r = ws;
+    double* c = ws + (size_t)GJ_B * n;
+    const unsigned tiles = (unsigned)((n + GJ_T - 1) / GJ_T);
+    hipLaunchKernelGGL(k_csr_to_dense, dim3(n), dim3(BLOCK), 0, s, n, rp, ci, v, inv);
+    for (int k0 = 0; k0 < n; k0 += GJ_B) {
+        hipLaunchKernelGGL(k_gj_panels, dim3(tiles), dim3(BLOCK), 0, s, n, k0, inv, r, c, info);
+        hipLaunchKernelGGL(k_gj_update, dim3(tiles, tiles), dim3(BLOCK), 0, s, n, k0, r, c, inv);
+    }
     return launch_status();
 }
 

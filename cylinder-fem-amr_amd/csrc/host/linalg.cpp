@@ -4,8 +4,8 @@
 // smoothing step with omega = 4 / (3 * 1.05 * rho(D^-1 A)) from 20 power iterations, Galerkin
 // R A P with R = P^T, stop at <= 300 rows, 15 levels or when P.cols >= 0.85 rows, dense Cholesky
 // inverse of the coarsest operator) is sequenced here level by level over the device kernels of
-// amg_setup.hip and aggregate.hip; the host inverts the coarse operator and, for remap(), fills
-// the prolongator rows of new nodes layer by layer.
+// amg_setup.hip and aggregate.hip; the host, for remap(), fills the prolongator rows of new nodes
+// layer by layer.
 #include "linalg.hpp"
 
 #include <algorithm>
@@ -605,47 +605,6 @@ std::vector<int> down_ints(const int* d, size_t n) {
     if (n) GPU_CHECK(cfa_memcpy(h.data(), d, n * sizeof(int), 1, solver_stream()));
     return h;
 }
-
-// Inverse of a small SPD matrix (the coarse level, at most a few hundred rows): Cholesky factor
-// L (row by row, in place in the lower triangle), W = L^-1 by forward substitution per column,
-// then M^-1 = W^T W. The reference inverts the same matrix through its Cholesky factor
-// (src/cfa/linalg.cuh:1395-1430); an indefinite pivot ends the run as there.
-std::vector<double> spd_inverse(std::vector<double> M, int n) {
-    auto at = [&](int i, int j) -> double& { return M[(size_t)i * n + j]; };
-    for (int i = 0; i < n; ++i)
-        for (int j = 0; j <= i; ++j) {
-            double s = at(i, j);
-            for (int k = 0; k < j; ++k) s -= at(i, k) * at(j, k);
-            if (i == j) {
-                if (!(s > 0.0)) {
-                    std::fprintf(stderr, "[AMG] coarse operator not SPD (pivot %.3e), aborting\n", s);
-                    std::exit(EXIT_FAILURE);
-                }
-                at(i, i) = std::sqrt(s);
-            } else {
-                at(i, j) = s / at(j, j);
-            }
-        }
-    std::vector<double> W((size_t)n * n, 0.0);
-#pragma omp parallel for schedule(dynamic, 8)
-    for (int c = 0; c < n; ++c) {
-        W[(size_t)c * n + c] = 1.0 / at(c, c);
-        for (int i = c + 1; i < n; ++i) {
-            double s = 0.0;
-            for (int k = c; k < i; ++k) s += at(i, k) * W[(size_t)k * n + c];
-            W[(size_t)i * n + c] = -s / at(i, i);
-        }
-    }
-    std::vector<double> inv((size_t)n * n);
-#pragma omp parallel for schedule(dynamic, 8)
-    for (int i = 0; i < n; ++i)
-        for (int j = 0; j <= i; ++j) {
-            double s = 0.0;
-            for (int k = i; k < n; ++k) s += W[(size_t)k * n + i] * W[(size_t)k * n + j];
-            inv[(size_t)i * n + j] = inv[(size_t)j * n + i] = s;
-        }
-    return inv;
-}
 }  // namespace
 
 // One level on the device: D^-1, the spectral radius of D^-1 A (power iteration), the
@@ -859,21 +818,23 @@ void AmgPreconditioner::setup(int n, int nnz, const int* d_row_ptr, const int* d
     }
     for (auto& L : old) spare_.push_back(std::move(L));
 
-    // coarse operator to the host, dense inverse back to the device
+    // dense inverse of the coarse operator; an indefinite pivot ends the run as in the reference
     phase_start();
     coarse_n = rows;
-    const std::vector<int> crp = down_ints(arp, rows + 1), cci = down_ints(aci, entries);
-    std::vector<double> cv(entries);
-    if (entries) GPU_CHECK(cfa_memcpy(cv.data(), av, entries * sizeof(double), 1, solver_stream()));
-    std::vector<double> D((size_t)coarse_n * coarse_n, 0.0);
-    for (int i = 0; i < coarse_n; ++i)
-        for (int a = crp[i]; a < crp[i + 1]; ++a) D[(size_t)i * coarse_n + cci[a]] = cv[a];
-    const std::vector<double> inv = spd_inverse(D, coarse_n);
-    d_coarse_inv.upload(inv);
+    d_coarse_inv.reserve(std::max<size_t>((size_t)rows * rows, 1));
+    d_gj_.reserve(cfa_amg_coarse_inverse_ws_doubles(rows));
+    d_gj_info_.reserve(2, 0);
+    GPU_CHECK(cfa_amg_coarse_inverse(rows, arp, aci, av, d_gj_, d_coarse_inv, d_gj_info_, solver_stream()));
     d_cx.reserve(std::max(coarse_n, 1), 16);
     d_cb.reserve(std::max(coarse_n, 1), 16);
     build_dense();
     refresh_view();
+    double pivot[2] = {0.0, 0.0};
+    d_gj_info_.download(pivot, 2);
+    if (pivot[0] != 0.0) {
+        std::fprintf(stderr, "[AMG] coarse operator not SPD (pivot %.3e), aborting\n", pivot[1]);
+        std::exit(EXIT_FAILURE);
+    }
     dev_sync();
     phase_end(PH_COARSE);
     setup_ms = ms_since(t0);

@@ -190,8 +190,7 @@ public:
     int dense_max_rows = 1536;
     bool fp32 = false;   // run the cycle in FP32 (coarse solve in FP64); FP32 copies made at set-up
     // The whole set-up runs on the device, level by level (D^-1, spectral radius, aggregation,
-    // P smoothing, transpose, Galerkin product); only the coarse operator comes to the host for
-    // its dense inverse.
+    // P smoothing, transpose, Galerkin product, dense inverse of the coarse operator).
     bool keep_p0_host = false;     // download the level-0 prolongator for remap() (without it, remap() sets up anew)
     bool keep_aggregates = false;  // download the level-0 aggregates into last_aggregates
     int device_levels = 0;         // levels the last set-up built
@@ -261,6 +260,7 @@ private:
     bool has_dense_ = false;
     DevArray<double> d_dense_[2], d_dense_tmp_, d_dense_f_;
     int dense_slot_ = 0;
+    DevArray<double> d_gj_, d_gj_info_;   // coarse inverse: panels, {failed, pivot}
     // the sliced-ELL copy of the level's operator when its rows are at most CFA_SELL_MAX_LEN long
     void build_sell(Level& L);
     DevArray<double> d_p0v_, d_x0_, d_pw_;

@@ -515,6 +515,14 @@ int cfa_amg_smooth_product(int n, const int* x_rp, const int* x_ci, const double
 int cfa_amg_dense_level(int rows, const int* a_rp, const int* a_ci, const double* a_v, const double* dinv,
                         double omega, const int* w_rp, const int* w_ci, const double* w_v, int cols,
                         const double* coarse, double* f, double* tmp, double* out, cfa_stream_t stream);
+/* cfa_amg_coarse_inverse: the dense inverse (row-major, n x n) of the coarsest operator, a symmetric
+ * positive definite n x n CSR matrix (invert_coarse, linalg.cuh:1395-1430, a host Cholesky there), by
+ * block Gauss-Jordan elimination; the pivots are the Cholesky factor's squared diagonal. info (device)
+ * [2] = 1 when a pivot is not positive, else 0, and that pivot (the result is then undefined).
+ * ws: cfa_amg_coarse_inverse_ws_doubles(n) doubles. */
+size_t cfa_amg_coarse_inverse_ws_doubles(int n);
+int cfa_amg_coarse_inverse(int n, const int* rp, const int* ci, const double* v, double* ws, double* inv, double* info,
+                           cfa_stream_t stream);
 /* cfa_amg_aggregate: the three-phase greedy aggregation of smoothed_prolongator (linalg.cuh:
  * 1306-1356) for the n x n CSR matrix (rp, ci, val) with inverse diagonal dinv and strength
  * threshold theta: agg [n] (aggregate of each row, numbered as the row-order loop numbers them),

@@ -5,7 +5,7 @@
 // block reductions or other summation orders must match to the stated relative tolerance.
 //
 //   parity <case> [level]    case: momentum pressure correction forces indicator mms oss ilu
-//                                  spmv amg sell coupled runs pcg bicgstab jacobi mixed topology outlet nvb remap reproject
+//                                  spmv amg sell coupled runs inverse pcg bicgstab jacobi mixed topology outlet nvb remap reproject
 //                                  all
 //
 // Prints one line per compared quantity and exits 0 when every comparison passes.
@@ -776,6 +776,63 @@ void case_runs() {
         close_rel("  Kp x - B^T M^-1 B x", down(d_out, n), out, 4e-13);
         close_rel("  M^-1 Bx x", down(d_gx, n), gx, 4e-13);
         close_rel("  M^-1 By x", down(d_gy, n), gy, 4e-13);
+    }
+}
+
+// The dense inverse of the coarsest operator at the edges of its blocks (32) and tiles (64): random
+// sparse SPD matrices of condition below 20 (unit off-diagonal row sums at most 0.9 on a diagonal in
+// [1, 2]) with isolated rows, as Dirichlet rows leave them. max |A inv - I| is held to n eps times
+// the largest row sum products (at most 3 x 20): 60 x 1400 x 1.1e-16 = 1e-11, and below 300 rows 2e-12.
+// A matrix with a negative pivot is reported with that pivot.
+void case_inverse() {
+    std::printf("[coarse inverse]\n");
+    std::mt19937_64 rng(11);
+    std::uniform_real_distribution<double> U(0.0, 1.0);
+    DevArray<int> d_rp, d_ci;
+    DevArray<double> d_v, d_ws, d_inv, d_info;
+    for (int n : {1, 2, 31, 32, 33, 63, 64, 65, 96, 135, 300, 613, 1340}) {
+        std::vector<std::vector<double>> A(n, std::vector<double>(n, 0.0));
+        for (int i = 0; i < n; ++i) {
+            A[i][i] = 1.0 + U(rng);
+            if (i % 5 == 4) continue;   // isolated
+            for (int q = 0; q < 3; ++q) {
+                const int j = (int)(rng() % n);
+                if (j == i || j % 5 == 4) continue;
+                A[i][j] = A[j][i] = -0.15 * U(rng);
+            }
+        }
+        for (int bad = 0; bad < 2; ++bad) {
+            if (bad) A[n / 2][n / 2] = -3.0;
+            std::vector<int> rp(1, 0), ci;
+            Vec v;
+            for (int i = 0; i < n; ++i) {
+                for (int j = 0; j < n; ++j)
+                    if (A[i][j] != 0.0) { ci.push_back(j); v.push_back(A[i][j]); }
+                rp.push_back((int)ci.size());
+            }
+            d_rp.upload(rp);
+            d_ci.upload(ci);
+            d_v.upload(v);
+            d_ws.reserve(cfa_amg_coarse_inverse_ws_doubles(n));
+            d_inv.reserve((size_t)n * n);
+            d_info.reserve(2);
+            GPU_CHECK(cfa_amg_coarse_inverse(n, d_rp, d_ci, d_v, d_ws, d_inv, d_info, solver_stream()));
+            const Vec info = down(d_info, 2), inv = down(d_inv, (size_t)n * n);
+            if (bad) {
+                expect(info[0] == 1.0 && info[1] < 0.0, "negative pivot reported");
+                continue;
+            }
+            double worst = 0.0;
+            for (int i = 0; i < n; ++i) {
+                Vec row(n, 0.0);
+                for (int k = rp[i]; k < rp[i + 1]; ++k)
+                    for (int j = 0; j < n; ++j) row[j] += v[k] * inv[(size_t)ci[k] * n + j];
+                row[i] -= 1.0;
+                for (double e : row) worst = std::max(worst, std::fabs(e));
+            }
+            std::printf("  n %d: max |A inv - I| %.2e\n", n, worst);
+            expect(info[0] == 0.0 && worst <= (n <= 300 ? 2e-12 : 1e-11), "inverse");
+        }
     }
 }
 
@@ -1569,6 +1626,7 @@ int main(int argc, char** argv) {
         if (all || what == "sell") case_sell(f);
         if (all || what == "coupled") case_coupled(f);
         if (all || what == "runs") case_runs();
+        if (all || what == "inverse") case_inverse();
         if (all || what == "pcg") case_pcg(f);
         if (all || what == "bicgstab") case_bicgstab(f);
         if (all || what == "jacobi") case_jacobi(f);
