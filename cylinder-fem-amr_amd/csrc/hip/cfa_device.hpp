@@ -73,20 +73,42 @@ __device__ __forceinline__ double sum_partials(const double* part, int count, in
 }
 
 // K sums of partials at once, each in the order of sum_partials (lane-strided, the wave tree, the
-// waves in order), so the values are bit-identical to K calls of it, with one pair of barriers
-// instead of K: out[q] = sum of parts[q][k * stride], k < count[q]; valid in all threads.
-// lds: at least K * blockDim.x / 64 doubles.
-template <int K>
+// waves in order), so the values are bit-identical to K calls of it: out[q] = sum of
+// parts[q][k * stride], k < count[q]; valid in all threads. The lane's first SUM_SLOTS partials of
+// every sum are loaded before any is added (all of them for the up to 1024 partials of the reductions
+// with 256 lanes), and one lane reads W of the state words st[0], st[2], st[3] beside them into
+// lds_word, so a consumer pays one round trip and one barrier for its sums and its state together (the
+// words are the same for the whole workgroup, also while another workgroup changes them).
+// lds: at least K * blockDim.x / 64 doubles. A caller that reuses lds passes a barrier first.
+constexpr int SUM_SLOTS = 4;
+template <int K, int W = 0>
 __device__ __forceinline__ void sum_partials_k(const double* const (&parts)[K], const int (&count)[K], int stride,
-                                               double (&out)[K], double* lds) {
-    double s[K];
+                                               double (&out)[K], double* lds, const int* st = nullptr,
+                                               int* lds_word = nullptr) {
+    double v[K][SUM_SLOTS];
     int cmax = 0;
 #pragma unroll
     for (int q = 0; q < K; ++q) {
-        s[q] = 0.0;
         cmax = count[q] > cmax ? count[q] : cmax;
+#pragma unroll
+        for (int u = 0; u < SUM_SLOTS; ++u) {
+            const int k = threadIdx.x + u * blockDim.x;
+            v[q][u] = k < count[q] ? parts[q][(size_t)k * stride] : 0.0;
+        }
     }
-    for (int k = threadIdx.x; k < cmax; k += blockDim.x)
+    if (W > 0 && threadIdx.x == 0) {
+        lds_word[0] = st[0];
+        if (W > 1) lds_word[1] = st[2];
+        if (W > 2) lds_word[2] = st[3];
+    }
+    double s[K];
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+        s[q] = 0.0;
+#pragma unroll
+        for (int u = 0; u < SUM_SLOTS; ++u) s[q] += v[q][u];
+    }
+    for (int k = threadIdx.x + SUM_SLOTS * blockDim.x; k < cmax; k += blockDim.x)
 #pragma unroll
         for (int q = 0; q < K; ++q)
             if (k < count[q]) s[q] += parts[q][(size_t)k * stride];
@@ -104,13 +126,13 @@ __device__ __forceinline__ void sum_partials_k(const double* const (&parts)[K], 
         for (int w = 0; w < nw; ++w) t += lds[q * nw + w];
         out[q] = t;
     }
-    __syncthreads();
 }
 
 // K block sums at once (block_sum's order: the wave tree, then the waves in order); valid in
 // thread 0. lds: at least K * blockDim.x / 64 doubles.
 template <int K>
 __device__ __forceinline__ void block_sum_k(double (&v)[K], double* lds) {
+    __syncthreads();   // lds may still be read from an earlier sum
     const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
     const int nw = (blockDim.x + WAVE - 1) / WAVE;
 #pragma unroll

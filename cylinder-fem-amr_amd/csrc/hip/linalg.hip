@@ -181,9 +181,12 @@ __global__ void k_sum_to(int nb, const double* __restrict__ part, double* __rest
     if (threadIdx.x == 0) *out = take_sqrt ? sqrt(s) : s;
 }
 
+// Workgroups of a vector kernel that leaves partial sums: every workgroup of the consumer reads them
+// all again, so vectors that one workgroup per CU can stream (up to 2^20 entries) get no more than
+// that, longer ones RED_BLOCKS for the bytes in flight. Time steps with 256 / 512 / 1024 workgroups at
+// most on such vectors: 4.97 / 4.97 / 5.02 ms on 115k nodes, 15.6 / 15.8 / 15.8 ms on 461k.
 inline int red_blocks(long long n) {
-    int nb = blocks_for(n > 0 ? n : 1);
-    return nb > RED_BLOCKS ? RED_BLOCKS : nb;
+    return std::min(blocks_for(n > 0 ? n : 1), n <= (1 << 20) ? RED_BLOCKS / 4 : RED_BLOCKS);
 }
 
 // ---- elementwise ------------------------------------------------------------------------------------
@@ -519,15 +522,6 @@ struct PcgArgs {
     double* sc; int* st; int* status;
 };
 
-// state word read once per block (block-uniform early exits in kernels with barriers)
-__device__ __forceinline__ int block_state(const int* st, int* it_out) {
-    __shared__ int s_state, s_it;
-    if (threadIdx.x == 0) { s_state = st[0]; s_it = st[2]; }
-    __syncthreads();
-    if (it_out) *it_out = s_it;
-    return s_state;
-}
-
 // Operator of iteration k (parity h): p_k formed on the fly and stored to p[h]; q = Kp p_k, and
 // with OSS g = M^-1 B p_k for the second stage, else the p.q partials here. Iteration cap check.
 // Row runs through LDS; the first run's entries and both gathers are loaded before the barrier of
@@ -575,19 +569,8 @@ k_fp_operator(PcgArgs a, int h) {
     };
     int r0 = blockIdx.x * RB;   // the grid has no empty workgroups
     load_run(r0);
-    // r_k.z_k, r_{k-1}.z_{k-1} and the state
-    double rz[2] = {0.0, 0.0};
-    for (int k = threadIdx.x; k < a.nb_rz; k += BLOCK) {
-        rz[0] += a.prz[h][k];
-        rz[1] += a.prz[1 - h][k];
-    }
-    if (threadIdx.x == 0) { lds_st[0] = a.st[0]; lds_st[1] = a.st[2]; }
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        rz[q] = wave_sum(rz[q]);
-        if ((threadIdx.x & (WAVE - 1)) == 0) lds[q * (BLOCK / WAVE) + threadIdx.x / WAVE] = rz[q];
-    }
-    __syncthreads();
+    double rz[2];   // r_k.z_k, r_{k-1}.z_{k-1}
+    sum_partials_k<2, 2>({a.prz[h], a.prz[1 - h]}, {a.nb_rz, a.nb_rz}, 1, rz, lds, a.st, lds_st);
     const int it = lds_st[1];
     if (lds_st[0] != ST_RUNNING) return;
     if (it >= a.max_iter) {
@@ -595,16 +578,7 @@ k_fp_operator(PcgArgs a, int h) {
         return;
     }
     const bool first = it == 0;   // p and r_{k-1}.z_{k-1} are not set yet
-    double beta = 0.0;
-    if (!first) {
-        double now = 0.0, before = 0.0;
-#pragma unroll
-        for (int w = 0; w < BLOCK / WAVE; ++w) {
-            now += lds[w];
-            before += lds[BLOCK / WAVE + w];
-        }
-        beta = now / (before + 1.0e-30);
-    }
+    const double beta = first ? 0.0 : rz[0] / (rz[1] + 1.0e-30);
     double contrib = 0.0;
     for (;;) {
         double s[NV];
@@ -650,11 +624,26 @@ k_fp_operator(PcgArgs a, int h) {
 // the completed-iteration counter advances here.
 __global__ void __launch_bounds__(BLOCK)
 k_fp_update(PcgArgs a, int h, int nb_pq) {
-    __shared__ double lds[2 * BLOCK / WAVE];
-    int it;
-    if (block_state(a.st, &it) != ST_RUNNING) return;
+    __shared__ double lds[2 * BLOCK / WAVE], lds_rr[BLOCK / WAVE];
+    __shared__ int word[2];
+    const double* __restrict__ p = a.p[h];
+    const double* __restrict__ q = a.q;
+    double* __restrict__ x = a.x;
+    double* __restrict__ r = a.r;
+    int i = blockIdx.x * BLOCK + threadIdx.x;
+    double xi = 0.0, pi = 0.0, qi = 0.0, ri = 0.0;
+    auto load = [&] {
+        if (i >= a.n) return;
+        xi = x[i];
+        pi = p[i];
+        qi = q[i];
+        ri = r[i];
+    };
+    load();   // beside the sums
     double sums[2];   // p.q, r.z
-    sum_partials_k<2>({a.ppq, a.prz[h]}, {nb_pq, a.nb_rz}, 1, sums, lds);
+    sum_partials_k<2, 2>({a.ppq, a.prz[h]}, {nb_pq, a.nb_rz}, 1, sums, lds, a.st, word);
+    const int it = word[1];
+    if (word[0] != ST_RUNNING) return;
     const double pq = sums[0];
     if (fabs(pq) < 1.0e-30) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -665,33 +654,36 @@ k_fp_update(PcgArgs a, int h, int nb_pq) {
         return;
     }
     const double alpha = sums[1] / pq;
-    const double* __restrict__ p = a.p[h];
-    const double* __restrict__ q = a.q;
-    double* __restrict__ x = a.x;
-    double* __restrict__ r = a.r;
     double acc = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
-        x[i] += alpha * p[i];
-        const double ri = r[i] + (-alpha) * q[i];
-        r[i] = ri;
-        acc += ri * ri;
+    while (i < a.n) {
+        x[i] = xi + alpha * pi;
+        const double rn = ri + (-alpha) * qi;
+        r[i] = rn;
+        acc += rn * rn;
+        i += gridDim.x * BLOCK;
+        load();
     }
-    acc = block_sum(acc, lds);
+    acc = block_sum(acc, lds_rr);
     if (threadIdx.x == 0) {
         a.prr[blockIdx.x] = acc;
         if (blockIdx.x == 0) a.st[2] = it + 1;
     }
 }
 
-// Residual test of the iteration (||r|| < tol ||b||, linalg.cuh:241-247) from the r.r
-// partials; returns true (in every thread of every block) when the solve goes on.
-__device__ __forceinline__ bool fp_residual_test(const double* prr, int nb_rr, double* sc, int* st, int* status,
-                                                 double* lds) {
-    const double r_norm = sqrt(sum_partials(prr, nb_rr, 1, lds));
-    const bool done = r_norm < sc[S_TOL] * sc[S_BNORM];
+// Residual test of the iteration (||r|| < tol ||b||, linalg.cuh:241-247) from the r.r partials, with
+// the state word; true (in every thread of every block) when the solve goes on. Kernels compute their
+// rows before it, so that its round trip runs beside theirs. lds: BLOCK / WAVE doubles.
+__device__ __forceinline__ bool residual_test_running(const double* prr, int nb_rr, double* sc, int* st, int* status,
+                                                      double* lds, int* lds_state) {
+    const double bnorm = sc[S_BNORM], limit = sc[S_TOL] * bnorm;
+    double rr[1];
+    sum_partials_k<1, 1>({prr}, {nb_rr}, 1, rr, lds, st, lds_state);
+    if (*lds_state != ST_RUNNING) return false;
+    const double r_norm = sqrt(rr[0]);
+    const bool done = r_norm < limit;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc[S_RNORM] = r_norm;
-        sc[S_REL] = r_norm / sc[S_BNORM];
+        sc[S_REL] = r_norm / bnorm;
         const int it = st[2];
         if (done) {
             st[0] = ST_CONVERGED;
@@ -705,8 +697,8 @@ __device__ __forceinline__ bool fp_residual_test(const double* prr, int nb_rr, d
 // One-workgroup residual test, for preconditioners whose first kernel cannot take it
 __global__ void k_fp_check(const double* prr, int nb_rr, double* sc, int* st, int* status) {
     __shared__ double lds[BLOCK / WAVE];
-    if (block_state(st, nullptr) != ST_RUNNING) return;
-    (void)fp_residual_test(prr, nb_rr, sc, st, status, lds);
+    __shared__ int word;
+    (void)residual_test_running(prr, nb_rr, sc, st, status, lds, &word);
 }
 
 // First two V-cycle sweeps from x = 0 on level 0 (as k_jacobi_from_zero), preceded by the
@@ -718,8 +710,7 @@ k_jacobi_from_zero_check(int rows, const int* __restrict__ rp, const int* __rest
                          const double* __restrict__ dinv, double omega, double* __restrict__ y,
                          const double* __restrict__ prr, int nb_rr, double* sc, int* st, int* status) {
     __shared__ double lds[BLOCK / WAVE];
-    if (block_state(st, nullptr) != ST_RUNNING) return;
-    if (!fp_residual_test(prr, nb_rr, sc, st, status, lds)) return;
+    __shared__ int word;
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     const int row = g / TPR, lane = g % TPR;
     double s = 0.0;
@@ -727,6 +718,7 @@ k_jacobi_from_zero_check(int rows, const int* __restrict__ rp, const int* __rest
         row_entries<TPR>(ci, val, rp[row], rp[row + 1], lane,
                          [&](double a, int j) { s += a * (omega * dinv[j] * b[j]); });
     s = group_sum<TPR>(s);
+    if (!residual_test_running(prr, nb_rr, sc, st, status, lds, &word)) return;
     if (row >= rows || lane != 0) return;
     const double x0 = omega * dinv[row] * b[row];
     y[row] = x0 + omega * dinv[row] * (b[row] - s);
@@ -742,7 +734,7 @@ k_jacobi_dot(int rows, const int* __restrict__ rp, const int* __restrict__ ci, c
              double* __restrict__ y, const double* __restrict__ rdot, double* __restrict__ part,
              const int* __restrict__ st) {
     __shared__ double lds[BLOCK / WAVE];
-    if (st && block_state(st, nullptr) != ST_RUNNING) return;
+    if (halted(st)) return;   // nothing writes the state while this kernel runs
     const int groups = gridDim.x * (blockDim.x / TPR);
     const int lane = threadIdx.x % TPR;
     double contrib = 0.0;
@@ -871,13 +863,16 @@ k_sell_from_zero_check(int positions, const int* __restrict__ sp, const int* __r
                        const double* __restrict__ dinv, double omega, double* __restrict__ y,
                        const double* __restrict__ prr, int nb_rr, double* sc, int* st, int* status) {
     __shared__ double lds[BLOCK / WAVE];
-    if (block_state(st, nullptr) != ST_RUNNING) return;
-    if (!fp_residual_test(prr, nb_rr, sc, st, status, lds)) return;
+    __shared__ int word;
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= positions) return;
-    int row, base, len;
-    (void)sell_slot(sp, srow, p, nullptr, row, base, len);
-    const double s = sell_row_sum<MAXL, G, NT>(ci, val, base, len, [&](int j) { return omega * dinv[j] * b[j]; });
+    int row = -1;
+    double s = 0.0;
+    if (p < positions) {
+        int base, len;
+        (void)sell_slot(sp, srow, p, nullptr, row, base, len);
+        s = sell_row_sum<MAXL, G, NT>(ci, val, base, len, [&](int j) { return omega * dinv[j] * b[j]; });
+    }
+    if (!residual_test_running(prr, nb_rr, sc, st, status, lds, &word)) return;
     if (row < 0) return;
     const double x0 = omega * dinv[row] * b[row];
     y[row] = x0 + omega * dinv[row] * (b[row] - s);
@@ -935,35 +930,6 @@ __device__ __forceinline__ T lanes_row_sum(const int* __restrict__ ci, const T* 
     }
     for (int o = tpr >> 1; o > 0; o >>= 1) s += __shfl_down(s, o, tpr);
     return s;
-}
-
-// The iteration's residual test as fp_residual_test, with the state word read beside the partials:
-// one pair of barriers. True (in every thread of every block) when the solve goes on.
-__device__ __forceinline__ bool residual_test_running(const double* prr, int nb_rr, double* sc, int* st, int* status,
-                                                      double* lds, int* lds_state) {
-    double v = 0.0;
-    for (int k = threadIdx.x; k < nb_rr; k += BLOCK) v += prr[k];
-    if (threadIdx.x == 0) *lds_state = st[0];
-    v = wave_sum(v);
-    if ((threadIdx.x & (WAVE - 1)) == 0) lds[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    double rr = 0.0;
-#pragma unroll
-    for (int w = 0; w < BLOCK / WAVE; ++w) rr += lds[w];
-    if (*lds_state != ST_RUNNING) return false;
-    const double r_norm = sqrt(rr);
-    const bool done = r_norm < sc[S_TOL] * sc[S_BNORM];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        sc[S_RNORM] = r_norm;
-        sc[S_REL] = r_norm / sc[S_BNORM];
-        const int it = st[2];
-        if (done) {
-            st[0] = ST_CONVERGED;
-            st[1] = it;
-        }
-        publish(status, it, done ? ST_CONVERGED : ST_RUNNING);
-    }
-    return !done;
 }
 
 // MAXL, G: the sliced-ELL copy of level 0 (MAXL 0: none in this stage). Every value is computed
@@ -1182,9 +1148,11 @@ __global__ void k_sell_fill(int positions, const int* __restrict__ rp, const int
 __global__ void k_to_f32_check(int n, const double* __restrict__ r, float* __restrict__ b32,
                                const double* __restrict__ prr, int nb_rr, double* sc, int* st, int* status) {
     __shared__ double lds[BLOCK / WAVE];
-    if (st) {
-        if (block_state(st, nullptr) != ST_RUNNING) return;
-        if (prr && !fp_residual_test(prr, nb_rr, sc, st, status, lds)) return;
+    __shared__ int word;
+    if (st && prr) {
+        if (!residual_test_running(prr, nb_rr, sc, st, status, lds, &word)) return;
+    } else if (halted(st)) {
+        return;
     }
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) b32[i] = (float)r[i];
 }
@@ -1197,16 +1165,20 @@ __global__ void k_f64_to_f32(size_t n, const double* __restrict__ in, float* __r
 // Jacobi preconditioner z = D^-1 r with the r.z partials, optionally after the residual test
 __global__ void __launch_bounds__(BLOCK)
 k_fp_jacobi_prec(PcgArgs a, int h_next, int check) {
-    __shared__ double lds[BLOCK / WAVE];
-    if (block_state(a.st, nullptr) != ST_RUNNING) return;
-    if (check && !fp_residual_test(a.prr, a.nb_rr, a.sc, a.st, a.status, lds)) return;
+    __shared__ double lds[BLOCK / WAVE], lds_rz[BLOCK / WAVE];
+    __shared__ int word;
+    if (check) {
+        if (!residual_test_running(a.prr, a.nb_rr, a.sc, a.st, a.status, lds, &word)) return;
+    } else if (halted(a.st)) {
+        return;
+    }
     double acc = 0.0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
         const double zi = a.inv_diag[i] * a.r[i];
         a.z[i] = zi;
         acc += a.r[i] * zi;
     }
-    acc = block_sum(acc, lds);
+    acc = block_sum(acc, lds_rz);
     if (threadIdx.x == 0) a.prz[h_next][blockIdx.x] = acc;
 }
 
@@ -1621,35 +1593,45 @@ k_bicg_s(int n, const double* __restrict__ r, const double* __restrict__ v, doub
          double* __restrict__ s, double* __restrict__ part, int nb_a, const double* __restrict__ part_a,
          int* __restrict__ st, int* __restrict__ status) {
     __shared__ double lds[2 * BLOCK / WAVE];
-    __shared__ int s_state, s_act[2];
-    if (threadIdx.x == 0) { s_state = st[0]; s_act[0] = st[2]; s_act[1] = st[3]; }
-    __syncthreads();
-    if (s_state != ST_RUNNING) return;
+    __shared__ int word[3];
+    int i = blockIdx.x * BLOCK + threadIdx.x;
+    double ri = 0.0, vi = 0.0;
+    auto load = [&] {
+        if (i >= 2 * n) return;
+        ri = r[i];
+        vi = v[i];
+    };
+    load();   // beside the sums
+    const double bd[2] = {sc[B_BD], sc[B_BD + 1]}, rho[2] = {sc[B_RHO], sc[B_RHO + 1]};
     double ca[2];
     bool act[2];
     double o2[2];
-    sum_partials_k<2>({part_a, part_a + 1}, {nb_a, nb_a}, 6, o2, lds);
+    sum_partials_k<2, 3>({part_a, part_a + 1}, {nb_a, nb_a}, 6, o2, lds, st, word);
+    if (word[0] != ST_RUNNING) return;
+#pragma unroll
     for (int c = 0; c < 2; ++c) {
-        const double o = o2[c];
-        act[c] = s_act[c] && !(fabs(o) < sc[B_BD + c]);
-        ca[c] = act[c] ? sc[B_RHO + c] / o : 0.0;
+        act[c] = word[1 + c] && !(fabs(o2[c]) < bd[c]);
+        ca[c] = act[c] ? rho[c] / o2[c] : 0.0;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const int it = st[10];
         for (int c = 0; c < 2; ++c) {
             sc[B_CA + c] = ca[c];
-            if (s_act[c] && !act[c]) bicg_stop(st, c, it, 0);
+            if (word[1 + c] && !act[c]) bicg_stop(st, c, it, 0);
             if (act[c]) sc[B_ALPHA + c] = ca[c];
         }
         if (!(act[0] || act[1])) { st[0] = ST_STOPPED; publish(status, it, ST_STOPPED); }
     }
     if (!(act[0] || act[1])) return;
     double acc[1][2] = {{0.0, 0.0}};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 2 * n; i += gridDim.x * blockDim.x) {
+    while (i < 2 * n) {
         const int c = i >= n;
-        const double si = r[i] - ca[c] * v[i];
+        const double si = ri - (c ? ca[1] : ca[0]) * vi;
         s[i] = si;
-        acc[0][c] += si * si;
+        if (c) acc[0][1] += si * si;
+        else acc[0][0] += si * si;
+        i += gridDim.x * BLOCK;
+        load();
     }
     write_partials2<1>(part, acc, lds);
 }
@@ -1662,30 +1644,37 @@ k_bicg_xr(int n, const double* __restrict__ ph, const double* __restrict__ sh, c
           double* __restrict__ r, double* __restrict__ part, int nb_s, const double* __restrict__ part_s, int nb_t,
           const double* __restrict__ part_t, int* __restrict__ st) {
     __shared__ double lds[6 * BLOCK / WAVE];
-    __shared__ int s_state, s_act[2];
-    if (threadIdx.x == 0) { s_state = st[0]; s_act[0] = st[2]; s_act[1] = st[3]; }
-    __syncthreads();
-    if (s_state != ST_RUNNING) return;
-    double a1[2], a2[2], om[2];
-    int half[2];
+    __shared__ int word[3];
+    int i = blockIdx.x * BLOCK + threadIdx.x;
+    double xi = 0.0, pi = 0.0, hi = 0.0, si = 0.0, ti = 0.0, oi = 0.0;
+    auto load = [&] {
+        if (i >= 2 * n) return;
+        xi = x[i];
+        pi = ph[i];
+        hi = sh[i];
+        si = s[i];
+        ti = t[i];
+        oi = r0[i];
+    };
+    load();   // beside the sums
+    const double tol = sc[B_TOL], rn0[2] = {sc[B_RN0], sc[B_RN0 + 1]}, bd[2] = {sc[B_BD], sc[B_BD + 1]},
+                 alpha[2] = {sc[B_ALPHA], sc[B_ALPHA + 1]};
     double sums[6];   // s.s, t.t, t.s of both components
-    sum_partials_k<6>({part_s, part_s + 1, part_t, part_t + 1, part_t + 2, part_t + 3},
-                      {nb_s, nb_s, nb_t, nb_t, nb_t, nb_t}, 6, sums, lds);
+    sum_partials_k<6, 3>({part_s, part_s + 1, part_t, part_t + 1, part_t + 2, part_t + 3},
+                         {nb_s, nb_s, nb_t, nb_t, nb_t, nb_t}, 6, sums, lds, st, word);
+    if (word[0] != ST_RUNNING) return;
+    double a1[2], a2[2];
+    int half[2];
+#pragma unroll
     for (int c = 0; c < 2; ++c) {
-        const double ss = sums[c];
-        const double tt = sums[2 + c];
-        const double ts = sums[4 + c];
-        a1[c] = a2[c] = om[c] = 0.0;
+        const double ss = sums[c], tt = sums[2 + c], ts = sums[4 + c];
+        a1[c] = a2[c] = 0.0;
         half[c] = 0;
-        if (!s_act[c]) continue;
-        a1[c] = sc[B_ALPHA + c];
+        if (!word[1 + c]) continue;
+        a1[c] = alpha[c];
         const double s_norm = sqrt(ss);
-        if (s_norm < sc[B_TOL] * sc[B_RN0 + c] || s_norm < 1.0e-11) {
-            half[c] = 1;
-            continue;
-        }
-        om[c] = (tt > sc[B_BD + c]) ? (ts / tt) : 0.0;
-        a2[c] = om[c];
+        if (s_norm < tol * rn0[c] || s_norm < 1.0e-11) half[c] = 1;
+        else a2[c] = (tt > bd[c]) ? (ts / tt) : 0.0;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0)
         for (int c = 0; c < 2; ++c) {
@@ -1693,47 +1682,92 @@ k_bicg_xr(int n, const double* __restrict__ ph, const double* __restrict__ sh, c
             sc[B_A2 + c] = a2[c];
             sc[B_CW + c] = a2[c];
             st[8 + c] = half[c];
-            if (s_act[c] && !half[c]) sc[B_OMEGA + c] = om[c];
+            if (word[1 + c] && !half[c]) sc[B_OMEGA + c] = a2[c];
         }
     double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 2 * n; i += gridDim.x * blockDim.x) {
+    while (i < 2 * n) {
         const int c = i >= n;
-        x[i] += a1[c] * ph[i] + a2[c] * sh[i];
-        const double ri = s[i] - a2[c] * t[i];
+        x[i] = xi + ((c ? a1[1] : a1[0]) * pi + (c ? a2[1] : a2[0]) * hi);
+        const double ri = si - (c ? a2[1] : a2[0]) * ti;
         r[i] = ri;
-        acc[0][c] += ri * ri;
-        acc[1][c] += r0[i] * ri;
+        if (c) {
+            acc[0][1] += ri * ri;
+            acc[1][1] += oi * ri;
+        } else {
+            acc[0][0] += ri * ri;
+            acc[1][0] += oi * ri;
+        }
+        i += gridDim.x * BLOCK;
+        load();
     }
     write_partials2<2>(part, acc, lds);
 }
 
 // end of an iteration: half-step stops, residual test, rho update, iteration cap; then the start
-// of the next one (breakdown check on rho, p-update coefficients)
+// of the next one (breakdown check on rho, p-update coefficients). The scalars and state are loaded
+// beside the partials, decided on in registers and written once.
 __global__ void k_bicg_final_post(int nb, const double* __restrict__ part, double* __restrict__ sc,
                                   int* __restrict__ st, int* __restrict__ status) {
     __shared__ double lds[4 * BLOCK / WAVE];
-    if (st[0] != ST_RUNNING) return;
+    double rho[2], rn0[2], bd[2], alpha[2], omega[2];
+    int act[2], half[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        rho[c] = sc[B_RHO + c];
+        rn0[c] = sc[B_RN0 + c];
+        bd[c] = sc[B_BD + c];
+        alpha[c] = sc[B_ALPHA + c];
+        omega[c] = sc[B_OMEGA + c];
+        act[c] = st[2 + c];
+        half[c] = st[8 + c];
+    }
+    const double tol = sc[B_TOL];
+    const int state0 = st[0], it = st[10], max_iter = st[11];
     double sums[4];
     sum_partials_k<4>({part, part + 1, part + 2, part + 3}, {nb, nb, nb, nb}, 6, sums, lds);
+    if (state0 != ST_RUNNING || threadIdx.x != 0) return;
     const double rr[2] = {sums[0], sums[1]}, r0r[2] = {sums[2], sums[3]};
-    if (threadIdx.x != 0) return;
-    const int it = st[10], max_iter = st[11];
-    for (int c = 0; c < 2; ++c)
-        if (st[8 + c]) bicg_stop(st, c, it + 1, 1);
+    double rho_old[2];
     for (int c = 0; c < 2; ++c) {
-        if (!st[2 + c]) continue;
+        rho_old[c] = rho[c];
+        if (half[c]) {
+            bicg_stop(st, c, it + 1, 1);
+            act[c] = 0;
+        }
+        if (!act[c]) continue;
         const double r_norm = sqrt(rr[c]);
-        sc[B_REL + c] = r_norm / sc[B_RN0 + c];
-        if (r_norm < sc[B_TOL] * sc[B_RN0 + c] || r_norm < 1.0e-11) { bicg_stop(st, c, it + 1, 1); continue; }
-        sc[B_RHO_OLD + c] = sc[B_RHO + c];
-        sc[B_RHO + c] = r0r[c];
-        if (it + 1 == max_iter) bicg_stop(st, c, max_iter, 0);
+        sc[B_REL + c] = r_norm / rn0[c];
+        if (r_norm < tol * rn0[c] || r_norm < 1.0e-11) {
+            bicg_stop(st, c, it + 1, 1);
+            act[c] = 0;
+            continue;
+        }
+        rho[c] = r0r[c];
+        sc[B_RHO_OLD + c] = rho_old[c];
+        sc[B_RHO + c] = rho[c];
+        if (it + 1 == max_iter) {
+            bicg_stop(st, c, max_iter, 0);
+            act[c] = 0;
+        }
     }
     st[10] = it + 1;
-    const int state = (st[2] || st[3]) ? ST_RUNNING : ST_STOPPED;
+    if (act[0] || act[1])   // start of the next iteration (bicg_pre_logic)
+        for (int c = 0; c < 2; ++c) {
+            double cb = 0.0, co = 0.0;
+            if (act[c] && fabs(rho[c]) < bd[c]) {
+                bicg_stop(st, c, it + 1, 0);
+                act[c] = 0;
+            }
+            if (act[c]) {
+                cb = (rho[c] / rho_old[c]) * (alpha[c] / (omega[c] + 1.0e-30));
+                co = omega[c];
+            }
+            sc[B_CB + c] = cb;
+            sc[B_CO + c] = co;
+        }
+    const int state = act[0] || act[1] ? ST_RUNNING : ST_STOPPED;
     st[0] = state;
     publish(status, it + 1, state);
-    bicg_pre_logic(sc, st, status);   // start of the next iteration
 }
 
 // ======================================================================================================
