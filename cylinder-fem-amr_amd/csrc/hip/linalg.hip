@@ -1291,6 +1291,15 @@ __global__ void k_ilu_unpermute(int n, const int* __restrict__ pos, const double
     for (int c = 0; c < NRHS; ++c) z[(size_t)c * n + i] = zp[(size_t)c * n + q];
 }
 
+// One entry's move into colour order with the forward sweep of colour 0: position q (at index k of
+// the component's vectors) below m0 goes to z (times dinv when colour 0 is also the last), else to r
+template <typename T>
+__device__ __forceinline__ void ilu_permuted_entry(size_t k, int q, int m0, int last, const T* __restrict__ dinv,
+                                                   double v, double* __restrict__ rp, double* __restrict__ zp) {
+    if (q >= m0) rp[k] = v;
+    else zp[k] = last ? v * (double)dinv[q] : v;
+}
+
 // The permutation into colour order fused with the forward sweep of colour 0. L holds the columns
 // of earlier colours, so colour 0 has no L entries and its sweep is z = r (times dinv when it is
 // also the last colour): its z entries are written here, and its r entries are not needed.
@@ -1302,17 +1311,9 @@ __global__ void k_ilu_permute_first(int n, int m0, const int* __restrict__ pos, 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int q = pos[i];
-    if (q < m0) {
-        const double d = (double)dinv[q];
 #pragma unroll
-        for (int c = 0; c < NRHS; ++c) {
-            const double acc = r[(size_t)c * n + i];
-            zp[(size_t)c * n + q] = last ? acc * d : acc;
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < NRHS; ++c) rp[(size_t)c * n + q] = r[(size_t)c * n + i];
-    }
+    for (int c = 0; c < NRHS; ++c)
+        ilu_permuted_entry((size_t)c * n + q, q, m0, last, dinv, r[(size_t)c * n + i], rp, zp);
 }
 
 // The backward sweep of colour 0 fused with the permutation back to row order, one thread per
@@ -1425,6 +1426,51 @@ k_ilu_lower_lanes(int m, int n, int cs, const int* __restrict__ lp, const int* _
     }
 }
 
+// The trailing colours of at most ILU_TAIL_ROWS rows each (greedy colouring leaves two or three of the
+// five or six with few rows), forward t..nc-1 and backward nc-2..t, in one launch: one workgroup with
+// a barrier between colours instead of a launch per colour and direction, since such a launch is all
+// latency. Each row is k_ilu_lower's and k_ilu_upper's, in their order. Uniform level 4 (two colours of
+// under 256 rows): 5.0 + 2.8 + 1.9 us and two gaps -> 7.9 us. A row per lane: with colours of 1280
+// and 2560 rows the workgroup took 24 and 63 us for what separate launches do in 12 and 23.
+constexpr int ILU_TAIL_ROWS = 1024;
+constexpr int ILU_TAIL_THREADS = 1024;
+constexpr int ILU_TAIL_COLOURS = 16;
+struct IluTail {
+    int first, nc;
+    int start[ILU_TAIL_COLOURS + 1];   // colour_start of colours first .. nc
+};
+template <int NRHS, typename T>
+__global__ void __launch_bounds__(ILU_TAIL_THREADS)
+k_ilu_tail(int n, IluTail a, const int* __restrict__ lp, const int* __restrict__ lc, const T* __restrict__ lv,
+           const int* __restrict__ up, const int* __restrict__ uc, const T* __restrict__ uv,
+           const T* __restrict__ dinv, const double* __restrict__ r, double* z, const int* __restrict__ st) {
+    if (halted(st)) return;
+    const int colours = a.nc - a.first;
+    for (int k = 0; k < 2 * colours - 1; ++k) {
+        const bool lower = k < colours;
+        const int c = lower ? k : 2 * colours - 2 - k;
+        const bool last = c == colours - 1;
+        const int* ptr = lower ? lp : up;
+        const int* col = lower ? lc : uc;
+        const T* val = lower ? lv : uv;
+        const double* src = lower ? r : z;
+        if (k > 0) __syncthreads();
+        for (int i = a.start[c] + (int)threadIdx.x; i < a.start[c + 1]; i += ILU_TAIL_THREADS) {
+            double acc[NRHS];
+#pragma unroll
+            for (int q = 0; q < NRHS; ++q) acc[q] = src[(size_t)q * n + i];
+            row_entries<1>(col, val, ptr[i], ptr[i + 1], 0, [&](T vt, int j) {
+                const double v = (double)vt;
+#pragma unroll
+                for (int q = 0; q < NRHS; ++q) acc[q] -= v * z[(size_t)q * n + j];
+            });
+            const double d = (double)dinv[i];
+#pragma unroll
+            for (int q = 0; q < NRHS; ++q) z[(size_t)q * n + i] = !lower || last ? acc[q] * d : acc[q];
+        }
+    }
+}
+
 // ======================================================================================================
 // Two-component BiCGSTAB (src/cfa/linalg.cuh:642-779)
 // ======================================================================================================
@@ -1451,33 +1497,54 @@ __device__ __forceinline__ void write_partials2(double* part, double (&acc)[NQ][
         for (int k = 0; k < 2 * NQ; ++k) part[(size_t)blockIdx.x * 6 + k] = v[k];
 }
 
+// Both components' products of a run of RB rows (one workgroup, k_apply_K_B's scheme): the lane's row
+// and component (part 0 and 1 of the workgroup) and its sum; prod: 2 RUN_TILE(RB) doubles
+template <int RB>
+__device__ __forceinline__ double run_product2(int n, const int* __restrict__ rp, const int* __restrict__ ci,
+                                               const double* __restrict__ val, const double* __restrict__ x, int r0,
+                                               double* prod) {
+    const RowValues<1, double> av{{val}};
+    const int row = r0 + (int)threadIdx.x % RB, e0 = rp[r0], e1 = rp[min(r0 + RB, n)];
+    const int k0 = row < n ? rp[row] : e1, k1 = row < n ? rp[row + 1] : e1;
+    double s[2] = {0.0, 0.0};
+    for (int t = e0; t < e1; t += RUN_TILE(RB)) {
+        RunTile<RB, 1> tile;
+        tile.load(ci, av, t, e1);
+#pragma unroll
+        for (int u = 0; u < RUN_SLOTS(RB); ++u) {
+            const int at = u * BLOCK + threadIdx.x, j = tile.c[u];
+            prod[at] = tile.v[u][0] * x[j];
+            prod[RUN_TILE(RB) + at] = tile.v[u][0] * x[n + j];
+        }
+        __syncthreads();
+        run_row_sums<RB, 2>(prod, t, k0, k1, s);
+        __syncthreads();
+    }
+    return run_part_has<RB>(0) ? s[0] : s[1];
+}
+
 // r = b - A x (both components), r0 = p = r, v = 0; partial r.r
-template <int TPR>
+template <int RB>
 __global__ void __launch_bounds__(BLOCK)
 k_bicg_init(int n, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ val,
             const double* __restrict__ b, const double* __restrict__ x, double* __restrict__ r,
-            double* __restrict__ r0, double* __restrict__ p, double* __restrict__ v, double* __restrict__ part) {
+            double* __restrict__ r0v, double* __restrict__ p, double* __restrict__ v, double* __restrict__ part) {
+    __shared__ double prod[2 * RUN_TILE(RB)];
     __shared__ double lds[2 * BLOCK / WAVE];
-    const int groups = gridDim.x * (blockDim.x / TPR);
-    const int g0 = (blockIdx.x * blockDim.x + threadIdx.x) / TPR, lane = threadIdx.x % TPR;
+    const int c = threadIdx.x / RB;
     double acc[1][2] = {{0.0, 0.0}};
-    for (int row = g0; row < n; row += groups) {
-        double s0 = 0.0, s1 = 0.0;
-        row_entries<TPR>(ci, val, rp[row], rp[row + 1], lane, [&](double a, int j) {
-            s0 += a * x[j];
-            s1 += a * x[n + j];
-        });
-        s0 = group_sum<TPR>(s0);
-        s1 = group_sum<TPR>(s1);
-        if (lane == 0) {
-            const double q0 = b[row] - 1.0 * s0, q1 = b[n + row] - 1.0 * s1;
-            r[row] = q0;  r[n + row] = q1;
-            r0[row] = q0; r0[n + row] = q1;
-            p[row] = q0;  p[n + row] = q1;
-            v[row] = 0.0; v[n + row] = 0.0;
-            acc[0][0] += q0 * q0;
-            acc[0][1] += q1 * q1;
-        }
+    for (int r0 = blockIdx.x * RB; r0 < n; r0 += gridDim.x * RB) {
+        const double s = run_product2<RB>(n, rp, ci, val, x, r0, prod);
+        const int row = r0 + (int)threadIdx.x % RB;
+        if (c > 1 || row >= n) continue;
+        const int i = c * n + row;
+        const double q = b[i] - s;
+        r[i] = q;
+        r0v[i] = q;
+        p[i] = q;
+        v[i] = 0.0;
+        if (c) acc[0][1] += q * q;
+        else acc[0][0] += q * q;
     }
     write_partials2<1>(part, acc, lds);
 }
@@ -1533,49 +1600,57 @@ __global__ void k_bicg_pre(double* __restrict__ sc, int* __restrict__ st, int* _
     bicg_pre_logic(sc, st, status);
 }
 
-// p = r + cb (p - co v), from the second iteration on
-__global__ void k_bicg_p(int n, const double* __restrict__ r, const double* __restrict__ v,
-                         const double* __restrict__ sc, double* __restrict__ p, const int* __restrict__ st) {
-    if (halted(st) || st[10] == 0) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 2 * n) return;
-    const int c = i >= n;
-    p[i] = r[i] + sc[B_CB + c] * (p[i] - sc[B_CO + c] * v[i]);
+// p = r + cb (p - co v), from the second iteration on, and the permutation of p into colour order with
+// the forward sweep of colour 0 (k_ilu_permute_first), one thread per row for both components
+template <typename T>
+__global__ void __launch_bounds__(BLOCK)
+k_bicg_p(int n, const double* __restrict__ r, const double* __restrict__ v, const double* __restrict__ sc,
+         double* __restrict__ p, int m0, const int* __restrict__ pos, const T* __restrict__ dinv, int last,
+         double* __restrict__ rp, double* __restrict__ zp, const int* __restrict__ st) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    const int state = st[0], it = st[10];
+    if (state != ST_RUNNING || i >= n) return;
+    const int q = pos[i];
+    double pv[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int k = c * n + i;
+        pv[c] = it > 0 ? r[k] + sc[B_CB + c] * (p[k] - sc[B_CO + c] * v[k]) : p[k];
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        if (it > 0) p[c * n + i] = pv[c];
+        ilu_permuted_entry(c * n + q, q, m0, last, dinv, pv[c], rp, zp);
+    }
 }
 
-// y = A x for both components; with dots: partial y.w0 (mode 1) or y.y, y.w0 (mode 2)
-template <int TPR>
+// y = A x for both components; with dots: partial y.w0 (mode 1) or y.y, y.w0 (mode 2). Row runs
+// through LDS (k_apply_K_B's scheme; two lanes per row took 82 us on 1.84 M nodes, 20 us on 461k)
+template <int RB>
 __global__ void __launch_bounds__(BLOCK)
 k_spmv2_dots(int n, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ val,
              const double* __restrict__ x, double* __restrict__ y, const double* __restrict__ w0, int mode,
              double* __restrict__ part, const int* __restrict__ st) {
+    __shared__ double prod[2 * RUN_TILE(RB)];
     __shared__ double lds[4 * BLOCK / WAVE];
     if (halted(st)) return;
-    const int groups = gridDim.x * (blockDim.x / TPR);
-    const int g0 = (blockIdx.x * blockDim.x + threadIdx.x) / TPR, lane = threadIdx.x % TPR;
-    double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-    for (int row = g0; row < n; row += groups) {
-        double s0 = 0.0, s1 = 0.0;
-        row_entries<TPR>(ci, val, rp[row], rp[row + 1], lane, [&](double a, int j) {
-            s0 += a * x[j];
-            s1 += a * x[n + j];
-        });
-        s0 = group_sum<TPR>(s0);
-        s1 = group_sum<TPR>(s1);
-        if (lane == 0) {
-            y[row] = s0;
-            y[n + row] = s1;
-            if (mode == 1) {   // r0 . v
-                acc[0][0] += w0[row] * s0;
-                acc[0][1] += w0[n + row] * s1;
-            } else {           // t . t, t . s
-                acc[0][0] += s0 * s0;
-                acc[0][1] += s1 * s1;
-                acc[1][0] += s0 * w0[row];
-                acc[1][1] += s1 * w0[n + row];
-            }
+    const int c = threadIdx.x / RB;
+    double dot0 = 0.0, dot1 = 0.0;   // of the lane's component
+    for (int r0 = blockIdx.x * RB; r0 < n; r0 += gridDim.x * RB) {
+        const int row = r0 + (int)threadIdx.x % RB, i = c * n + row;
+        const bool own = c < 2 && row < n;
+        const double wi = own ? w0[i] : 0.0;
+        const double s = run_product2<RB>(n, rp, ci, val, x, r0, prod);
+        if (!own) continue;
+        y[i] = s;
+        if (mode == 1) {   // r0 . v
+            dot0 += wi * s;
+        } else {           // t . t, t . s
+            dot0 += s * s;
+            dot1 += s * wi;
         }
     }
+    double acc[2][2] = {{c == 0 ? dot0 : 0.0, c == 1 ? dot0 : 0.0}, {c == 0 ? dot1 : 0.0, c == 1 ? dot1 : 0.0}};
     if (mode == 1) write_partials2<1>(part, reinterpret_cast<double(&)[1][2]>(acc), lds);
     else write_partials2<2>(part, acc, lds);
 }
@@ -1586,20 +1661,27 @@ k_spmv2_dots(int n, const int* __restrict__ rp, const int* __restrict__ ci, cons
 // as an already inactive one (zero coefficient), so a block that reads the state before or after
 // block 0's write computes the same values.
 
-// alpha = rho / (r0 . v) with the breakdown guard (from the r0.v partials), then s = r - alpha v
-// and the s.s partials
+// alpha = rho / (r0 . v) with the breakdown guard (from the r0.v partials), then s = r - alpha v, the
+// s.s partials, and the permutation of s into colour order with the forward sweep of colour 0, one
+// thread per row for both components
+template <typename T>
 __global__ void __launch_bounds__(BLOCK)
 k_bicg_s(int n, const double* __restrict__ r, const double* __restrict__ v, double* __restrict__ sc,
          double* __restrict__ s, double* __restrict__ part, int nb_a, const double* __restrict__ part_a,
-         int* __restrict__ st, int* __restrict__ status) {
+         int m0, const int* __restrict__ pos, const T* __restrict__ dinv, int last, double* __restrict__ rp,
+         double* __restrict__ zp, int* __restrict__ st, int* __restrict__ status) {
     __shared__ double lds[2 * BLOCK / WAVE];
     __shared__ int word[3];
-    int i = blockIdx.x * BLOCK + threadIdx.x;
-    double ri = 0.0, vi = 0.0;
+    int i = blockIdx.x * BLOCK + threadIdx.x, q = 0;
+    double ri[2] = {0.0, 0.0}, vi[2] = {0.0, 0.0};
     auto load = [&] {
-        if (i >= 2 * n) return;
-        ri = r[i];
-        vi = v[i];
+        if (i >= n) return;
+        q = pos[i];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            ri[c] = r[c * n + i];
+            vi[c] = v[c * n + i];
+        }
     };
     load();   // beside the sums
     const double bd[2] = {sc[B_BD], sc[B_BD + 1]}, rho[2] = {sc[B_RHO], sc[B_RHO + 1]};
@@ -1624,12 +1706,14 @@ k_bicg_s(int n, const double* __restrict__ r, const double* __restrict__ v, doub
     }
     if (!(act[0] || act[1])) return;
     double acc[1][2] = {{0.0, 0.0}};
-    while (i < 2 * n) {
-        const int c = i >= n;
-        const double si = ri - (c ? ca[1] : ca[0]) * vi;
-        s[i] = si;
-        if (c) acc[0][1] += si * si;
-        else acc[0][0] += si * si;
+    while (i < n) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const double si = ri[c] - ca[c] * vi[c];
+            s[c * n + i] = si;
+            acc[0][c] += si * si;
+            ilu_permuted_entry(c * n + q, q, m0, last, dinv, si, rp, zp);
+        }
         i += gridDim.x * BLOCK;
         load();
     }
@@ -2204,18 +2288,25 @@ void amg_apply_enqueue(const cfa_amg_t* amg, const double* r, double* z, const i
     }
 }
 
+// First colour of the trailing run that k_ilu_tail takes (n_colours when fewer than two colours qualify)
+int ilu_tail_first(const cfa_ilu_t* ilu) {
+    const int nc = ilu->n_colours;
+    int t = nc;
+    while (t > 1 && nc - t < ILU_TAIL_COLOURS && ilu->colour_start[t] - ilu->colour_start[t - 1] <= ILU_TAIL_ROWS) --t;
+    return nc - t >= 2 ? t : nc;
+}
+
+// The sweeps after the permutation into colour order (r_perm, and colour 0 in z_perm): colours 1..
+// forward, colours nc-2..1 backward (the trailing small ones in one launch), colour 0 backward with the
+// permutation back (the last colour has no U entries)
 template <int NRHS, typename T>
-void ilu_apply_impl(const cfa_ilu_t* ilu, const T* lv, const T* uv, const T* dinv, const double* r, double* z,
-                    const int* st, hipStream_t s) {
+void ilu_sweeps(const cfa_ilu_t* ilu, const T* lv, const T* uv, const T* dinv, double* z, const int* st,
+                hipStream_t s) {
     const int nc = ilu->n_colours, n = ilu->n;
-    if (n == 0 || nc == 0) return;
+    if (nc == 0) return;
     double* rp = ilu->r_perm;
     double* zp = ilu->z_perm;
     const int m0 = ilu->colour_start[1] - ilu->colour_start[0];
-    // colour 0 forward with the permutation, colours 1.. forward, colours nc-2..1 backward, colour 0
-    // backward with the permutation back (the last colour has no U entries)
-    hipLaunchKernelGGL((k_ilu_permute_first<NRHS, T>), dim3(blocks_for(n)), dim3(BLOCK), 0, s, n, m0, ilu->pos, r,
-                       dinv, nc == 1 ? 1 : 0, rp, zp, st);
     // forward sweeps with the FP32 factors (mixed precision): two lanes per row; FP64: one lane, the
     // reference's order (the backward sweeps take one lane either way: two were no faster)
     constexpr bool lanes = std::is_same<T, float>::value;
@@ -2236,7 +2327,8 @@ void ilu_apply_impl(const cfa_ilu_t* ilu, const T* lv, const T* uv, const T* din
         else if (len <= 12) go(std::integral_constant<int, 12>{});
         else go(std::integral_constant<int, 16>{});
     };
-    for (int c = 1; c < nc; ++c) {
+    const int tail = ilu_tail_first(ilu);
+    for (int c = 1; c < tail; ++c) {
         const int cs = ilu->colour_start[c], m = ilu->colour_start[c + 1] - cs;
         if (m == 0) continue;
         if (!lanes && sell_l)
@@ -2248,7 +2340,15 @@ void ilu_apply_impl(const cfa_ilu_t* ilu, const T* lv, const T* uv, const T* din
             hipLaunchKernelGGL((k_ilu_lower<NRHS, T>), dim3(blocks_for(m)), dim3(BLOCK), 0, s, m, n, cs, ilu->lp + cs,
                                ilu->lc, lv, dinv + cs, c == nc - 1 ? 1 : 0, rp, zp, st);
     }
-    for (int c = nc - 2; c >= 1; --c) {
+    if (tail < nc) {
+        IluTail a;
+        a.first = tail;
+        a.nc = nc;
+        for (int c = tail; c <= nc; ++c) a.start[c - tail] = ilu->colour_start[c];
+        hipLaunchKernelGGL((k_ilu_tail<NRHS, T>), dim3(1), dim3(ILU_TAIL_THREADS), 0, s, n, a, ilu->lp, ilu->lc, lv,
+                           ilu->up, ilu->uc, uv, dinv, rp, zp, st);
+    }
+    for (int c = std::min(nc - 2, tail - 1); c >= 1; --c) {
         const int cs = ilu->colour_start[c], m = ilu->colour_start[c + 1] - cs;
         if (m == 0) continue;
         if (sell_u) {
@@ -2265,15 +2365,24 @@ void ilu_apply_impl(const cfa_ilu_t* ilu, const T* lv, const T* uv, const T* din
         hipLaunchKernelGGL((k_ilu_unpermute<NRHS>), dim3(blocks_for(n)), dim3(BLOCK), 0, s, n, ilu->pos, zp, z, st);
 }
 
-void ilu_apply_any(const cfa_ilu_t* ilu, int use_f32, const double* r, double* z, int nrhs, const int* st,
-                   hipStream_t s) {
-    if (use_f32 && ilu->lv32) {
-        if (nrhs == 2) ilu_apply_impl<2, float>(ilu, ilu->lv32, ilu->uv32, ilu->dinv32, r, z, st, s);
-        else ilu_apply_impl<1, float>(ilu, ilu->lv32, ilu->uv32, ilu->dinv32, r, z, st, s);
-    } else {
-        if (nrhs == 2) ilu_apply_impl<2, double>(ilu, ilu->lv, ilu->uv, ilu->dinv, r, z, st, s);
-        else ilu_apply_impl<1, double>(ilu, ilu->lv, ilu->uv, ilu->dinv, r, z, st, s);
-    }
+// Calls f with the factor's values in the precision applied: (lv, uv, dinv)
+template <typename F>
+void ilu_values(const cfa_ilu_t* ilu, int use_f32, F f) {
+    if (use_f32 && ilu->lv32) f((const float*)ilu->lv32, (const float*)ilu->uv32, (const float*)ilu->dinv32);
+    else f((const double*)ilu->lv, (const double*)ilu->uv, (const double*)ilu->dinv);
+}
+
+template <int NRHS>
+void ilu_apply_impl(const cfa_ilu_t* ilu, const double* r, double* z, hipStream_t s) {
+    const int nc = ilu->n_colours, n = ilu->n;
+    if (n == 0 || nc == 0) return;
+    ilu_values(ilu, 0, [&](auto lv, auto uv, auto dinv) {
+        using T = typename std::remove_const<typename std::remove_pointer<decltype(lv)>::type>::type;
+        hipLaunchKernelGGL((k_ilu_permute_first<NRHS, T>), dim3(blocks_for(n)), dim3(BLOCK), 0, s, n,
+                           ilu->colour_start[1] - ilu->colour_start[0], ilu->pos, r, dinv, nc == 1 ? 1 : 0, ilu->r_perm,
+                           ilu->z_perm, nullptr);
+        ilu_sweeps<NRHS, T>(ilu, lv, uv, dinv, z, nullptr, s);
+    });
 }
 
 // Host wait on the progress word: returns when progress >= target, the solve stopped, or the
@@ -2862,7 +2971,8 @@ int cfa_ilu0_apply(const cfa_ilu_t* ilu, const double* r, double* z, int nrhs, c
         !ilu->z_perm)
         return CFA_E_ARG;
     if (ilu->n == 0) return CFA_OK;
-    ilu_apply_any(ilu, 0, r, z, nrhs, nullptr, S(stream));
+    if (nrhs == 2) ilu_apply_impl<2>(ilu, r, z, S(stream));
+    else ilu_apply_impl<1>(ilu, r, z, S(stream));
     return launch_status();
 }
 
@@ -2903,30 +3013,19 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
     ws->status_host[0] = 0;
     ws->status_host[1] = ST_RUNNING;
 
-    // 2 lanes per row for rows of about 7 entries (4 for longer ones): with the partial sums
-    // capped at RED_BLOCKS workgroups, 2 lanes also keep one row per group up to 131k rows
-    int nnz = 0;
-    CFA_TRY(hipMemcpyAsync(&nnz, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
-    CFA_TRY(hipStreamSynchronize(s));
-    const int TPR = operator_lanes(n, nnz);
-    const int groups_per_block = BLOCK / TPR;
-    const int nb_rows = std::min((n + groups_per_block - 1) / groups_per_block, RED_BLOCKS);
-    const int nb2 = red_blocks(2LL * n);
-    const int blocks2 = blocks_for(2LL * n);
+    const int nb_rows = run_blocks(n), nb1 = red_blocks(n), nb2 = red_blocks(2LL * n);
     auto spmv2_dots = [&](const double* xin, double* yout, const double* w0, int mode, double* partials,
                           hipStream_t q_s) {
-        if (TPR == 2)
-            hipLaunchKernelGGL(k_spmv2_dots<2>, dim3(nb_rows), dim3(BLOCK), 0, q_s, n, rp, ci, val, xin, yout, w0, mode,
-                               partials, st);
-        else
-            hipLaunchKernelGGL(k_spmv2_dots<4>, dim3(nb_rows), dim3(BLOCK), 0, q_s, n, rp, ci, val, xin, yout, w0, mode,
-                               partials, st);
+        run_dispatch(n, [&](auto rb) {
+            constexpr int RB = decltype(rb)::value;
+            hipLaunchKernelGGL(k_spmv2_dots<RB>, dim3(nb_rows), dim3(BLOCK), 0, q_s, n, rp, ci, val, xin, yout, w0,
+                               mode, partials, st);
+        });
     };
-
-    if (TPR == 2)
-        hipLaunchKernelGGL(k_bicg_init<2>, dim3(nb_rows), dim3(BLOCK), 0, s, n, rp, ci, val, bb, x, r, r0, p, v, part_a);
-    else
-        hipLaunchKernelGGL(k_bicg_init<4>, dim3(nb_rows), dim3(BLOCK), 0, s, n, rp, ci, val, bb, x, r, r0, p, v, part_a);
+    run_dispatch(n, [&](auto rb) {
+        constexpr int RB = decltype(rb)::value;
+        hipLaunchKernelGGL(k_bicg_init<RB>, dim3(nb_rows), dim3(BLOCK), 0, s, n, rp, ci, val, bb, x, r, r0, p, v, part_a);
+    });
     hipLaunchKernelGGL(k_bicg_final_init, dim3(1), dim3(BLOCK), 0, s, nb_rows, part_a, sc, st, status, max_iter);
     hipLaunchKernelGGL(k_bicg_pre, dim3(1), dim3(1), 0, s, sc, st, status);
     int rc = launch_status();
@@ -2934,21 +3033,27 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
 
     // one iteration for both components (src/cfa/linalg.cuh:700-775)
     auto iteration = [&](hipStream_t q_s) {
-        hipLaunchKernelGGL(k_bicg_p, dim3(blocks2), dim3(BLOCK), 0, q_s, n, r, v, sc, p, st);
-        ilu_apply_any(ilu, use_f32, p, ph, 2, st, q_s);
-        spmv2_dots(ph, v, r0, 1, part_a, q_s);
-        hipLaunchKernelGGL(k_bicg_s, dim3(nb2), dim3(BLOCK), 0, q_s, n, r, v, sc, sv, part_b, nb_rows, part_a, st,
-                           status);
-        ilu_apply_any(ilu, use_f32, sv, sh, 2, st, q_s);
+        ilu_values(ilu, use_f32, [&](auto lv, auto uv, auto dinv) {
+            using T = typename std::remove_const<typename std::remove_pointer<decltype(lv)>::type>::type;
+            const int m0 = ilu->n_colours ? ilu->colour_start[1] - ilu->colour_start[0] : 0,
+                      last = ilu->n_colours == 1 ? 1 : 0;
+            hipLaunchKernelGGL(k_bicg_p<T>, dim3(blocks_for(n)), dim3(BLOCK), 0, q_s, n, r, v, sc, p, m0, ilu->pos, dinv,
+                               last, ilu->r_perm, ilu->z_perm, st);
+            ilu_sweeps<2, T>(ilu, lv, uv, dinv, ph, st, q_s);
+            spmv2_dots(ph, v, r0, 1, part_a, q_s);
+            hipLaunchKernelGGL(k_bicg_s<T>, dim3(nb1), dim3(BLOCK), 0, q_s, n, r, v, sc, sv, part_b, nb_rows, part_a, m0,
+                               ilu->pos, dinv, last, ilu->r_perm, ilu->z_perm, st, status);
+            ilu_sweeps<2, T>(ilu, lv, uv, dinv, sh, st, q_s);
+        });
         spmv2_dots(sh, t, sv, 2, part_c, q_s);
-        hipLaunchKernelGGL(k_bicg_xr, dim3(nb2), dim3(BLOCK), 0, q_s, n, ph, sh, sv, t, r0, sc, x, r, part_d, nb2,
+        hipLaunchKernelGGL(k_bicg_xr, dim3(nb2), dim3(BLOCK), 0, q_s, n, ph, sh, sv, t, r0, sc, x, r, part_d, nb1,
                            part_b, nb_rows, part_c, st);
         hipLaunchKernelGGL(k_bicg_final_post, dim3(1), dim3(BLOCK), 0, q_s, nb2, part_d, sc, st, status);
     };
     hipGraphExec_t graph = nullptr;
     if (max_iter > 0) {
         KeyBuilder kb;
-        kb.add(n); kb.add(rp); kb.add(ci); kb.add(val); kb.add(use_f32); kb.add(TPR); kb.add(ilu->n_colours);
+        kb.add(n); kb.add(rp); kb.add(ci); kb.add(val); kb.add(use_f32); kb.add(ilu->n_colours);
         kb.add_bytes(ilu->colour_start, sizeof(int) * (size_t)(ilu->n_colours + 1));
         kb.add(ilu->pos); kb.add(ilu->r_perm); kb.add(ilu->z_perm);
         kb.add(ilu->rows); kb.add(ilu->lp); kb.add(ilu->up); kb.add(ilu->lc); kb.add(ilu->uc); kb.add(ilu->lv);

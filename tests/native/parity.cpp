@@ -5,7 +5,7 @@
 // block reductions or other summation orders must match to the stated relative tolerance.
 //
 //   parity <case> [level]    case: momentum pressure correction forces indicator mms oss ilu
-//                                  spmv amg sell coupled runs inverse pcg bicgstab jacobi mixed topology outlet nvb remap reproject
+//                                  spmv amg sell coupled runs inverse ilutail pcg bicgstab jacobi mixed topology outlet nvb remap reproject
 //                                  all
 //
 // Prints one line per compared quantity and exits 0 when every comparison passes.
@@ -836,6 +836,85 @@ void case_inverse() {
     }
 }
 
+// The ILU(0) sweeps where the trailing colours change path (one workgroup up to 1024 rows per colour, at
+// least two and at most 16 colours), against the colour-order sweeps on the host with the device's
+// factor: one row; two; cliques of 2, 15, 17 and 20 rows (as many colours); paths (two colours)
+// around 1024 rows per colour; a path with cliques hung on it, so that large colours precede small
+// ones. Diagonally dominant values: each row's result is a sum of at most 19 terms below 1, carried
+// through at most 20 colours: 20 x 20 eps relative to entries of order 1: 5e-14.
+void case_ilu_tail() {
+    std::printf("[ILU sweeps: trailing colours]\n");
+    std::mt19937_64 rng(5);
+    std::uniform_real_distribution<double> U(-1.0, 1.0);
+    struct Graph {
+        const char* name;
+        int path, cliques, size;
+    };
+    const Graph graphs[] = {{"one row", 1, 0, 0},          {"two rows", 2, 0, 0},         {"clique 15", 0, 1, 15},
+                            {"clique 17", 0, 1, 17},       {"clique 20", 0, 1, 20},       {"path 2047", 2047, 0, 0},
+                            {"path 2048", 2048, 0, 0},     {"path 2049", 2049, 0, 0},     {"path 2051", 2051, 0, 0},
+                            {"path 9000 + cliques of 5", 9000, 300, 5}, {"path 400 + cliques of 6", 400, 1025, 6}};
+    for (const Graph& gr : graphs) {
+        const int n = gr.path + gr.cliques * gr.size;
+        std::vector<std::vector<int>> nb(n);
+        auto edge = [&](int i, int j) { nb[i].push_back(j); nb[j].push_back(i); };
+        for (int i = 0; i + 1 < gr.path; ++i) edge(i, i + 1);
+        for (int k = 0; k < gr.cliques; ++k) {
+            const int c0 = gr.path + k * gr.size;
+            for (int i = 0; i < gr.size; ++i)
+                for (int j = 0; j < i; ++j) edge(c0 + i, c0 + j);
+            if (gr.path) edge(c0, (int)(rng() % gr.path));
+        }
+        std::vector<int> rp(1, 0), ci;
+        Vec val;
+        for (int i = 0; i < n; ++i) {
+            nb[i].push_back(i);
+            std::sort(nb[i].begin(), nb[i].end());
+            nb[i].erase(std::unique(nb[i].begin(), nb[i].end()), nb[i].end());
+            if (nb[i].size() > 32) nb[i].resize(32);   // the factor's row limit
+            for (int j : nb[i]) {
+                ci.push_back(j);
+                val.push_back(j == i ? 2.0 + (double)nb[i].size() : U(rng));
+            }
+            rp.push_back((int)ci.size());
+        }
+        DevArray<int> d_rp, d_ci;
+        DevArray<double> d_val, d_r, d_z;
+        d_rp.upload(rp);
+        d_ci.upload(ci);
+        d_val.upload(val);
+        MulticolourIlu0 ilu;
+        const MulticolourIlu0::Pattern P = MulticolourIlu0::build_pattern(n, rp, ci, 1 << 30);
+        ilu.set_pattern(P, d_rp, d_ci);
+        ilu.factor(d_val);
+        std::vector<double> lu(ci.size());
+        GPU_CHECK(cfa_memcpy(lu.data(), ilu.view()->lu, lu.size() * sizeof(double), 1, solver_stream()));
+        Vec r(2 * (size_t)n), ref(2 * (size_t)n);
+        for (double& v : r) v = U(rng);
+        d_r.upload(r);
+        d_z.reserve(2 * (size_t)n);
+        for (int c = 0; c < 2; ++c) {
+            Vec z(n);
+            for (int t = 0; t < n; ++t) {
+                double acc = r[(size_t)c * n + P.rows[t]];
+                for (int k = P.lp[t]; k < P.lp[t + 1]; ++k) acc -= lu[P.l_src[k]] * z[P.lc[k]];
+                z[t] = acc;
+            }
+            for (int t = n - 1; t >= 0; --t) {
+                double acc = z[t];
+                for (int k = P.up[t]; k < P.up[t + 1]; ++k) acc -= lu[P.u_src[k]] * z[P.uc[k]];
+                z[t] = acc / lu[P.d_src[t]];
+            }
+            for (int t = 0; t < n; ++t) ref[(size_t)c * n + P.rows[t]] = z[t];
+        }
+        std::printf("  %s: %d rows, %d colours\n", gr.name, n, P.n_colours);
+        ilu.apply(d_r, d_z, 2);
+        close_rel("  two components", down(d_z, 2 * (size_t)n), ref, 5e-14);
+        ilu.apply(d_r, d_z, 1);
+        close_rel("  one component", down(d_z, n), Vec(ref.begin(), ref.begin() + n), 5e-14);
+    }
+}
+
 // The scheme-consistent re-projection after a remesh with its two solves (u^{n-1} and u^n) side by
 // side on two streams against the same two solves one after the other, from the same state: the
 // velocities, the vorticity and the last increment bit for bit.
@@ -1627,6 +1706,7 @@ int main(int argc, char** argv) {
         if (all || what == "coupled") case_coupled(f);
         if (all || what == "runs") case_runs();
         if (all || what == "inverse") case_inverse();
+        if (all || what == "ilutail") case_ilu_tail();
         if (all || what == "pcg") case_pcg(f);
         if (all || what == "bicgstab") case_bicgstab(f);
         if (all || what == "jacobi") case_jacobi(f);
