@@ -3058,6 +3058,9 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
         kb.add(ilu->pos); kb.add(ilu->r_perm); kb.add(ilu->z_perm);
         kb.add(ilu->rows); kb.add(ilu->lp); kb.add(ilu->up); kb.add(ilu->lc); kb.add(ilu->uc); kb.add(ilu->lv);
         kb.add(ilu->uv); kb.add(ilu->dinv); kb.add(ilu->lv32); kb.add(ilu->uv32); kb.add(ilu->dinv32);
+        kb.add(ilu->s_lrow); kb.add(ilu->s_lsp); kb.add(ilu->s_lc); kb.add(ilu->s_lv); kb.add(ilu->s_lv32);
+        kb.add(ilu->s_urow); kb.add(ilu->s_usp); kb.add(ilu->s_uc); kb.add(ilu->s_uv); kb.add(ilu->s_uv32);
+        kb.add(ilu->s_llen); kb.add(ilu->s_ulen);
         for (int k = 0; k < 10; ++k) kb.add(ws->vec[k]);
         kb.add(ws->part); kb.add(sc); kb.add(status);
         graph = iteration_graph(ws, internal_of(ws)->bicg, kb.k, iteration);
