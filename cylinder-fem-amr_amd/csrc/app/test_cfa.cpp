@@ -13,8 +13,11 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <map>
+#include <mutex>
 #include <random>
 #include <string>
+#include <thread>
 
 #include "../host/device.hpp"
 
@@ -515,6 +518,98 @@ void ilu_sell_layout() {
     EXPECT(Q.s_pos0.empty(), "a layout below the default row threshold");
 }
 
+// Host check of the block pool (no device; blocks are counters' values): sizes, reuse within 1.5
+// times, a full synchronisation before a block freed since the last one is given out again and none
+// otherwise, the bound, trimming, the retry after a failed allocation, and no block held twice by four
+// threads that get and put at random.
+void block_pool() {
+    std::mutex m;
+    std::map<size_t, size_t> live;   // fake address -> size
+    size_t next = 1 << 20, limit = (size_t)-1;
+    int syncs = 0, frees = 0;
+    BlockPool pool;
+    pool.alloc = [&](void** p, size_t bytes) {
+        std::lock_guard<std::mutex> lock(m);
+        size_t total = bytes;
+        for (const auto& b : live) total += b.second;
+        if (total > limit) return 1;
+        *p = reinterpret_cast<void*>(next);
+        live[next] = bytes;
+        next += bytes + 4096;
+        return 0;
+    };
+    pool.free = [&](void* p) {
+        std::lock_guard<std::mutex> lock(m);
+        frees += (int)live.erase(reinterpret_cast<size_t>(p));
+        return 0;
+    };
+    pool.sync = [&] { ++syncs; return 0; };
+    for (size_t b : {(size_t)1, (size_t)511, (size_t)512, (size_t)8192, (size_t)8193, (size_t)1 << 20, ((size_t)1 << 30) + 1}) {
+        const size_t c = BlockPool::class_of(b);
+        EXPECT(c >= b && (b < 8192 ? c - b < 512 : c - b <= b / 8), "size class of %zu: %zu", b, c);
+    }
+    void *a = nullptr, *b = nullptr, *c = nullptr;
+    EXPECT(pool.get(&a, 100000) == 0 && pool.get(&b, 100000) == 0 && a != b, "two blocks");
+    pool.put(a);
+    EXPECT(pool.get(&c, 70000) == 0 && c == a && syncs == 1, "reuse after one synchronisation");
+    pool.put(c);
+    pool.put(b);
+    EXPECT(pool.get(&c, 60000) == 0 && c != a && c != b && syncs == 1, "not within 1.5 times: a new block");
+    EXPECT(pool.get(&a, 100000) == 0 && syncs == 2, "freed since: synchronised");
+    EXPECT(pool.get(&b, 100000) == 0 && syncs == 2, "freed before the last one: not again");
+    pool.bound = 150000;
+    pool.put(a);
+    pool.put(b);
+    EXPECT(frees == 1 && pool.kept_bytes() <= pool.bound, "beyond the bound a block is freed");
+    limit = 200000;
+    EXPECT(pool.get(&a, 120000) == 0 && pool.kept_bytes() == 0 && frees == 2, "a failed allocation gives the blocks back");
+    EXPECT(pool.get(&b, 1 << 20) != 0, "failure is reported");
+    pool.put(a);
+    pool.put(c);
+    pool.trim();
+    EXPECT(live.empty() && pool.kept_bytes() == 0, "trimmed");
+    limit = (size_t)-1;
+    pool.bound = 1 << 20;
+    std::mutex hm;
+    std::map<void*, int> held;
+    int twice = 0;
+    std::vector<std::thread> threads;
+    for (int t = 0; t < 4; ++t)
+        threads.emplace_back([&, t] {
+            std::mt19937 rng(t);
+            std::vector<void*> mine;
+            for (int k = 0; k < 4000; ++k) {
+                if (mine.size() < 20 && rng() % 2) {
+                    void* p = nullptr;
+                    if (pool.get(&p, 256 << rng() % 9)) continue;
+                    std::lock_guard<std::mutex> lock(hm);
+                    twice += held[p]++ != 0;
+                    mine.push_back(p);
+                } else if (!mine.empty()) {
+                    std::swap(mine[rng() % mine.size()], mine.back());
+                    {
+                        std::lock_guard<std::mutex> lock(hm);
+                        --held[mine.back()];
+                    }
+                    pool.put(mine.back());
+                    mine.pop_back();
+                }
+            }
+            for (void* p : mine) {
+                {
+                    std::lock_guard<std::mutex> lock(hm);
+                    --held[p];
+                }
+                pool.put(p);
+            }
+        });
+    for (auto& t : threads) t.join();
+    EXPECT(twice == 0 && pool.kept_bytes() <= pool.bound, "threads: %d blocks held twice", twice);
+    pool.trim();
+    EXPECT(live.empty(), "every block given back");
+    std::printf("  block pool: %d synchronisations, %d frees\n", syncs, frees);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -524,7 +619,10 @@ int main(int argc, char** argv) {
         return 2;
     }
     std::printf("cylinder_fem_amr unit tests (%s)\n", what.c_str());
-    if (what != "gpu") ilu_sell_layout();
+    if (what != "gpu") {
+        ilu_sell_layout();
+        block_pool();
+    }
     if (what != "host") {
         GPU_CHECK(cfa_init(0));
         random_adaptation();

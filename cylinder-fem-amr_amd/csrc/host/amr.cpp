@@ -23,16 +23,16 @@ struct Buf {
     Buf() = default;
     Buf(const Buf&) = delete;
     Buf& operator=(const Buf&) = delete;
-    ~Buf() { if (ptr) cfa_free(ptr); }
+    ~Buf() { if (ptr) device_pool().put(ptr); }
     void ensure(size_t need, size_t used, cfa_stream_t s) {
         if (need <= cap && ptr) return;
         const size_t c = need + need / 2 + 256;
         void* p = nullptr;
-        GPU_CHECK(cfa_malloc(&p, c * sizeof(T)));
+        GPU_CHECK(device_pool().get(&p, c * sizeof(T)));
         if (ptr && used) GPU_CHECK(cfa_memcpy(p, ptr, std::min(used, cap) * sizeof(T), 2, s));
         if (ptr) {
             GPU_CHECK(cfa_stream_sync(s));
-            cfa_free(ptr);
+            device_pool().put(ptr);
         }
         ptr = static_cast<T*>(p);
         cap = c;
@@ -274,7 +274,7 @@ AdaptiveMesh::~AdaptiveMesh() {
     if (d_ && d_->s) {
         cfa_stream_sync(d_->s);
         cfa_stream_t s = d_->s;
-        d_.reset();   // frees the arrays (cfa_free synchronises the device)
+        d_.reset();   // frees the arrays
         cfa_stream_destroy(s);
     }
 }

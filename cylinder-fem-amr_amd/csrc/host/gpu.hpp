@@ -10,6 +10,7 @@
 
 #include "../../../include/cfa_hip.h"
 #include "cfa_common.hpp"
+#include "pool.hpp"
 
 namespace cfa {
 
@@ -28,7 +29,8 @@ inline cfa_stream_t& solver_stream() {
     return s;
 }
 
-// Device array with capacity growth; memory is kept when a smaller size is requested.
+// Device array with capacity growth; memory is kept when a smaller size is requested. A new block holds
+// whatever its last user left.
 template <typename T>
 struct DevArray {
     T* ptr = nullptr;
@@ -43,7 +45,7 @@ struct DevArray {
     }
     ~DevArray() { release(); }
     void release() {
-        if (ptr) cfa_free(ptr);
+        if (ptr) device_pool().put(ptr);
         ptr = nullptr;
         cap = 0;
     }
@@ -53,7 +55,7 @@ struct DevArray {
         release();
         const size_t c = n + n / 2 + pad;
         void* p = nullptr;
-        GPU_CHECK(cfa_malloc(&p, c * sizeof(T)));
+        GPU_CHECK(device_pool().get(&p, c * sizeof(T)));
         ptr = static_cast<T*>(p);
         cap = c;
     }

@@ -124,6 +124,12 @@ int cfa_dumped_pressure_solve(const char* path, double tol, int max_iter, int pr
 int cfa_force_statistics(int n, const double* t, const double* cd, const double* cl, const double* dp,
                          double window, double* out);
 
+/* The host layer's device arrays are taken from freed blocks where one fits (no counterpart in the
+ * reference, which calls cudaMalloc and cudaFree each time). cfa_pool_trim gives all of them back to
+ * the device; cfa_pool_bytes is how much is kept (at most 2 GiB). */
+void cfa_pool_trim(void);
+long long cfa_pool_bytes(void);
+
 /* Host SA-AMG set-up (src/cfa/linalg.cuh:995-1060, 1276-1431) of a host CSR matrix: per level
  * rows, (nnz A, nnz P), Jacobi weight, the coarse size and the level-0 aggregates [n].
  * Returns the number of smoothed levels (<= 16 reported). Needs a GPU (the hierarchy is
