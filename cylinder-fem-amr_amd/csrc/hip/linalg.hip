@@ -252,19 +252,46 @@ k_spmv_multi(int n, const int* __restrict__ rp, const int* __restrict__ ci, cons
 enum { S_BNORM = 0, S_RZ_OLD, S_PQ, S_ALPHA, S_RNORM, S_REL, S_BETA, S_TOL };
 // ints: [0] state, [1] final iteration count, [2] current iteration
 
-// ||b||; x = 0 and stop when ||b|| < 1e-14 (linalg.cuh:205-209)
-__global__ void k_pcg_init_bnorm(int nb, const double* __restrict__ part, double* __restrict__ sc,
-                                 int* __restrict__ st, int* __restrict__ status) {
-    __shared__ double lds[BLOCK / WAVE];
-    const double bb = sum_partials(part, nb, 1, lds);
+// Start of a solve from the b.b and r.r partials: ||b||, x = 0 and stop when ||b|| < 1e-14
+// (linalg.cuh:205-209, the caller's k_zero_if_trivial), converged with 0 iterations when ||r|| < tol ||b||
+// (linalg.cuh:217-218); the tolerance and the "not computed" relative residual -1
+__global__ void k_pcg_init(int nb, const double* __restrict__ part_b, const double* __restrict__ part_r, double tol,
+                           double* __restrict__ sc, int* __restrict__ st, int* __restrict__ status) {
+    __shared__ double lds[2 * BLOCK / WAVE];
+    double s[2];
+    sum_partials_k<2>({part_b, part_r}, {nb, nb}, 1, s, lds);
     if (threadIdx.x != 0) return;
-    const double b_norm = sqrt(bb);
+    const double b_norm = sqrt(s[0]);
     sc[S_BNORM] = b_norm;
+    sc[S_TOL] = tol;
+    sc[S_REL] = -1.0;
     st[1] = 0;
     st[2] = 0;
-    st[0] = b_norm < 1.0e-14 ? ST_TRIVIAL : ST_RUNNING;
-    publish(status, 0, st[0]);
+    const int state = b_norm < 1.0e-14 ? ST_TRIVIAL : sqrt(s[1]) < tol * b_norm ? ST_CONVERGED : ST_RUNNING;
+    st[0] = state;
+    publish(status, 0, state);
 }
+
+// The solve's outcome in the pinned status words [2..7]: state, iterations, relative residual(s) (as
+// two words each), read by the host after it has waited for the stream
+__device__ __forceinline__ void publish_double(int* status, double v) {
+    const unsigned long long b = __double_as_longlong(v);
+    __hip_atomic_store(&status[0], (int)(unsigned)b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&status[1], (int)(unsigned)(b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+double published_double(const volatile int* status) {
+    const unsigned long long b = (unsigned)status[0] | ((unsigned long long)(unsigned)status[1] << 32);
+    double v;
+    std::memcpy(&v, &b, sizeof(v));
+    return v;
+}
+__global__ void k_pcg_outcome(const double* __restrict__ sc, const int* __restrict__ st, int* __restrict__ status) {
+    __hip_atomic_store(&status[2], st[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&status[3], st[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    publish_double(status + 4, sc[S_REL]);
+}
+
+__global__ void k_pcg_start(int* __restrict__ st) { st[0] = ST_RUNNING; }
 
 __global__ void k_zero_if_trivial(int n, double* __restrict__ x, const int* __restrict__ st) {
     if (st[0] != ST_TRIVIAL) return;
@@ -272,34 +299,22 @@ __global__ void k_zero_if_trivial(int n, double* __restrict__ x, const int* __re
     if (i < n) x[i] = 0.0;
 }
 
-// r = b - q; partial r.r
+// r = b - q; partials b.b and r.r
 __global__ void __launch_bounds__(BLOCK)
 k_pcg_residual(int n, const double* __restrict__ b, const double* __restrict__ q, double* __restrict__ r,
-               double* __restrict__ part, const int* __restrict__ st) {
-    __shared__ double lds[BLOCK / WAVE];
-    if (halted(st)) return;
-    double acc = 0.0;
+               double* __restrict__ part_b, double* __restrict__ part_r) {
+    __shared__ double lds[2 * BLOCK / WAVE];
+    double acc[2] = {0.0, 0.0};
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double ri = b[i] + (-1.0) * q[i];
+        const double bi = b[i], ri = bi + (-1.0) * q[i];
         r[i] = ri;
-        acc += ri * ri;
+        acc[0] += bi * bi;
+        acc[1] += ri * ri;
     }
-    acc = block_sum(acc, lds);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc;
-}
-
-// initial residual test (linalg.cuh:217-218): converged with 0 iterations
-__global__ void k_pcg_init_rnorm(int nb, const double* __restrict__ part, double* __restrict__ sc,
-                                 int* __restrict__ st, int* __restrict__ status) {
-    __shared__ double lds[BLOCK / WAVE];
-    if (st[0] != ST_RUNNING) return;
-    const double rr = sum_partials(part, nb, 1, lds);
-    if (threadIdx.x != 0) return;
-    const double r_norm = sqrt(rr);
-    if (r_norm < sc[S_TOL] * sc[S_BNORM]) {
-        st[0] = ST_CONVERGED;
-        st[1] = 0;
-        publish(status, 0, ST_CONVERGED);
+    block_sum_k<2>(acc, lds);
+    if (threadIdx.x == 0) {
+        part_b[blockIdx.x] = acc[0];
+        part_r[blockIdx.x] = acc[1];
     }
 }
 
@@ -423,12 +438,12 @@ __device__ __forceinline__ bool run_part_has(int m) { return m % (BLOCK / RB) ==
 // Fused operator, stage 1: q = Kp p (CSR) and g = M^-1 B p, all on the same row pattern
 template <int RB>
 __global__ void __launch_bounds__(BLOCK)
-k_apply_K_B(int n, int nnz, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ val,
+k_apply_K_B(int n, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ val,
             const double* __restrict__ oss, const double* __restrict__ inv_m, const double* __restrict__ in,
             double* __restrict__ q, double* __restrict__ gx, double* __restrict__ gy, const int* __restrict__ st) {
     __shared__ double prod[3 * RUN_TILE(RB)];
     if (halted(st)) return;
-    const RowValues<3, double> kb{{val, oss, oss + (size_t)nnz}};
+    const RowValues<3, double> kb{{val, oss, oss + (size_t)rp[n]}};
     for (int r0 = blockIdx.x * RB; r0 < n; r0 += gridDim.x * RB) {
         const int row = r0 + (int)threadIdx.x % RB, e0 = rp[r0], e1 = rp[min(r0 + RB, n)];
         const int k0 = row < n ? rp[row] : e1, k1 = row < n ? rp[row + 1] : e1;
@@ -457,14 +472,15 @@ k_apply_K_B(int n, int nnz, const int* __restrict__ rp, const int* __restrict__ 
 // capped (grid-stride over row runs) so that the consumers' re-summation stays short.
 template <int RB>
 __global__ void __launch_bounds__(BLOCK)
-k_apply_BT_dot(int n, int nnz, const int* __restrict__ rp, const int* __restrict__ ci,
+k_apply_BT_dot(int n, const int* __restrict__ rp, const int* __restrict__ ci,
                const double* __restrict__ oss, const int* __restrict__ tag, OutletMode om,
                const double* __restrict__ gx, const double* __restrict__ gy, const double* __restrict__ p,
                double* __restrict__ q, double* __restrict__ part, const int* __restrict__ st) {
     __shared__ double prod[RUN_TILE(RB)];
     __shared__ double lds[BLOCK / WAVE];
     if (halted(st)) return;
-    const RowValues<2, double> bt{{oss + 2 * (size_t)nnz, oss + 3 * (size_t)nnz}};
+    const size_t nnz = (size_t)rp[n];
+    const RowValues<2, double> bt{{oss + 2 * nnz, oss + 3 * nnz}};
     double contrib = 0.0;
     for (int r0 = blockIdx.x * RB; r0 < n; r0 += gridDim.x * RB) {
         const int row = r0 + (int)threadIdx.x, e0 = rp[r0], e1 = rp[min(r0 + RB, n)];
@@ -511,7 +527,7 @@ k_apply_BT_dot(int n, int nnz, const int* __restrict__ rp, const int* __restrict
 enum { ST_CAPPED = 4 };
 
 struct PcgArgs {
-    int n, nnz, max_iter;
+    int n, max_iter;
     const int* rp; const int* ci; const double* val;
     const double* oss; const double* inv_m; const int* tag; double* gx; double* gy;
     OutletMode om;
@@ -542,7 +558,7 @@ k_fp_operator(PcgArgs a, int h) {
     kb.p[0] = a.val;
     if constexpr (OSS) {
         kb.p[1] = a.oss;
-        kb.p[2] = a.oss + (size_t)a.nnz;
+        kb.p[2] = a.oss + (size_t)a.rp[a.n];
     }
     RunTile<RB, NV> tile;
     double zj[U], pj[U], zi = 0.0, pi = 0.0;
@@ -1501,8 +1517,8 @@ __device__ __forceinline__ void write_partials2(double* part, double (&acc)[NQ][
 // and component (part 0 and 1 of the workgroup) and its sum; prod: 2 RUN_TILE(RB) doubles
 template <int RB>
 __device__ __forceinline__ double run_product2(int n, const int* __restrict__ rp, const int* __restrict__ ci,
-                                               const double* __restrict__ val, const double* __restrict__ x, int r0,
-                                               double* prod) {
+                                               const double* __restrict__ val, const double* __restrict__ x_u,
+                                               const double* __restrict__ x_v, int r0, double* prod) {
     const RowValues<1, double> av{{val}};
     const int row = r0 + (int)threadIdx.x % RB, e0 = rp[r0], e1 = rp[min(r0 + RB, n)];
     const int k0 = row < n ? rp[row] : e1, k1 = row < n ? rp[row + 1] : e1;
@@ -1513,8 +1529,8 @@ __device__ __forceinline__ double run_product2(int n, const int* __restrict__ rp
 #pragma unroll
         for (int u = 0; u < RUN_SLOTS(RB); ++u) {
             const int at = u * BLOCK + threadIdx.x, j = tile.c[u];
-            prod[at] = tile.v[u][0] * x[j];
-            prod[RUN_TILE(RB) + at] = tile.v[u][0] * x[n + j];
+            prod[at] = tile.v[u][0] * x_u[j];
+            prod[RUN_TILE(RB) + at] = tile.v[u][0] * x_v[j];
         }
         __syncthreads();
         run_row_sums<RB, 2>(prod, t, k0, k1, s);
@@ -1523,22 +1539,24 @@ __device__ __forceinline__ double run_product2(int n, const int* __restrict__ rp
     return run_part_has<RB>(0) ? s[0] : s[1];
 }
 
-// r = b - A x (both components), r0 = p = r, v = 0; partial r.r
+// The iterate from the caller's guesses, r = b - A x (both components), r0 = p = r, v = 0; partial r.r
 template <int RB>
 __global__ void __launch_bounds__(BLOCK)
 k_bicg_init(int n, const int* __restrict__ rp, const int* __restrict__ ci, const double* __restrict__ val,
-            const double* __restrict__ b, const double* __restrict__ x, double* __restrict__ r,
-            double* __restrict__ r0v, double* __restrict__ p, double* __restrict__ v, double* __restrict__ part) {
+            const double* __restrict__ b_u, const double* __restrict__ b_v, const double* __restrict__ x_u,
+            const double* __restrict__ x_v, double* __restrict__ x, double* __restrict__ r, double* __restrict__ r0v,
+            double* __restrict__ p, double* __restrict__ v, double* __restrict__ part) {
     __shared__ double prod[2 * RUN_TILE(RB)];
     __shared__ double lds[2 * BLOCK / WAVE];
     const int c = threadIdx.x / RB;
     double acc[1][2] = {{0.0, 0.0}};
     for (int r0 = blockIdx.x * RB; r0 < n; r0 += gridDim.x * RB) {
-        const double s = run_product2<RB>(n, rp, ci, val, x, r0, prod);
+        const double s = run_product2<RB>(n, rp, ci, val, x_u, x_v, r0, prod);
         const int row = r0 + (int)threadIdx.x % RB;
         if (c > 1 || row >= n) continue;
         const int i = c * n + row;
-        const double q = b[i] - s;
+        const double q = (c ? b_v : b_u)[row] - s;
+        x[i] = (c ? x_v : x_u)[row];
         r[i] = q;
         r0v[i] = q;
         p[i] = q;
@@ -1555,49 +1573,59 @@ __device__ __forceinline__ void bicg_stop(int* st, int c, int it, int ok) {
     st[6 + c] = ok;
 }
 
-__global__ void k_bicg_final_init(int nb, const double* __restrict__ part, double* __restrict__ sc,
+// Scalars and state of a solve from the r.r partials; the first iteration's p update takes no
+// coefficients (p = r), and a component whose rho breaks down at once stops with 0 iterations
+__global__ void k_bicg_final_init(int nb, const double* __restrict__ part, double tol, double* __restrict__ sc,
                                   int* __restrict__ st, int* __restrict__ status, int max_iter) {
     __shared__ double lds[2 * BLOCK / WAVE];
     double rr[2];
     sum_partials_k<2>({part, part + 1}, {nb, nb}, 6, rr, lds);
     if (threadIdx.x != 0) return;
+    int act[2];
+    sc[B_TOL] = tol;
     for (int c = 0; c < 2; ++c) {
-        sc[B_RN0 + c] = sqrt(rr[c]);
+        const double rn0 = sqrt(rr[c]), bd = 1.0e-30 * rn0 * rn0 + 1.0e-300;
+        sc[B_RN0 + c] = rn0;
         sc[B_RHO + c] = rr[c];
-        sc[B_BD + c] = 1.0e-30 * sc[B_RN0 + c] * sc[B_RN0 + c] + 1.0e-300;
+        sc[B_BD + c] = bd;
         sc[B_RHO_OLD + c] = 1.0;
         sc[B_ALPHA + c] = 1.0;
         sc[B_OMEGA + c] = 1.0;
         sc[B_REL + c] = 0.0;
-        st[2 + c] = sc[B_RN0 + c] >= 1.0e-13 ? 1 : 0;
+        sc[B_CB + c] = 0.0;
+        sc[B_CO + c] = 0.0;
+        act[c] = rn0 >= 1.0e-13 ? 1 : 0;
+        st[2 + c] = act[c];
         st[4 + c] = 0;
         st[6 + c] = 1;
         st[8 + c] = 0;
     }
     st[10] = 0;
     st[11] = max_iter;
-    st[0] = (st[2] || st[3]) && max_iter > 0 ? ST_RUNNING : ST_STOPPED;
-    publish(status, 0, st[0]);
-}
-
-// Start of an iteration: breakdown check on rho, coefficients of the p update
-__device__ void bicg_pre_logic(double* __restrict__ sc, int* __restrict__ st, int* __restrict__ status) {
-    if (st[0] != ST_RUNNING) return;
-    const int it = st[10];
-    for (int c = 0; c < 2; ++c) {
-        sc[B_CB + c] = 0.0;
-        sc[B_CO + c] = 0.0;
-        if (st[2 + c] && fabs(sc[B_RHO + c]) < sc[B_BD + c]) bicg_stop(st, c, it, 0);
-        if (st[2 + c] && it > 0) {
-            sc[B_CB + c] = (sc[B_RHO + c] / sc[B_RHO_OLD + c]) * (sc[B_ALPHA + c] / (sc[B_OMEGA + c] + 1.0e-30));
-            sc[B_CO + c] = sc[B_OMEGA + c];
-        }
+    int state = (act[0] || act[1]) && max_iter > 0 ? ST_RUNNING : ST_STOPPED;
+    if (state == ST_RUNNING) {
+        for (int c = 0; c < 2; ++c)
+            if (act[c] && fabs(rr[c]) < sc[B_BD + c]) {
+                bicg_stop(st, c, 0, 0);
+                act[c] = 0;
+            }
+        if (!(act[0] || act[1])) state = ST_STOPPED;
     }
-    if (!(st[2] || st[3])) { st[0] = ST_STOPPED; publish(status, it, ST_STOPPED); }
+    st[0] = state;
+    publish(status, 0, state);
 }
 
-__global__ void k_bicg_pre(double* __restrict__ sc, int* __restrict__ st, int* __restrict__ status) {
-    bicg_pre_logic(sc, st, status);
+// The solutions to the caller's vectors and the outcome (status [2..13]: active, iterations, converged
+// and relative residual of both components)
+__global__ void k_bicg_outcome(int n, const double* __restrict__ x, double* __restrict__ x_u, double* __restrict__ x_v,
+                               const double* __restrict__ sc, const int* __restrict__ st, int* __restrict__ status) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) {
+        x_u[i] = x[i];
+        x_v[i] = x[n + i];
+    }
+    if (i < 6) __hip_atomic_store(&status[2 + i], st[2 + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (blockIdx.x == 0 && threadIdx.x < 2) publish_double(status + 8 + 2 * threadIdx.x, sc[B_REL + threadIdx.x]);
 }
 
 // p = r + cb (p - co v), from the second iteration on, and the permutation of p into colour order with
@@ -1640,7 +1668,7 @@ k_spmv2_dots(int n, const int* __restrict__ rp, const int* __restrict__ ci, cons
         const int row = r0 + (int)threadIdx.x % RB, i = c * n + row;
         const bool own = c < 2 && row < n;
         const double wi = own ? w0[i] : 0.0;
-        const double s = run_product2<RB>(n, rp, ci, val, x, r0, prod);
+        const double s = run_product2<RB>(n, rp, ci, val, x, x + n, r0, prod);
         if (!own) continue;
         y[i] = s;
         if (mode == 1) {   // r0 . v
@@ -2577,9 +2605,6 @@ namespace {
 // PCG with the reductions folded into the consuming kernels (k_fp_*), two iterations per
 // captured graph (the search direction and the r.z partials alternate between two buffers).
 // Same algorithm, guards and stopping rules as the reference (src/cfa/linalg.cuh:183-256).
-// BiCGSTAB2's product runs with 2 or 4 lanes per row (about four entries per lane).
-int operator_lanes(int n, long long nnz) { return nnz <= 12LL * n ? 2 : 4; }
-
 // Rows per workgroup of the operator kernels and their workgroups (at most RED_BLOCKS, so that the
 // consumers re-sum at most that many partials; 1536 and 2048 ran the same). 64 rows split a small mesh
 // over the CUs; 128 leave room for six workgroups' LDS on a CU. Stage 1 with 64 / 128 / 256 rows:
@@ -2601,22 +2626,22 @@ void launch_fp_operator(bool oss, hipStream_t s, const PcgArgs& a, int h) {
         else hipLaunchKernelGGL((k_fp_operator<RB, false>), dim3(run_blocks(a.n)), dim3(BLOCK), 0, s, a, h);
     });
 }
-void launch_apply_K_B(hipStream_t s, int n, int nnz, const int* rp, const int* ci, const double* val,
+void launch_apply_K_B(hipStream_t s, int n, const int* rp, const int* ci, const double* val,
                       const double* oss, const double* inv_m, const double* in, double* q, double* gx, double* gy,
                       const int* st) {
     run_dispatch(n, [&](auto rb) {
         constexpr int RB = decltype(rb)::value;
-        hipLaunchKernelGGL(k_apply_K_B<RB>, dim3(run_blocks(n)), dim3(BLOCK), 0, s, n, nnz, rp, ci, val, oss, inv_m, in,
+        hipLaunchKernelGGL(k_apply_K_B<RB>, dim3(run_blocks(n)), dim3(BLOCK), 0, s, n, rp, ci, val, oss, inv_m, in,
                            q, gx, gy, st);
     });
 }
 // returns the number of partials
-int launch_apply_BT_dot(hipStream_t s, int n, int nnz, const int* rp, const int* ci, const double* oss,
+int launch_apply_BT_dot(hipStream_t s, int n, const int* rp, const int* ci, const double* oss,
                         const int* tag, OutletMode om, const double* gx, const double* gy, const double* p, double* q,
                         double* part, const int* st) {
     run_dispatch(n, [&](auto rb) {
         constexpr int RB = decltype(rb)::value;
-        hipLaunchKernelGGL(k_apply_BT_dot<RB>, dim3(run_blocks(n)), dim3(BLOCK), 0, s, n, nnz, rp, ci, oss, tag, om, gx,
+        hipLaunchKernelGGL(k_apply_BT_dot<RB>, dim3(run_blocks(n)), dim3(BLOCK), 0, s, n, rp, ci, oss, tag, om, gx,
                            gy, p, q, part, st);
     });
     return run_blocks(n);
@@ -2625,6 +2650,16 @@ int launch_apply_BT_dot(hipStream_t s, int n, int nnz, const int* rp, const int*
 // pressure-Dirichlet rows of the operator: node p_pin with the outlet Dirichlet condition, else outlet nodes
 OutletMode outlet_of(const cfa_oss_op_t* oss) {
     return OutletMode{oss->outlet_dirichlet, oss->p_pin, 0.0};
+}
+
+// k_pcg_outcome's words as the solve's result
+void pcg_outcome(const cfa_krylov_ws_t* ws, int max_iter, cfa_solve_result_t* result) {
+    const volatile int* w = ws->status_host;
+    const int state = w[2];
+    const bool capped = state == ST_RUNNING || state == ST_CAPPED;   // iteration cap
+    result->iters[0] = capped ? max_iter : w[3];
+    result->converged[0] = !capped && state != ST_STOPPED;
+    result->rel_residual[0] = published_double(w + 4);
 }
 
 int pcg_fused(int n, const int* rp, const int* ci, const double* val, const double* b, double* x, int max_iter,
@@ -2645,16 +2680,10 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
     a.prr = ws->part + 3 * OP_BLOCKS;
     double* scratch = ws->part + 4 * OP_BLOCKS;
     a.sc = ws->scal; a.st = state_words(ws); a.status = ws->status_dev;
-    CFA_TRY(hipMemcpyAsync(&a.nnz, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
-    CFA_TRY(hipStreamSynchronize(s));
     if (oss) {
         a.oss = oss->oss_val; a.inv_m = oss->inv_m; a.tag = oss->bc_tag; a.gx = oss->gx; a.gy = oss->gy;
         a.om = outlet_of(oss);
     }
-    const int TPR = operator_lanes(n, a.nnz);
-    const double init_sc[2] = {tol, -1.0};   // S_TOL, and S_REL "not computed"
-    CFA_TRY(hipMemcpyAsync(a.sc + S_TOL, &init_sc[0], sizeof(double), hipMemcpyHostToDevice, s));
-    CFA_TRY(hipMemcpyAsync(a.sc + S_REL, &init_sc[1], sizeof(double), hipMemcpyHostToDevice, s));
     ws->status_host[0] = 0;
     ws->status_host[1] = ST_RUNNING;
     const int nb = red_blocks(n);
@@ -2662,19 +2691,17 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
     const int nb_op = run_blocks(n);
     const int* st_r = a.st;
 
-    // prologue (linalg.cuh:205-227): ||b||, x = 0 when trivial, r = b - A x, initial test, z = M^-1 r
-    hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(BLOCK), 0, s, n, b, b, scratch, nullptr);
-    hipLaunchKernelGGL(k_pcg_init_bnorm, dim3(1), dim3(BLOCK), 0, s, nb, scratch, a.sc, a.st, a.status);
-    hipLaunchKernelGGL(k_zero_if_trivial, dim3(blocks), dim3(BLOCK), 0, s, n, x, st_r);
+    // prologue (linalg.cuh:205-227): r = b - A x, ||b||, x = 0 when trivial, initial test, z = M^-1 r
     if (!amg) hipLaunchKernelGGL(k_inv_diag, dim3(blocks), dim3(BLOCK), 0, s, n, rp, ci, val, 1.0e-14, inv_diag);
     if (oss) {
-        launch_apply_K_B(s, n, a.nnz, rp, ci, val, a.oss, a.inv_m, x, a.q, a.gx, a.gy, st_r);
-        (void)launch_apply_BT_dot(s, n, a.nnz, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.q, a.q, scratch, st_r);
+        launch_apply_K_B(s, n, rp, ci, val, a.oss, a.inv_m, x, a.q, a.gx, a.gy, nullptr);
+        (void)launch_apply_BT_dot(s, n, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.q, a.q, scratch, nullptr);
     } else {
-        csr_op_launch<OP_SPMV, double>(TPR, n, rp, ci, val, x, nullptr, nullptr, 0.0, a.q, st_r, s);
+        csr_op_launch<OP_SPMV, double>(2, n, rp, ci, val, x, nullptr, nullptr, 0.0, a.q, nullptr, s);
     }
-    hipLaunchKernelGGL(k_pcg_residual, dim3(nb), dim3(BLOCK), 0, s, n, b, a.q, a.r, scratch, st_r);
-    hipLaunchKernelGGL(k_pcg_init_rnorm, dim3(1), dim3(BLOCK), 0, s, nb, scratch, a.sc, a.st, a.status);
+    hipLaunchKernelGGL(k_pcg_residual, dim3(nb), dim3(BLOCK), 0, s, n, b, a.q, a.r, scratch, a.prr);
+    hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(BLOCK), 0, s, nb, scratch, a.prr, tol, a.sc, a.st, a.status);
+    hipLaunchKernelGGL(k_zero_if_trivial, dim3(blocks), dim3(BLOCK), 0, s, n, x, st_r);
     auto apply_prec = [&](int h_next, bool check, hipStream_t q_s) {
         if (amg) {
             PrecHooks hk;
@@ -2697,7 +2724,7 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
     auto iteration = [&](int h, hipStream_t q_s) {
         launch_fp_operator(oss != nullptr, q_s, a, h);
         if (oss)
-            (void)launch_apply_BT_dot(q_s, n, a.nnz, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.p[h], a.q, a.ppq, st_r);
+            (void)launch_apply_BT_dot(q_s, n, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.p[h], a.q, a.ppq, st_r);
         hipLaunchKernelGGL(k_fp_update, dim3(nb), dim3(BLOCK), 0, q_s, a, h, nb_op);
         (void)apply_prec(1 - h, true, q_s);
     };
@@ -2728,21 +2755,11 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
         if (graph) CFA_TRY(hipGraphLaunch(graph, s));
         else two_iterations(s);
     }
+    hipLaunchKernelGGL(k_pcg_outcome, dim3(1), dim3(1), 0, s, a.sc, a.st, a.status);
     rc = launch_status();
     if (rc) return rc;
-    int fin[3];
-    double rel;
-    CFA_TRY(hipMemcpyAsync(fin, a.st, sizeof(fin), hipMemcpyDeviceToHost, s));
-    CFA_TRY(hipMemcpyAsync(&rel, a.sc + S_REL, sizeof(double), hipMemcpyDeviceToHost, s));
     CFA_TRY(hipStreamSynchronize(s));
-    if (fin[0] == ST_RUNNING || fin[0] == ST_CAPPED) {   // iteration cap
-        result->iters[0] = max_iter;
-        result->converged[0] = 0;
-    } else {
-        result->iters[0] = fin[1];
-        result->converged[0] = fin[0] != ST_STOPPED;
-    }
-    result->rel_residual[0] = rel;
+    pcg_outcome(ws, max_iter, result);
     return launch_status();
 }
 
@@ -2822,13 +2839,10 @@ int cfa_pcg_operator(int n, const int* rp, const int* ci, const double* val, con
     if (oss->outlet_dirichlet && n > 0 && (oss->p_pin < 0 || oss->p_pin >= n)) return CFA_E_ARG;
     if (n == 0) return CFA_OK;
     hipStream_t s = S(stream);
-    int nnz = 0;
-    CFA_TRY(hipMemcpyAsync(&nnz, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
-    CFA_TRY(hipStreamSynchronize(s));
     if (stage != 2)
-        launch_apply_K_B(s, n, nnz, rp, ci, val, oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy, nullptr);
+        launch_apply_K_B(s, n, rp, ci, val, oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy, nullptr);
     if (stage != 1)
-        (void)launch_apply_BT_dot(s, n, nnz, rp, ci, oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx, oss->gy, in,
+        (void)launch_apply_BT_dot(s, n, rp, ci, oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx, oss->gy, in,
                                   out, part, nullptr);
     return launch_status();
 }
@@ -2861,20 +2875,12 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
     const int nb = red_blocks(n);
     const int blocks = blocks_for(n);
     constexpr int TPR = 4;
-    int nnz = 0;
-    if (oss) {
-        CFA_TRY(hipMemcpyAsync(&nnz, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
-        CFA_TRY(hipStreamSynchronize(s));
-    }
-    const double init_sc[2] = {tol, -1.0};   // S_TOL, and S_REL "not computed"
-    CFA_TRY(hipMemcpyAsync(sc + S_TOL, &init_sc[0], sizeof(double), hipMemcpyHostToDevice, s));
-    CFA_TRY(hipMemcpyAsync(sc + S_REL, &init_sc[1], sizeof(double), hipMemcpyHostToDevice, s));
     ws->status_host[0] = 0;
     ws->status_host[1] = ST_RUNNING;
 
     auto apply_op = [&](const double* in, double* out, hipStream_t q_s) {
         if (oss) {
-            launch_apply_K_B(q_s, n, nnz, rp, ci, val, oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy, st);
+            launch_apply_K_B(q_s, n, rp, ci, val, oss->oss_val, oss->inv_m, in, out, oss->gx, oss->gy, st);
         } else {
             csr_op_launch<OP_SPMV, double>(TPR, n, rp, ci, val, in, nullptr, nullptr, 0.0, out, st, q_s);
             if (extra_cb) extra_cb(in, out, extra_ctx);
@@ -2883,7 +2889,7 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
     // second stage of the fused operator (q -= B^T g) with the p.q partials, or a plain dot
     auto finish_op_dot = [&](const double* pv, double* qv, hipStream_t q_s) {
         if (oss) {
-            return launch_apply_BT_dot(q_s, n, nnz, rp, ci, oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx, oss->gy,
+            return launch_apply_BT_dot(q_s, n, rp, ci, oss->oss_val, oss->bc_tag, outlet_of(oss), oss->gx, oss->gy,
                                        pv, qv, part, st);
         }
         hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(BLOCK), 0, q_s, n, pv, qv, part, st);
@@ -2895,16 +2901,16 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
         else hipLaunchKernelGGL(k_vec_mul, dim3(blocks), dim3(BLOCK), 0, q_s, n, inv_diag, rv, zv, st);
     };
 
-    // prologue (src/cfa/linalg.cuh:205-227), all decisions on the device
-    hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(BLOCK), 0, s, n, b, b, part, nullptr);
-    hipLaunchKernelGGL(k_pcg_init_bnorm, dim3(1), dim3(BLOCK), 0, s, nb, part, sc, st, status);
-    hipLaunchKernelGGL(k_zero_if_trivial, dim3(blocks), dim3(BLOCK), 0, s, n, x, st);
+    // prologue (src/cfa/linalg.cuh:205-227), all decisions on the device (the state is set by k_pcg_init;
+    // until then the kernels run whatever an earlier solve left there)
+    hipLaunchKernelGGL(k_pcg_start, dim3(1), dim3(1), 0, s, st);
     if (!amg && !prec_cb)
         hipLaunchKernelGGL(k_inv_diag, dim3(blocks), dim3(BLOCK), 0, s, n, rp, ci, val, 1.0e-14, inv_diag);
     apply_op(x, q, s);
     if (oss) (void)finish_op_dot(q, q, s);   // q -= B^T g (its dot is not used)
-    hipLaunchKernelGGL(k_pcg_residual, dim3(nb), dim3(BLOCK), 0, s, n, b, q, r, part, st);
-    hipLaunchKernelGGL(k_pcg_init_rnorm, dim3(1), dim3(BLOCK), 0, s, nb, part, sc, st, status);
+    hipLaunchKernelGGL(k_pcg_residual, dim3(nb), dim3(BLOCK), 0, s, n, b, q, r, part, part + OP_BLOCKS);
+    hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(BLOCK), 0, s, nb, part, part + OP_BLOCKS, tol, sc, st, status);
+    hipLaunchKernelGGL(k_zero_if_trivial, dim3(blocks), dim3(BLOCK), 0, s, n, x, st);
     apply_prec(r, z, s);
     hipLaunchKernelGGL(k_copy, dim3(blocks), dim3(BLOCK), 0, s, n, z, p, st);
     hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(BLOCK), 0, s, n, r, z, part, st);
@@ -2926,19 +2932,9 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
     };
     rc = run_iterations(ws, nullptr, max_iter, iteration, s);
     if (rc) return rc;
-    int fin[3];
-    double rel;
-    CFA_TRY(hipMemcpyAsync(fin, st, sizeof(fin), hipMemcpyDeviceToHost, s));
-    CFA_TRY(hipMemcpyAsync(&rel, sc + S_REL, sizeof(double), hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(k_pcg_outcome, dim3(1), dim3(1), 0, s, sc, st, status);
     CFA_TRY(hipStreamSynchronize(s));
-    if (fin[0] == ST_RUNNING) {   // iteration cap
-        result->iters[0] = max_iter;
-        result->converged[0] = 0;
-    } else {
-        result->iters[0] = fin[1];
-        result->converged[0] = fin[0] != ST_STOPPED;
-    }
-    result->rel_residual[0] = rel;
+    pcg_outcome(ws, max_iter, result);
     return launch_status();
 }
 
@@ -2986,9 +2982,7 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
     hipStream_t s = S(stream);
     for (int c = 0; c < 2; ++c) { result->iters[c] = 0; result->converged[c] = 1; result->rel_residual[c] = 0.0; }
     if (n == 0) return CFA_OK;
-    const size_t bytes = (size_t)n * sizeof(double);
     double* x = ws->vec[0];
-    double* bb = ws->vec[1];
     double* r = ws->vec[2];
     double* r0 = ws->vec[3];
     double* p = ws->vec[4];
@@ -3004,12 +2998,6 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
     double* sc = ws->scal;
     int* st = state_words(ws);
     int* status = ws->status_dev;
-    CFA_TRY(hipMemcpyAsync(x, x_u, bytes, hipMemcpyDeviceToDevice, s));
-    CFA_TRY(hipMemcpyAsync(x + n, x_v, bytes, hipMemcpyDeviceToDevice, s));
-    CFA_TRY(hipMemcpyAsync(bb, b_u, bytes, hipMemcpyDeviceToDevice, s));
-    CFA_TRY(hipMemcpyAsync(bb + n, b_v, bytes, hipMemcpyDeviceToDevice, s));
-    const double tol_v = tol;
-    CFA_TRY(hipMemcpyAsync(sc + B_TOL, &tol_v, sizeof(double), hipMemcpyHostToDevice, s));
     ws->status_host[0] = 0;
     ws->status_host[1] = ST_RUNNING;
 
@@ -3024,10 +3012,10 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
     };
     run_dispatch(n, [&](auto rb) {
         constexpr int RB = decltype(rb)::value;
-        hipLaunchKernelGGL(k_bicg_init<RB>, dim3(nb_rows), dim3(BLOCK), 0, s, n, rp, ci, val, bb, x, r, r0, p, v, part_a);
+        hipLaunchKernelGGL(k_bicg_init<RB>, dim3(nb_rows), dim3(BLOCK), 0, s, n, rp, ci, val, b_u, b_v, x_u, x_v, x, r, r0,
+                           p, v, part_a);
     });
-    hipLaunchKernelGGL(k_bicg_final_init, dim3(1), dim3(BLOCK), 0, s, nb_rows, part_a, sc, st, status, max_iter);
-    hipLaunchKernelGGL(k_bicg_pre, dim3(1), dim3(1), 0, s, sc, st, status);
+    hipLaunchKernelGGL(k_bicg_final_init, dim3(1), dim3(BLOCK), 0, s, nb_rows, part_a, tol, sc, st, status, max_iter);
     int rc = launch_status();
     if (rc) return rc;
 
@@ -3067,22 +3055,17 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
     }
     rc = run_iterations(ws, graph, max_iter, iteration, s);
     if (rc) return rc;
-    int fin[12];
-    double rel[2];
-    CFA_TRY(hipMemcpyAsync(fin, st, sizeof(fin), hipMemcpyDeviceToHost, s));
-    CFA_TRY(hipMemcpyAsync(rel, sc + B_REL, sizeof(rel), hipMemcpyDeviceToHost, s));
-    CFA_TRY(hipMemcpyAsync(x_u, x, bytes, hipMemcpyDeviceToDevice, s));
-    CFA_TRY(hipMemcpyAsync(x_v, x + n, bytes, hipMemcpyDeviceToDevice, s));
+    // at least 8 lanes in the first workgroup for the outcome's words
+    hipLaunchKernelGGL(k_bicg_outcome, dim3(blocks_for(n)), dim3(BLOCK), 0, s, n, x, x_u, x_v, sc, st, status);
+    rc = launch_status();
+    if (rc) return rc;
     CFA_TRY(hipStreamSynchronize(s));
+    const volatile int* w = ws->status_host;
     for (int c = 0; c < 2; ++c) {
-        if (fin[2 + c]) {   // still active when the loop ended (cap reached without the in-kernel stop)
-            result->iters[c] = max_iter;
-            result->converged[c] = 0;
-        } else {
-            result->iters[c] = fin[4 + c];
-            result->converged[c] = fin[6 + c];
-        }
-        result->rel_residual[c] = rel[c];
+        const bool active = w[2 + c] != 0;   // still so when the loop ended: cap reached without the in-kernel stop
+        result->iters[c] = active ? max_iter : w[4 + c];
+        result->converged[c] = active ? 0 : w[6 + c];
+        result->rel_residual[c] = published_double(w + 8 + 2 * c);
     }
     return launch_status();
 }
