@@ -532,6 +532,7 @@ struct PcgArgs {
     const double* oss; const double* inv_m; const int* tag; double* gx; double* gy;
     OutletMode om;
     double* x; double* r; double* z; double* q; double* p[2];
+    double* rbuf[2];   // residual by parity: r and the merged update's second buffer
     double* prz[2]; double* ppq; double* prr;
     int nb_rz, nb_rr;
     const double* inv_diag;
@@ -1036,6 +1037,150 @@ k_coupled_stage(CoupledStage<T, B, B2> a) {
     bool running = sv == ST_RUNNING;
     if (a.prr) running = residual_test_running(a.prr, a.nb_rr, a.sc, a.st, a.status, lds, &lds_state);
     if (running && row >= 0) dst[row] = out;
+}
+
+// The PCG update and the first stage of the cycle on the new residual in one launch: alpha with the
+// breakdown guard (k_fp_update), x += alpha p, r_new = r - alpha q into the other residual buffer, the
+// r.r partials, and stage 0 of the descent on r_new, whose entries at the neighbours are not stored yet:
+// the row sums are linear in it, so each row sums r's and q's terms apart (in FP64 also in the FP32
+// cycle) and combines them once alpha is known. The residual test moves to the next stage. Saves a launch
+// per iteration on small meshes: 4.6 + 8.0 us and a gap -> 9.6 us on 29k nodes; on 115k it is no faster
+// (5.5 + 15.4 -> 21.6 us, and the next stage 10.2 -> 12.7 us).
+constexpr int UPDATE_STAGE_ROWS = 1 << 16;
+template <typename T>
+struct UpdateStage {
+    RowSet<T, double> zero, mul;   // as in CoupledStage; b unused
+    int sell;
+    const int* s_sp; const int* s_row; const int* s_ci; const T* s_v;
+    const double* r; const double* q; const double* p;
+    double* rn; double* x;
+    const double* ppq; int nb_pq; const double* prz; int nb_rz;
+    double* prr;
+    int* st; int* status;
+};
+struct Pair {
+    double r, q;
+};
+template <typename T, typename F>
+__device__ __forceinline__ Pair lanes_row_sum2(const int* __restrict__ ci, const T* __restrict__ v, int k0, int k1,
+                                               int lane, int shift, F term) {
+    const int tpr = 1 << shift;
+    Pair s = {0.0, 0.0};
+    for (int k = k0 + lane; k < k1; k += ROW_UNROLL * tpr) {
+        int c[ROW_UNROLL];
+        T a[ROW_UNROLL];
+#pragma unroll
+        for (int u = 0; u < ROW_UNROLL; ++u) {
+            const int idx = k + u * tpr;
+            const bool ok = idx < k1;
+            c[u] = ok ? ci[idx] : 0;
+            a[u] = ok ? v[idx] : T(0);
+        }
+#pragma unroll
+        for (int u = 0; u < ROW_UNROLL; ++u) term((double)a[u], c[u], s);
+    }
+    for (int o = tpr >> 1; o > 0; o >>= 1) {
+        s.r += __shfl_down(s.r, o, tpr);
+        s.q += __shfl_down(s.q, o, tpr);
+    }
+    return s;
+}
+template <int MAXL, typename T>
+__global__ void __launch_bounds__(BLOCK)
+k_update_stage(UpdateStage<T> a) {
+    __shared__ double lds[2 * BLOCK / WAVE], lds_rr[BLOCK / WAVE];
+    __shared__ int word[2];
+    const double* __restrict__ r = a.r;
+    const double* __restrict__ q = a.q;
+    const bool first = (int)blockIdx.x >= a.mul.blocks;   // the rows of the from-zero steps and of r, x
+    int row = -1;
+    Pair s = {0.0, 0.0};
+    T wd = 0;   // omega dinv of the row
+    double ri = 0.0, qi = 0.0, pi = 0.0, xi = 0.0;
+    if (!first) {
+        const RowSet<T, double>& m = a.mul;
+        const int g = blockIdx.x * BLOCK + threadIdx.x, i = g >> m.shift, lane = g & ((1 << m.shift) - 1);
+        const int k0 = i < m.rows ? m.rp[i] : 0, k1 = i < m.rows ? m.rp[i + 1] : 0;
+        s = lanes_row_sum2(m.ci, m.v, k0, k1, lane, m.shift, [&](double v, int j, Pair& t) {
+            t.r += v * r[j];
+            t.q += v * q[j];
+        });
+        if (i < m.rows && lane == 0) row = i;
+    } else {
+        const RowSet<T, double>& m = a.zero;
+        const int blk = (int)blockIdx.x - a.mul.blocks;
+        const T* __restrict__ dinv = m.dinv;
+        const auto term = [&](double v, int j, Pair& t) {
+            const double w = v * (double)(m.omega * dinv[j]);
+            t.r += w * r[j];
+            t.q += w * q[j];
+        };
+        bool done = false;
+        if constexpr (MAXL > 0) {
+            if (a.sell == 0) {
+                const int pos = blk * BLOCK + threadIdx.x;
+                if (pos < sell_positions(m.rows)) {
+                    int base, len;
+                    (void)sell_slot(a.s_sp, a.s_row, pos, nullptr, row, base, len);
+                    int c[MAXL];
+                    T v[MAXL];
+#pragma unroll
+                    for (int k = 0; k < MAXL; ++k) {
+                        const bool ok = k < len;
+                        c[k] = ok ? a.s_ci[base + SELL_SLICE * k] : 0;
+                        v[k] = ok ? a.s_v[base + SELL_SLICE * k] : T(0);
+                    }
+#pragma unroll
+                    for (int k = 0; k < MAXL; ++k) term((double)v[k], c[k], s);
+                }
+                done = true;
+            }
+        }
+        if (!done) {
+            const int g = blk * BLOCK + threadIdx.x, i = g >> m.shift, lane = g & ((1 << m.shift) - 1);
+            const int k0 = i < m.rows ? m.rp[i] : 0, k1 = i < m.rows ? m.rp[i + 1] : 0;
+            s = lanes_row_sum2(m.ci, m.v, k0, k1, lane, m.shift, term);
+            if (i < m.rows && lane == 0) row = i;
+        }
+        if (row >= 0) {
+            wd = m.omega * dinv[row];
+            ri = r[row];
+            qi = q[row];
+            pi = a.p[row];
+            xi = a.x[row];
+        }
+    }
+    double sums[2];   // p.q, r.z
+    sum_partials_k<2, 2>({a.ppq, a.prz}, {a.nb_pq, a.nb_rz}, 1, sums, lds, a.st, word);
+    const int it = word[1];
+    if (word[0] != ST_RUNNING) return;
+    const double pq = sums[0];
+    if (fabs(pq) < 1.0e-30) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            a.st[0] = ST_STOPPED;
+            a.st[1] = it;
+            publish(a.status, it, ST_STOPPED);
+        }
+        return;
+    }
+    const double alpha = sums[1] / pq;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.st[2] = it + 1;
+    const T sum = (T)(s.r - alpha * s.q);
+    if (!first) {
+        if (row >= 0) a.mul.y[row] = sum;
+        return;
+    }
+    double acc = 0.0;
+    if (row >= 0) {
+        const double rn = ri + (-alpha) * qi;
+        a.rn[row] = rn;
+        a.x[row] = xi + alpha * pi;
+        acc = rn * rn;
+        const T b = (T)rn, x0 = wd * b;
+        a.zero.y[row] = x0 + wd * (b - sum);
+    }
+    acc = block_sum(acc, lds_rr);
+    if (threadIdx.x == 0) a.prr[blockIdx.x - a.mul.blocks] = acc;
 }
 
 // The ascent of a level: second step and coarse correction, y = x + omega dinv (b - A x) + W e
@@ -1935,6 +2080,10 @@ struct PrecHooks {
     int* status = nullptr;
     double* dot_part = nullptr;    // r.z partials out (when set)
     int dot_blocks = 0;            // set: number of r.z partials written
+    // the iteration's update runs in the cycle's first launch (k_update_stage; a hierarchy coupled from
+    // level 0 only): its arguments, and the parity of the iteration
+    const PcgArgs* update = nullptr;
+    int h = 0, nb_pq = 0;
 };
 
 // last level-0 sweep into the FP64 output, with the r.z partials when part is set; returns the
@@ -2135,9 +2284,9 @@ void coupled_stage(const cfa_amg_t* amg, int l0, int l, const B0* b0, const int*
         if (L.s_sp) a.zero.blocks = use_sell(L, 0);
         T* cb = l + 1 < bottom ? Lv<T>::b(amg->levels[l + 1]) : bottom_of<T>(amg).b;
         a.mul = {row_blocks(L.cols, shq), L.cols, shq, L.q_rp, L.q_ci, Lv<T>::q(L), nullptr, b, nullptr, T(0), cb};
-        if (l == 0 && hk && hk->prr) {
-            a.prr = hk->prr; a.nb_rr = hk->nb_rr; a.sc = hk->sc; a.st = hk->st_w; a.status = hk->status;
-        }
+    }
+    if (l == (hk && hk->update ? 1 : 0) && hk && hk->prr) {
+        a.prr = hk->prr; a.nb_rr = hk->nb_rr; a.sc = hk->sc; a.st = hk->st_w; a.status = hk->status;
     }
     if (l > l0) {
         const cfa_amg_level_t& F = amg->levels[l - 1];
@@ -2152,6 +2301,38 @@ void coupled_stage(const cfa_amg_t* amg, int l0, int l, const B0* b0, const int*
     coupled_stage_launch(a, sell, s);
 }
 
+// Workgroups of the from-zero rows of level 0, whose r.r partials k_update_stage leaves
+int update_blocks(const cfa_amg_level_t& L) {
+    return L.s_sp ? blocks_for(sell_positions(L.rows)) : row_blocks(L.rows, log2_of(L.tpr_a));
+}
+
+template <typename T>
+void update_stage(const cfa_amg_t* amg, const PrecHooks& hk, hipStream_t s) {
+    const cfa_amg_level_t& L = amg->levels[0];
+    const PcgArgs& g = *hk.update;
+    UpdateStage<T> a;
+    std::memset(&a, 0, sizeof(a));
+    const int sh = log2_of(L.tpr_a), shq = log2_of(L.tpr_q);
+    T* cb = bottom_level(amg) > 1 ? Lv<T>::b(amg->levels[1]) : bottom_of<T>(amg).b;
+    a.zero = {update_blocks(L), L.rows, sh, L.a_rp, L.a_ci, Lv<T>::a(L), nullptr, nullptr, Lv<T>::dinv(L), (T)L.omega,
+              Lv<T>::x(L)};
+    a.mul = {row_blocks(L.cols, shq), L.cols, shq, L.q_rp, L.q_ci, Lv<T>::q(L), nullptr, nullptr, nullptr, T(0), cb};
+    a.sell = L.s_sp ? 0 : -1;
+    a.s_sp = L.s_sp; a.s_row = L.s_row; a.s_ci = L.s_ci; a.s_v = L.s_sp ? Lv<T>::sv(L) : nullptr;
+    a.r = g.rbuf[hk.h]; a.q = g.q; a.p = g.p[hk.h];
+    a.rn = g.rbuf[1 - hk.h]; a.x = g.x;
+    a.ppq = g.ppq; a.nb_pq = hk.nb_pq; a.prz = g.prz[hk.h]; a.nb_rz = g.nb_rz;
+    a.prr = g.prr; a.st = g.st; a.status = g.status;
+    auto go = [&](auto m) {
+        hipLaunchKernelGGL((k_update_stage<decltype(m)::value, T>), dim3(a.mul.blocks + a.zero.blocks), dim3(BLOCK), 0, s,
+                           a);
+    };
+    if (!L.s_sp) go(std::integral_constant<int, 0>{});
+    else if (L.s_len <= 8) go(std::integral_constant<int, 8>{});
+    else if (L.s_len <= 12) go(std::integral_constant<int, 12>{});
+    else go(std::integral_constant<int, 16>{});
+}
+
 // The coupled cycle from level l0 with right-hand side b0 (FP64 on level 0, also in the FP32 cycle);
 // the result in level l0's x buffer, or on level 0 in the FP64 `out`, with the r.z partials.
 template <typename T, typename B0>
@@ -2159,7 +2340,8 @@ T* coupled_vcycle(const cfa_amg_t* amg, int l0, const B0* b0, double* out, const
                   PrecHooks* hk) {
     const int bottom = bottom_level(amg);
     for (int l = l0; l <= bottom; ++l) {
-        if (l == l0) coupled_stage<T, B0, T, B0>(amg, l0, l, b0, st, s, hk);
+        if (l == 0 && hk && hk->update) update_stage<T>(amg, *hk, s);
+        else if (l == l0) coupled_stage<T, B0, T, B0>(amg, l0, l, b0, st, s, hk);
         else if (l == l0 + 1) coupled_stage<T, T, B0, B0>(amg, l0, l, b0, st, s, hk);
         else coupled_stage<T, T, T, B0>(amg, l0, l, b0, st, s, hk);
     }
@@ -2674,6 +2856,14 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
     double* inv_diag = ws->vec[4];
     a.inv_diag = inv_diag;
     a.x = x;
+    a.rbuf[0] = a.r;
+    a.rbuf[1] = ws->vec[6];
+    // The update in the cycle's first launch where a launch costs more than what it adds: both gathers of
+    // every level-0 entry of A and W^T, and the residual test's sums in every workgroup of the next stage.
+    // Time steps merged / apart: 2.53 / 2.60 ms on 29k nodes, 4.85 / 4.74 ms on 115k. Its partials (at most
+    // one per 8 rows' lanes, 2048) fit their segment.
+    const bool merged = amg && amg->n_levels > 0 && coupled_from(amg, 0) && n <= UPDATE_STAGE_ROWS &&
+                        update_blocks(amg->levels[0]) <= OP_BLOCKS;
     // block partials: four segments of OP_BLOCKS doubles, then the prologue's (5 * 4096 of the
     // workspace's 8 * 4096)
     a.prz[0] = ws->part; a.prz[1] = ws->part + OP_BLOCKS; a.ppq = ws->part + 2 * OP_BLOCKS;
@@ -2716,7 +2906,7 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
         return nb;
     };
     a.nb_rz = apply_prec(0, false, s);
-    a.nb_rr = nb;
+    a.nb_rr = merged ? update_blocks(amg->levels[0]) : nb;
     int rc = launch_status();
     if (rc) return rc;
 
@@ -2725,6 +2915,14 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
         launch_fp_operator(oss != nullptr, q_s, a, h);
         if (oss)
             (void)launch_apply_BT_dot(q_s, n, rp, ci, a.oss, a.tag, a.om, a.gx, a.gy, a.p[h], a.q, a.ppq, st_r);
+        if (merged) {
+            PrecHooks hk;
+            hk.prr = a.prr; hk.nb_rr = a.nb_rr; hk.sc = a.sc; hk.st_w = a.st; hk.status = a.status;
+            hk.dot_part = a.prz[1 - h];
+            hk.update = &a; hk.h = h; hk.nb_pq = nb_op;
+            amg_apply_enqueue(amg, a.rbuf[1 - h], a.z, st_r, q_s, &hk);
+            return;
+        }
         hipLaunchKernelGGL(k_fp_update, dim3(nb), dim3(BLOCK), 0, q_s, a, h, nb_op);
         (void)apply_prec(1 - h, true, q_s);
     };

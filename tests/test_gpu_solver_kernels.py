@@ -2,8 +2,9 @@
 the cycle against the one with separate residual, restriction and prolongation (uniform levels 1, 3
 and 4: one to four smoothed levels, with the dense bottom at none, the last or the first coarse one);
 the pressure operator's row runs at the edges of their tiles against sums on the host; the dense
-inverse of the coarsest operator at the edges of its blocks; and the ILU(0) sweeps where the trailing
-colours change path."""
+inverse of the coarsest operator at the edges of its blocks; the ILU(0) sweeps where the trailing
+colours change path; and pressure solves in FP64 and with the FP32 cycle against the oracle's on both
+sides of 65,536 rows, up to where the PCG update runs in the cycle's first launch."""
 import subprocess
 from pathlib import Path
 
@@ -26,5 +27,14 @@ def test_coupled_cycle(level):
 def test_tile_edges(case):
     print(f"[case] {case}", flush=True)
     r = subprocess.run([str(BIN), case, "0"], capture_output=True, text=True, timeout=120)
+    print(r.stdout)
+    assert r.returncode == 0 and "ALL PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("case", ["pcg", "mixed"])
+@pytest.mark.parametrize("level", [2, 4])
+def test_pressure_solve(case, level):
+    print(f"[case] {case} level {level}", flush=True)
+    r = subprocess.run([str(BIN), case, str(level)], capture_output=True, text=True, timeout=120)
     print(r.stdout)
     assert r.returncode == 0 and "ALL PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-2000:]
