@@ -703,6 +703,36 @@ void gather(const cfa_mesh_t* m, int nf, const double* contrib, double* const* o
                        m->inc_ptr, m->inc_elem, contrib, o);
 }
 
+// ---- contraction with the boundary modes ----------------------------------------------------------
+// A lane per mode, a wavefront per node in turn: the node's coordinates and sensitivities are the same for
+// all lanes, its radius and angle are taken once, and each lane adds its Gaussian's term. Partials per
+// wavefront, added in their order. On the host the 64 x n weights (hypot, atan2 and exp each) took 22 ms
+// on 29k nodes.
+constexpr int SHAPE_WAVES = CFA_ADJ_SHAPE_WS / WAVE;
+__global__ void __launch_bounds__(BLOCK)
+k_adj_shape(int n, const double* __restrict__ x0, const double* __restrict__ y0, const double* __restrict__ xb,
+            const double* __restrict__ yb, double xc, double yc, double radius, double* __restrict__ part) {
+    const int k = threadIdx.x % WAVE, w = (blockIdx.x * BLOCK + threadIdx.x) / WAVE;
+    constexpr double pi = 3.14159265358979323846;
+    const double sigma = 2.0 * pi / WAVE, outer = 3.0 * radius;
+    double acc = 0.0;
+    for (int i = w; i < n; i += SHAPE_WAVES) {
+        const double dx = x0[i] - xc, dy = y0[i] - yc, r = hypot(dx, dy);
+        if (r >= outer || r <= 0.0) continue;
+        const double t = fmin(1.0, fmax(0.0, (r - radius) / (outer - radius)));
+        const double chi = 1.0 - t * t * (3.0 - 2.0 * t);
+        const double d = remainder(atan2(dy, dx) - 2.0 * pi * k / WAVE, 2.0 * pi);
+        acc += radius * exp(-0.5 * (d / sigma) * (d / sigma)) * chi / r * (xb[i] * dx + yb[i] * dy);
+    }
+    part[(size_t)w * WAVE + k] = acc;
+}
+__global__ void __launch_bounds__(WAVE) k_adj_shape_sum(const double* __restrict__ part, double* __restrict__ out) {
+    double s = 0.0;
+#pragma unroll 16
+    for (int w = 0; w < SHAPE_WAVES; ++w) s += part[(size_t)w * WAVE + threadIdx.x];
+    out[threadIdx.x] = s;
+}
+
 void accumulate(int count, const double* part, double* theta_bar, int slot, hipStream_t st) {
     hipLaunchKernelGGL(k_adj_accumulate, dim3(ADJ_OUT_BLOCKS), dim3(BLOCK), 0, st, count, part, theta_bar, slot);
 }
@@ -859,6 +889,16 @@ int cfa_scale(int n, double a, double* x, cfa_stream_t stream) {
     if (n < 0 || (n > 0 && !x)) return CFA_E_ARG;
     if (n == 0) return CFA_OK;
     hipLaunchKernelGGL(k_scale, dim3(blocks_for(n)), dim3(BLOCK), 0, as_stream(stream), n, a, x);
+    return launch_status();
+}
+
+int cfa_adj_shape_modes(int n, const double* x0, const double* y0, const double* x_bar, const double* y_bar, double xc,
+                        double yc, double radius, double* ws, double* out, cfa_stream_t stream) {
+    if (n < 0 || (n > 0 && (!x0 || !y0 || !x_bar || !y_bar)) || !(radius > 0.0) || !ws || !out) return CFA_E_ARG;
+    const hipStream_t s = as_stream(stream);
+    hipLaunchKernelGGL(k_adj_shape, dim3(SHAPE_WAVES * WAVE / BLOCK), dim3(BLOCK), 0, s, n, x0, y0, x_bar, y_bar, xc, yc,
+                       radius, ws);
+    hipLaunchKernelGGL(k_adj_shape_sum, dim3(1), dim3(WAVE), 0, s, ws, out);
     return launch_status();
 }
 

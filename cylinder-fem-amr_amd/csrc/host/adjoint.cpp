@@ -159,17 +159,16 @@ public:
         dev_sync();
     }
     // dJ/deps_k = sum_i x_bar_i dx_i/deps_k + y_bar_i dy_i/deps_k
-    void shape_gradient(double* out) const {
-        const std::vector<double> xb = d_xb_.to_host(n), yb = d_yb_.to_host(n);
-        for (int k = 0; k < kModes; ++k) {
-            double acc = 0.0;
-            for (int i = 0; i < n; ++i) {
-                const double dx = x0_[i] - Sim::X_CYL, dy = y0_[i] - Sim::Y_CYL;
-                const double w = mode_weight(k, dx, dy);
-                if (w != 0.0) acc += w * (xb[i] * dx + yb[i] * dy);
-            }
-            out[k] = acc;
+    void shape_gradient(double* out) {
+        static_assert(kModes == 64, "cfa_adj_shape_modes");
+        if (!d_x0_.ptr) {
+            d_x0_.upload(x0_);
+            d_y0_.upload(y0_);
         }
+        d_shape_.reserve(kModes + CFA_ADJ_SHAPE_WS, 0);
+        GPU_CHECK(cfa_adj_shape_modes(n, d_x0_, d_y0_, d_xb_, d_yb_, Sim::X_CYL, Sim::Y_CYL, Sim::R_CYL,
+                                      d_shape_ + kModes, d_shape_, solver_stream()));
+        d_shape_.download(out, kModes);
     }
 
     // device state [u | v | u_old | v_old | p | dp] <-> the working arrays
@@ -316,6 +315,7 @@ private:
     DevArray<int> d_perm_;
     DevArray<double> d_AT_, d_ws_, d_theta_bar_, d_state_, ustar_, lam_m_, lam_p_, dpb_, usb_, vec_tmp_;
     DevArray<double> adj_a_, adj_b_, d_xb_, d_yb_;
+    DevArray<double> d_x0_, d_y0_, d_shape_;   // undeformed coordinates and mode sums of the shape gradient
     std::vector<double> initial_[5];
     std::vector<double> x0_, y0_;       // undeformed node coordinates
     double eps_[kModes] = {};            // radial boundary modes in use

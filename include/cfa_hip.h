@@ -748,6 +748,13 @@ int cfa_adj_forces(const cfa_mesh_t* m, const double* u, const double* v, const 
                    double b1, double b2, double nu, double rho, double wx, double wy, double* ws, double* u_bar,
                    double* v_bar, double* u_old_bar, double* v_old_bar, double* u_prev_bar, double* v_prev_bar,
                    double* p_bar, double* x_bar, double* y_bar, double* theta_bar, cfa_stream_t stream);
+/* out[k] = sum_i w_k(i) (x_bar_i dx_i + y_bar_i dy_i), k < 64: the contraction of coordinate
+ * sensitivities with the 64 radial modes of the hole boundary of cfa_adjoint_set_shape, (dx, dy) = (x0 - xc,
+ * y0 - yc) at the undeformed coordinates and w_k(i) = radius g_k(phi) chi(r) / r. out (device) [64];
+ * ws: CFA_ADJ_SHAPE_WS doubles. Summed in a fixed order. */
+#define CFA_ADJ_SHAPE_WS 65536
+int cfa_adj_shape_modes(int n, const double* x0, const double* y0, const double* x_bar, const double* y_bar, double xc,
+                        double yc, double radius, double* ws, double* out, cfa_stream_t stream);
 /* out[k] = in[perm[k]], k < nnz (CSR values of A^T on a symmetric pattern); x *= a. */
 int cfa_gather_values(int nnz, const int* perm, const double* in, double* out, cfa_stream_t stream);
 int cfa_scale(int n, double a, double* x, cfa_stream_t stream);
