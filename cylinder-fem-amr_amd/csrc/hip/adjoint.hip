@@ -165,6 +165,9 @@ __device__ __forceinline__ bool dirichlet_velocity(int t) {
     return t == BC_INLET || t == BC_WALL || t == BC_CYLINDER;
 }
 
+// The element kernels state their workgroup size: without it the compiler assumes 1024 threads and gives
+// each 128 registers, and the dual numbers spilled up to 3.4 KB a lane. With 256 threads a wave may have
+// all 512: momentum, forces, pressure on 57k elements 386 -> 62, 223 -> 75, 110 -> 32 us.
 // Gradient of an element functional phi(in[0..n_in)) by forward passes of ND directions over the
 // inputs from `first` on: grad[q] = d phi / d in[q]. `f(in, value_pass)` returns phi as a dual and
 // reports a degenerate element by returning false in its ok flag.
@@ -192,7 +195,8 @@ __device__ __forceinline__ bool element_gradient(int n_in, int first, const doub
 // inputs: X[3], Y[3] (coordinates), WU[3], WV[3] (advecting velocity c1 u^n + c2 u^{n-1}), nu;
 // the right-hand-side data u^h, p enter linearly (their derivatives from the value pass).
 // contrib fields (stride 3 ne): 0 u_n, 1 v_n, 2 u_{n-1}, 3 v_{n-1}, 4 p, 5 x, 6 y; nu_part[e]
-__global__ void k_adj_momentum_elems(int ne, const int* __restrict__ ev, const double* __restrict__ x,
+__global__ void __launch_bounds__(BLOCK)
+k_adj_momentum_elems(int ne, const int* __restrict__ ev, const double* __restrict__ x,
                                      const double* __restrict__ y, const int* __restrict__ tag,
                                      const double* __restrict__ un, const double* __restrict__ vn,
                                      const double* __restrict__ um, const double* __restrict__ vm,
@@ -310,7 +314,8 @@ __global__ void k_adj_momentum_elems(int ne, const int* __restrict__ ev, const d
 // with s_K = s(mean u*, nu, |K|) as k_oss_weights (fem_kernels.cuh:697-719).
 // inputs: X[3], Y[3], US[3], VS[3], nu; y enters linearly (p^n derivative from the value pass).
 // contrib fields: 0 u*, 1 v*, 2 p, 3 x, 4 y; nu_part[e]
-__global__ void k_adj_pressure_elems(int ne, const int* __restrict__ ev, const double* __restrict__ x,
+__global__ void __launch_bounds__(BLOCK)
+k_adj_pressure_elems(int ne, const int* __restrict__ ev, const double* __restrict__ x,
                                      const double* __restrict__ y, const double* __restrict__ us,
                                      const double* __restrict__ vs, const double* __restrict__ lam,
                                      const double* __restrict__ yv, const double* __restrict__ dp,
@@ -406,7 +411,8 @@ __global__ void k_adj_pressure_elems(int ne, const int* __restrict__ ev, const d
 // / m, q = p1_bar / m and c_i = [-(dt/rho) z_i.(G dp)_i + nu dt q_i (K dp)_i] / m_i held fixed,
 //   Phi_K = sum_i [-(dt/rho) z_i.grad dp_K |K|/3 + nu dt q_i |K| grad N_i.grad dp_K - c_i |K|/3]
 // inputs X[3], Y[3]; contrib fields: 0 x, 1 y
-__global__ void k_adj_corr_geom_elems(int ne, const int* __restrict__ ev, const double* __restrict__ x,
+__global__ void __launch_bounds__(BLOCK)
+k_adj_corr_geom_elems(int ne, const int* __restrict__ ev, const double* __restrict__ x,
                                       const double* __restrict__ y, const double* __restrict__ dp,
                                       const double* __restrict__ zx, const double* __restrict__ zy,
                                       const double* __restrict__ q, const double* __restrict__ c, double nu,
@@ -466,7 +472,8 @@ __global__ void k_adj_corr_c(int n, const double* __restrict__ mass, const doubl
 // inputs (28): X[3], Y[3], then u, v, u_old, v_old, u_prev, v_prev, p at the three corners, nu
 // contrib fields: 0 u, 1 v, 2 u_old, 3 v_old, 4 u_prev, 5 v_prev, 6 p, 7 x, 8 y; nu_part[e].
 // Elements that do not touch the cylinder write zeros.
-__global__ void k_adj_forces_elems(int ne, const int* __restrict__ ev, const int* __restrict__ tag,
+__global__ void __launch_bounds__(BLOCK)
+k_adj_forces_elems(int ne, const int* __restrict__ ev, const int* __restrict__ tag,
                                    const double* __restrict__ x, const double* __restrict__ y,
                                    const double* __restrict__ u, const double* __restrict__ v,
                                    const double* __restrict__ uo, const double* __restrict__ vo,
@@ -562,11 +569,25 @@ __global__ void k_adj_gather(int n, int ne, int nf, const int* __restrict__ inc_
     }
 }
 
-// theta_bar[slot] += sum of part[0..count) (one workgroup, fixed order)
-__global__ void k_adj_accumulate(int count, const double* __restrict__ part, double* __restrict__ theta_bar,
-                                 int slot) {
-    __shared__ double lds[BLOCK / WAVE];
-    const double s = sum_partials(part, count, 1, lds);
+// theta_bar[slot] += sum of part[0..count) (one workgroup, fixed order; eight loads in flight per lane:
+// 45 -> 7.6 us for 57k partials)
+constexpr int ACC_THREADS = 1024;
+__global__ void __launch_bounds__(ACC_THREADS)
+k_adj_accumulate(int count, const double* __restrict__ part, double* __restrict__ theta_bar, int slot) {
+    __shared__ double lds[ACC_THREADS / WAVE];
+    constexpr int U = 8;
+    double s = 0.0;
+    for (int k0 = 0; k0 < count; k0 += U * ACC_THREADS) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * ACC_THREADS + (int)threadIdx.x;
+            v[u] = k < count ? part[k] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += v[u];
+    }
+    s = block_sum(s, lds);
     if (threadIdx.x == 0) theta_bar[slot] += s;
 }
 
@@ -734,7 +755,7 @@ __global__ void __launch_bounds__(WAVE) k_adj_shape_sum(const double* __restrict
 }
 
 void accumulate(int count, const double* part, double* theta_bar, int slot, hipStream_t st) {
-    hipLaunchKernelGGL(k_adj_accumulate, dim3(ADJ_OUT_BLOCKS), dim3(BLOCK), 0, st, count, part, theta_bar, slot);
+    hipLaunchKernelGGL(k_adj_accumulate, dim3(ADJ_OUT_BLOCKS), dim3(ACC_THREADS), 0, st, count, part, theta_bar, slot);
 }
 
 }  // namespace
