@@ -2834,6 +2834,18 @@ OutletMode outlet_of(const cfa_oss_op_t* oss) {
     return OutletMode{oss->outlet_dirichlet, oss->p_pin, 0.0};
 }
 
+// Where the outcome kernels write: the mapped words, or the head of the (then idle) partials for a
+// workspace without a device view of them, from where outcome_arrived copies them
+int* outcome_words(const cfa_krylov_ws_t* ws) {
+    return ws->status_dev ? ws->status_dev : reinterpret_cast<int*>(ws->part);
+}
+int outcome_arrived(const cfa_krylov_ws_t* ws, hipStream_t s) {
+    if (!ws->status_dev)
+        CFA_TRY(hipMemcpyAsync(ws->status_host + 2, outcome_words(ws) + 2, 12 * sizeof(int), hipMemcpyDeviceToHost, s));
+    CFA_TRY(hipStreamSynchronize(s));
+    return CFA_OK;
+}
+
 // k_pcg_outcome's words as the solve's result
 void pcg_outcome(const cfa_krylov_ws_t* ws, int max_iter, cfa_solve_result_t* result) {
     const volatile int* w = ws->status_host;
@@ -2953,10 +2965,11 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
         if (graph) CFA_TRY(hipGraphLaunch(graph, s));
         else two_iterations(s);
     }
-    hipLaunchKernelGGL(k_pcg_outcome, dim3(1), dim3(1), 0, s, a.sc, a.st, a.status);
+    hipLaunchKernelGGL(k_pcg_outcome, dim3(1), dim3(1), 0, s, a.sc, a.st, outcome_words(ws));
     rc = launch_status();
     if (rc) return rc;
-    CFA_TRY(hipStreamSynchronize(s));
+    rc = outcome_arrived(ws, s);
+    if (rc) return rc;
     pcg_outcome(ws, max_iter, result);
     return launch_status();
 }
@@ -3130,8 +3143,9 @@ int cfa_pcg(int n, const int* rp, const int* ci, const double* val, const double
     };
     rc = run_iterations(ws, nullptr, max_iter, iteration, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_pcg_outcome, dim3(1), dim3(1), 0, s, sc, st, status);
-    CFA_TRY(hipStreamSynchronize(s));
+    hipLaunchKernelGGL(k_pcg_outcome, dim3(1), dim3(1), 0, s, sc, st, outcome_words(ws));
+    rc = outcome_arrived(ws, s);
+    if (rc) return rc;
     pcg_outcome(ws, max_iter, result);
     return launch_status();
 }
@@ -3254,10 +3268,12 @@ int cfa_bicgstab2(int n, const int* rp, const int* ci, const double* val, const 
     rc = run_iterations(ws, graph, max_iter, iteration, s);
     if (rc) return rc;
     // at least 8 lanes in the first workgroup for the outcome's words
-    hipLaunchKernelGGL(k_bicg_outcome, dim3(blocks_for(n)), dim3(BLOCK), 0, s, n, x, x_u, x_v, sc, st, status);
+    hipLaunchKernelGGL(k_bicg_outcome, dim3(blocks_for(n)), dim3(BLOCK), 0, s, n, x, x_u, x_v, sc, st,
+                       outcome_words(ws));
     rc = launch_status();
     if (rc) return rc;
-    CFA_TRY(hipStreamSynchronize(s));
+    rc = outcome_arrived(ws, s);
+    if (rc) return rc;
     const volatile int* w = ws->status_host;
     for (int c = 0; c < 2; ++c) {
         const bool active = w[2 + c] != 0;   // still so when the loop ended: cap reached without the in-kernel stop

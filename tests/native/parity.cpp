@@ -1384,6 +1384,32 @@ void case_pcg(Fixture& f) {
         expect(std::abs(it - si.iters) <= 1 && solver.converged && si.converged, "iterations and convergence");
         close_rel("solution", down(f.g.d_dp, f.n), x, 1e-8);
         // the graph-replayed solve and the kernel-by-kernel solve agree
+        // and a workspace without the device view of its status words gives the same bits
+        const Vec xs = down(f.g.d_dp, f.n);
+        for (int cb = 0; cb < 2; ++cb) {   // fused, and with a host callback (its V-cycle as one)
+            auto amg_cb = [](const double* r, double* z, void* ctx) {
+                GPU_CHECK(cfa_amg_apply(static_cast<const cfa_amg_t*>(ctx), r, z, solver_stream()));
+            };
+            Vec x_dev[2];
+            for (int null_dev = 0; null_dev < 2; ++null_dev) {
+                f.g.d_dp.upload(x0);
+                KrylovWorkspace kw;
+                cfa_krylov_ws_t* ws = kw.get(f.n);
+                int* mapped = ws->status_dev;
+                if (null_dev) ws->status_dev = nullptr;
+                cfa_solve_result_t res{};
+                GPU_CHECK(cfa_pcg(f.n, f.g.d_row_ptr, f.g.d_col_ind, f.g.d_Kp_val, f.g.d_rhs_p, f.g.d_dp, 4000, tol,
+                                  &op, nullptr, nullptr, cb ? nullptr : amg.view(),
+                                  cb ? static_cast<cfa_op_cb>(amg_cb) : nullptr, const_cast<cfa_amg_t*>(amg.view()), ws,
+                                  &res, solver_stream()));
+                ws->status_dev = mapped;
+                x_dev[null_dev] = down(f.g.d_dp, f.n);
+                expect(res.converged[0] == 1 && std::abs(res.iters[0] - it) <= 1 && res.rel_residual[0] < tol,
+                       null_dev ? "outcome without mapped status words" : "outcome through mapped status words");
+            }
+            same_bits(cb ? "solution, host callback" : "solution", x_dev[1], x_dev[0]);
+            if (!cb) same_bits("solution of the solver class", x_dev[1], xs);
+        }
     }
 }
 
@@ -1455,6 +1481,25 @@ void case_bicgstab(Fixture& f) {
         close_rel(prec ? "u (FP32 factors)" : "u (FP64 factors)", down(f.g.d_u, f.n), ou, prec ? 1e-8 : 1e-9);
         close_rel(prec ? "v (FP32 factors)" : "v (FP64 factors)", down(f.g.d_v, f.n), ov, prec ? 1e-8 : 1e-9);
     }
+    // without the device view of the status words: the same bits and outcome
+    Vec x_dev[2];
+    for (int null_dev = 0; null_dev < 2; ++null_dev) {
+        f.g.d_u.upload(u0);
+        f.g.d_v.upload(v0);
+        KrylovWorkspace kw;
+        cfa_krylov_ws_t* ws = kw.get(f.n);
+        int* mapped = ws->status_dev;
+        if (null_dev) ws->status_dev = nullptr;
+        cfa_solve_result_t res{};
+        GPU_CHECK(cfa_bicgstab2(f.n, f.g.d_row_ptr, f.g.d_col_ind, f.g.d_A_val, f.g.d_rhs_u, f.g.d_rhs_v, f.g.d_u,
+                                f.g.d_v, 150, 1e-10, ilu.view(), 0, ws, &res, solver_stream()));
+        ws->status_dev = mapped;
+        x_dev[null_dev] = down(f.g.d_u, f.n);
+        expect(std::abs(res.iters[0] - bi.iters[0]) <= 1 && std::abs(res.iters[1] - bi.iters[1]) <= 1 &&
+                   res.converged[0] == 1 && res.converged[1] == 1 && res.rel_residual[1] < 1e-10,
+               null_dev ? "outcome without mapped status words" : "outcome through mapped status words");
+    }
+    same_bits("u", x_dev[1], x_dev[0]);
     // the same solves with the sweeps on the split rows' sliced-ELL copies (built at this size on
     // request; by default from 2^20 rows): iterates bit for bit, FP64 and FP32 factors
     MulticolourIlu0 ilu_csr, ilu_sell;
