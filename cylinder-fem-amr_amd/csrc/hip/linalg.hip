@@ -2190,8 +2190,11 @@ void level_from_zero_check_launch(const cfa_amg_level_t& L, const double* b, dou
     });
 }
 
+// The dense matrix is the V(2,2) cycle from its level down: other cycles go through the levels
+bool dense_bottom(const cfa_amg_t* amg) { return amg->dense && amg->smooth_steps == 2; }
+
 // The level index of the cycle's bottom: the dense level when there is one, else past the last level
-int bottom_level(const cfa_amg_t* amg) { return amg->dense ? amg->dense_level : amg->n_levels; }
+int bottom_level(const cfa_amg_t* amg) { return dense_bottom(amg) ? amg->dense_level : amg->n_levels; }
 
 // Level l and every level above the bottom carry the coupled transfers, for the V(2,2) cycle
 bool coupled_from(const cfa_amg_t* amg, int l) {
@@ -2211,7 +2214,7 @@ struct Bottom {
 };
 template <typename T>
 Bottom<T> bottom_of(const cfa_amg_t* amg) {
-    if (amg->dense) {
+    if (dense_bottom(amg)) {
         const cfa_amg_level_t& L = amg->levels[amg->dense_level];
         return {L.rows, amg->dense, Lv<T>::b(L), Lv<T>::x(L)};
     }

@@ -692,7 +692,7 @@ void case_coupled(Fixture& f) {
                           {"from level 0, dense level 1", 1 << 30, CFA_AMG_DENSE_MAX},
                           {"from level 1", f.n - 1, 0},
                           {"from level 1, dense bottom", f.n - 1, 1536}};
-    Vec plain;
+    Vec plain, plain_one;
     for (int f32 = 0; f32 < 2; ++f32) {
         for (int k = -1; k < 5; ++k) {
             AmgPreconditioner amg;
@@ -711,6 +711,13 @@ void case_coupled(Fixture& f) {
                 expect(with == (int)amg.levels.size() - (forms[k].couple < f.n ? 1 : 0), "levels coupled");
                 expect((amg.view()->dense != nullptr) == (forms[k].dense > 0), "dense bottom");
             }
+            if (f32) continue;
+            // V(1,1) on the same hierarchy: the dense matrix is V(2,2)'s and stays out of it
+            cfa_amg_t one = *amg.view();
+            one.smooth_steps = 1;
+            GPU_CHECK(cfa_amg_apply(&one, d_r, d_z, solver_stream()));
+            if (k < 0) plain_one = down(d_z, f.n);
+            else same_bits("one sweep", down(d_z, f.n), plain_one);
         }
     }
 }
