@@ -31,6 +31,10 @@ namespace {
 constexpr int FRONT_THREADS = 1024;
 constexpr int FRONT_ROWS = 8;                                // window rows per thread
 constexpr int FRONT_WINDOW = FRONT_THREADS * FRONT_ROWS;    // rows per window at most
+constexpr int ROUND_LANES = 8;                              // lanes per queued row
+constexpr int ROUND_ENTRIES = 2;                             // list entries a lane handles together
+constexpr int STAGE_ENTRIES = 16;                            // conflicts of a row staged together
+constexpr int Q_LEN = 0xffff, Q_PENDING = 1 << 16;           // word of a round: queue length, rows that walk
 constexpr int FRONT_LIST = 45056;                            // staged upper-list entries (LDS, 88 KB)
 
 int nblk(long long n) { return blocks_for(n > 0 ? n : 1); }
@@ -169,34 +173,31 @@ __device__ __forceinline__ void wave_append(bool want, unsigned short item, unsi
     const int lane = threadIdx.x & (WAVE - 1), leader = __ffsll((long long)m) - 1;
     int b = 0;
     if (lane == leader) b = atomicAdd(qn, __popcll(m));
-    b = __shfl(b, leader, WAVE);
+    b = __builtin_amdgcn_readlane(b, __builtin_amdgcn_readfirstlane(leader));
     if (want) q[b + __popcll(m & ((1ull << lane) - 1))] = item;
 }
 
-// LDS word of a window row: bits 0-7 its lower conflicts in the window not yet decided, bit 8 a
-// lower root seen, bit 9 a row with a long list (decides by walking the graph), bits 10-11 its
-// decision once processed (1 root, 2 not a root), bits 16-31 the start of its upper list (the
-// window rows that have it as a lower conflict; lists in row order, word wn holds the end).
-constexpr unsigned W_FLAG = 1u << 8, W_LONG = 1u << 9, W_ROOT = 1u << 10, W_NOT = 2u << 10, W_DONE = 3u << 10;
+// LDS word of a window row: bits 0-7 its lower conflicts in the window not yet decided as no roots
+// (W_LONG: a row that decides by walking the graph), bits 8-15 the lower roots seen (one for all below
+// the window; one for a row outside the phase), bits 16-31 the start of its upper list (the window rows
+// that have it as a lower conflict; lists in row order, word wn holds the end). A row is decided as no
+// root once it has seen a root, and as a root once nothing is left in bits 0-7 without one. Slots hold
+// at most 128 conflicts, so neither count runs over.
+constexpr unsigned W_COUNT = 0xffu, W_LONG = 0xffu, W_ROOT_SEEN = 1u << 8, W_ROOTS = 0xff00u;
 
-// stage the lower conflicts of the window rows (vector loads of the row's slot): f(r) per entry
-template <typename F>
-__device__ __forceinline__ void for_lower(const int* __restrict__ lc, int cap, int i, int raw, F f) {
-    const int4* row4 = reinterpret_cast<const int4*>(lc + (size_t)i * cap);
-    for (int b = 0; b < raw; b += 16) {
-        int4 v[4];
+// The entries [b, b + STAGE_ENTRIES) of row i's `len` conflicts (slots are multiples of 8 entries, so
+// whole vectors stay inside)
+__device__ __forceinline__ void load_lower(const int* __restrict__ lc, int cap, int i, int b,
+                                           int len, int (&e)[STAGE_ENTRIES]) {
+    const int4* row4 = reinterpret_cast<const int4*>(lc + (size_t)i * cap + b);
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (b + 4 * c < raw) v[c] = row4[b / 4 + c];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int e[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (b + 4 * c + j >= raw) break;
-                f(e[j]);
-            }
-        }
+    for (int c = 0; c < STAGE_ENTRIES / 4; ++c) {
+        int4 v = make_int4(0, 0, 0, 0);
+        if (b + 4 * c < len) v = row4[c];
+        e[4 * c] = v.x;
+        e[4 * c + 1] = v.y;
+        e[4 * c + 2] = v.z;
+        e[4 * c + 3] = v.w;
     }
 }
 
@@ -207,11 +208,20 @@ __device__ __forceinline__ void for_lower(const int* __restrict__ lc, int cap, i
 // conflicts in the window and the list of window rows it is a lower conflict of. A row whose
 // count reaches zero without a lower root (a root), or that meets a lower root (not a root), is
 // queued by the update that decided it; each round processes the queue: the row's decision goes
-// to `state`, and to its upper rows (a flag, or a decrement, by LDS atomics whose old value shows
+// to its word, and to its upper rows (a flag, or a decrement, by LDS atomics whose old value shows
 // whether this update decided that row). Rows with more lower conflicts than their slot holds
 // walk the graph every round until they decide, then join the queue. The lowest undecided row is
 // always decidable, so every window ends. state (global): 0 undecided, 1 root, 2 not a root
-// (rows outside the phase are 2 from the start).
+// (rows outside the phase are 2 from the start); written from the words when the window has ended.
+//
+// A round is a chain of LDS round trips between two barriers (item, word, list entries, atomics, queue
+// cursor), some 90 rounds a window, bound by its latency and by the instructions of the waves that share
+// a SIMD. So nothing else lies in it: the states are stored once per window (a store would be waited for
+// at the round's barrier), the queue length is carried from the round before, a root's flag and a
+// no-root's decrement are one add, idle lanes add 0 instead of branching, and waves past the queue go
+// straight to the barrier. A round takes 0.83 us (it was 1.35), the aggregation of the 1.84 million
+// rows' hierarchy 60 ms (75), of 116 thousand 5.1 ms (6.25). Lanes and entries per queued row: 8 x 2
+// 21.1 ms of rounds on the large mesh, 8 x 1 the same, 4 x 4 23.3, 16 x 1 23.8; 512 threads 24.4.
 __global__ __launch_bounds__(FRONT_THREADS) void k_front(int n, int mode, const int* __restrict__ s_rp,
                                                          const int* __restrict__ s_ci, const int* __restrict__ t_rp,
                                                          const int* __restrict__ t_ci, const int* __restrict__ lc,
@@ -221,20 +231,22 @@ __global__ __launch_bounds__(FRONT_THREADS) void k_front(int n, int mode, const 
     __shared__ unsigned s_word[FRONT_WINDOW + 1];
     __shared__ unsigned short s_q[2][FRONT_WINDOW];
     __shared__ int s_scan[FRONT_THREADS / WAVE];
-    __shared__ int s_qn[3], s_pend[3];
-    const int t = threadIdx.x;
+    __shared__ int s_qn[3];
+    const int t = threadIdx.x, lane = t & (WAVE - 1);
+    const int wave_item = t / WAVE * (WAVE / ROUND_LANES);   // first queue item of this wave
     int rounds = 0;
     for (int lo = 0; lo < n;) {
         // the window: as many rows as their listed conflicts allow
         int width = FRONT_WINDOW, hi = lo, total = 0;
+        int raw[FRONT_ROWS];
+#pragma unroll
+        for (int k = 0; k < FRONT_ROWS; ++k) raw[k] = lc_len[min(lo + t + k * FRONT_THREADS, n - 1)];
         while (true) {
             hi = min(n, lo + width);
             int mine = 0;
 #pragma unroll
-            for (int k = 0; k < FRONT_ROWS; ++k) {
-                const int i = lo + t + k * FRONT_THREADS;
-                if (i < hi) mine += max(lc_len[i], 0);
-            }
+            for (int k = 0; k < FRONT_ROWS; ++k)
+                if (lo + t + k * FRONT_THREADS < hi) mine += max(raw[k], 0);
             (void)block_scan_front(mine, s_scan, total);
             if (total <= FRONT_LIST) break;
             const int cut = (int)((long long)width * FRONT_LIST / total);   // uniform: every thread saw total
@@ -252,68 +264,84 @@ __global__ __launch_bounds__(FRONT_THREADS) void k_front(int n, int mode, const 
         unsigned longs = 0;   // row slots of this thread with a long list, undecided
 #pragma unroll
         for (int k = 0; k < FRONT_ROWS; ++k) {
-            const int loc = t + k * FRONT_THREADS;
-            own[k] = 0;
-            if (loc >= wn) continue;
-            const int i = lo + loc;
-            const int raw = lc_len[i];
+            const int loc = t + k * FRONT_THREADS, i = min(lo + loc, n - 1);
+            const int len = loc < wn ? raw[k] : 0;
             unsigned w = 0;
-            if (raw < 0) {
+            for (int b = 0; b < len; b += STAGE_ENTRIES) {
+                // the states of the conflicts below the window in flight together
+                int e[STAGE_ENTRIES], sv[STAGE_ENTRIES];
+                load_lower(lc, cap, i, b, len, e);
+#pragma unroll
+                for (int j = 0; j < STAGE_ENTRIES; ++j) {
+                    sv[j] = 0;
+                    if (b + j < len && e[j] < lo) sv[j] = state[e[j]];
+                }
+#pragma unroll
+                for (int j = 0; j < STAGE_ENTRIES; ++j)
+                    if (b + j < len) {
+                        if (e[j] >= lo) {
+                            ++w;
+                            atomicAdd(&s_word[e[j] - lo], 1u);
+                        } else if (sv[j] == 1) {
+                            w |= W_ROOT_SEEN;
+                        }
+                    }
+            }
+            if (loc < wn && raw[k] < 0) {
                 w = W_LONG;
                 longs |= 1u << k;
-            } else {
-                for_lower(lc, cap, i, raw, [&](int r) {
-                    if (r < lo) {
-                        if (state[r] == 1) w |= W_FLAG;
-                    } else {
-                        ++w;
-                        atomicAdd(&s_word[r - lo], 1u);
-                    }
-                });
             }
             if (state[i] != 0) {   // outside the phase: not a root
-                w |= W_FLAG;
+                w |= W_ROOT_SEEN;
                 longs &= ~(1u << k);
             }
             own[k] = w;
         }
         __syncthreads();
-        // pass 2: upper-list starts in row order (one scan per row slot), fill cursors in s_word
-        int ucnt[FRONT_ROWS], ubeg[FRONT_ROWS];
+        // pass 2: upper-list starts in row order (each thread scans FRONT_ROWS consecutive rows), as
+        // fill cursors in s_word
+        unsigned ubeg[FRONT_ROWS];
+        {
+            int mine = 0, all = 0;
+#pragma unroll
+            for (int k = 0; k < FRONT_ROWS; ++k) {
+                const int loc = t * FRONT_ROWS + k;
+                ubeg[k] = loc < wn ? s_word[loc] : 0;
+                mine += (int)ubeg[k];
+            }
+            int at = block_scan_front(mine, s_scan, all);
+#pragma unroll
+            for (int k = 0; k < FRONT_ROWS; ++k) {
+                const int loc = t * FRONT_ROWS + k;
+                if (loc < wn) s_word[loc] = (unsigned)at;
+                at += (int)ubeg[k];
+            }
+            if (t == 0) s_word[wn] = (unsigned)all;
+        }
+        __syncthreads();
+        bool upper[FRONT_ROWS];   // the row has upper rows
 #pragma unroll
         for (int k = 0; k < FRONT_ROWS; ++k) {
             const int loc = t + k * FRONT_THREADS;
-            ucnt[k] = loc < wn ? (int)s_word[loc] : 0;
-        }
-        int run = 0;
-#pragma unroll
-        for (int k = 0; k < FRONT_ROWS; ++k) {
-            int tot = 0;
-            ubeg[k] = run + block_scan_front(ucnt[k], s_scan, tot);
-            run += tot;
-        }
-#pragma unroll
-        for (int k = 0; k < FRONT_ROWS; ++k) {
-            const int loc = t + k * FRONT_THREADS;
-            if (loc < wn) s_word[loc] = ubeg[k];
+            ubeg[k] = loc < wn ? s_word[loc] : 0;
+            upper[k] = loc < wn && s_word[loc + 1] > ubeg[k];
         }
         __syncthreads();
         // pass 3: the upper lists
 #pragma unroll
         for (int k = 0; k < FRONT_ROWS; ++k) {
-            const int loc = t + k * FRONT_THREADS;
-            if (loc >= wn) continue;
-            const int i = lo + loc;
-            const int raw = lc_len[i];
-            if (raw > 0)
-                for_lower(lc, cap, i, raw, [&](int r) {
-                    if (r >= lo) s_up[atomicAdd(&s_word[r - lo], 1u)] = (unsigned short)loc;
-                });
+            const int loc = t + k * FRONT_THREADS, i = min(lo + loc, n - 1);
+            const int len = loc < wn ? raw[k] : 0;
+            for (int b = 0; b < len; b += STAGE_ENTRIES) {
+                int e[STAGE_ENTRIES];
+                load_lower(lc, cap, i, b, len, e);
+#pragma unroll
+                for (int j = 0; j < STAGE_ENTRIES; ++j)
+                    if (b + j < len && e[j] >= lo)
+                        s_up[atomicAdd(&s_word[e[j] - lo], 1u)] = (unsigned short)loc;
+            }
         }
-        if (t < 3) {
-            s_qn[t] = 0;
-            s_pend[t] = 0;
-        }
+        if (t < 3) s_qn[t] = 0;
         __syncthreads();
         // row words and the first queue: rows decided by staging (a lower root below the window,
         // outside the phase, or no lower conflict in the window)
@@ -323,31 +351,25 @@ __global__ __launch_bounds__(FRONT_THREADS) void k_front(int n, int mode, const 
             bool want = false;
             unsigned short item = 0;
             if (loc < wn) {
-                s_word[loc] = ((unsigned)ubeg[k] << 16) | own[k];
-                if (own[k] & W_FLAG) {
-                    want = true;
-                    item = (unsigned short)loc;
-                } else if (!(own[k] & W_LONG) && (own[k] & 0xffu) == 0) {
-                    want = true;
-                    item = (unsigned short)(loc | 0x8000);
-                }
+                const bool not_root = (own[k] & W_ROOTS) != 0;
+                want = (not_root || (own[k] & W_COUNT) == 0) && upper[k];   // no upper rows: nothing to update
+                item = (unsigned short)(not_root ? loc : (loc | 0x8000));
+                s_word[loc] = (ubeg[k] << 16) | own[k];
             }
             wave_append(want, item, s_q[0], &s_qn[0]);
         }
-        if (t == 0) s_word[wn] = (unsigned)run << 16;
+        if (t == 0) s_word[wn] <<= 16;
         __syncthreads();
         // rounds: queued rows publish their decision and update their upper rows; long rows walk
+        int qword = s_qn[0];
         for (int r = 0;; ++r) {
-            const int cur = r % 3, nxt = (r + 1) % 3;
-            const int qn = s_qn[cur];
-            if (t == 0) {
-                s_qn[(r + 2) % 3] = 0;
-                s_pend[(r + 2) % 3] = 0;
-            }
+            const int nxt = (r + 1) % 3;
             const unsigned short* q = s_q[r & 1];
             unsigned short* qo = s_q[(r + 1) & 1];
-            for (int base = 0; base < qn; base += FRONT_THREADS / 8) {
-                const int qi = base + t / 8, sub = t & 7;
+            const int qn = qword & Q_LEN;
+            if (t == 0) s_qn[(r + 2) % 3] = 0;
+            for (int base = wave_item; base < qn; base += FRONT_THREADS / ROUND_LANES) {
+                const int qi = base + lane / ROUND_LANES, sub = lane & (ROUND_LANES - 1);
                 int e = 0, e1 = 0;
                 bool root = false;
                 if (qi < qn) {
@@ -356,32 +378,46 @@ __global__ __launch_bounds__(FRONT_THREADS) void k_front(int n, int mode, const 
                     root = (item >> 15) != 0;
                     e = (int)(s_word[loc] >> 16) + sub;
                     e1 = (int)(s_word[loc + 1] >> 16);
-                    if (sub == 0) {
-                        state[lo + loc] = root ? 1 : 2;
-                        atomicOr(&s_word[loc], root ? W_ROOT : W_NOT);
-                    }
                 }
-                for (;; e += 8) {
-                    const bool act = e < e1;
-                    if (!__any(act)) break;
-                    bool want = false;
-                    unsigned short item = 0;
-                    if (act) {
-                        const int up = s_up[e];
-                        if (root) {
-                            want = !(atomicOr(&s_word[up], W_FLAG) & W_FLAG);
-                            item = (unsigned short)up;
-                        } else {
-                            const unsigned old = atomicSub(&s_word[up], 1u);
-                            want = (old & 0xffu) == 1 && !(old & W_FLAG);
-                            item = (unsigned short)(up | 0x8000);
-                        }
+                const unsigned delta = root ? W_ROOT_SEEN : ~0u;
+                for (; __any(e < e1); e += ROUND_LANES * ROUND_ENTRIES) {
+                    // lanes without an entry add 0 to a word of their own: no branches in the chain
+                    int up[ROUND_ENTRIES];
+                    unsigned old[ROUND_ENTRIES];
+#pragma unroll
+                    for (int u = 0; u < ROUND_ENTRIES; ++u)
+                        up[u] = s_up[min(e + ROUND_LANES * u, FRONT_LIST - 1)];
+#pragma unroll
+                    for (int u = 0; u < ROUND_ENTRIES; ++u) {
+                        const bool act = e + ROUND_LANES * u < e1;
+                        old[u] = atomicAdd(&s_word[act ? up[u] : lane], act ? delta : 0u);
                     }
-                    wave_append(want, item, qo, &s_qn[nxt]);
+                    // rows this update decided: a first root seen, or the last conflict gone without one
+                    unsigned long long want[ROUND_ENTRIES];
+                    bool mine[ROUND_ENTRIES];
+                    int total = 0;
+#pragma unroll
+                    for (int u = 0; u < ROUND_ENTRIES; ++u) {
+                        const unsigned seen = root ? old[u] & W_ROOTS : (old[u] & (W_ROOTS | W_COUNT)) ^ 1u;
+                        mine[u] = (seen == 0) & (e + ROUND_LANES * u < e1);
+                        want[u] = __ballot(mine[u]);
+                        total += __popcll(want[u]);
+                    }
+                    if (total == 0) continue;
+                    int b = 0;
+                    if (lane == 0) b = atomicAdd(&s_qn[nxt], total);
+                    b = __builtin_amdgcn_readfirstlane(b) & Q_LEN;
+#pragma unroll
+                    for (int u = 0; u < ROUND_ENTRIES; ++u) {
+                        const int at = __builtin_amdgcn_mbcnt_hi((unsigned)(want[u] >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)want[u], 0));
+                        if (mine[u]) qo[b + at] = (unsigned short)(root ? up[u] : (up[u] | 0x8000));
+                        b += __popcll(want[u]);
+                    }
                 }
             }
             // rows with long lists: a lower root decides "not a root", all lower rows decided "root"
-            int pending = 0;
+            bool pending = false;
             if (longs) {
 #pragma unroll
                 for (int k = 0; k < FRONT_ROWS; ++k) {
@@ -389,9 +425,15 @@ __global__ __launch_bounds__(FRONT_THREADS) void k_front(int n, int mode, const 
                     const int loc = t + k * FRONT_THREADS, i = lo + loc;
                     bool lower_root = false, undecided = false;
                     auto see = [&](int x) {
-                        const unsigned sx = x < lo ? (unsigned)state[x] << 10 : (s_word[x - lo] & W_DONE);
-                        if (sx == W_ROOT) lower_root = true;
-                        else if (sx == 0) undecided = true;
+                        if (x < lo) {
+                            lower_root |= state[x] == 1;
+                        } else {
+                            const unsigned wx = s_word[x - lo];
+                            if (!(wx & W_ROOTS)) {
+                                if (wx & W_COUNT) undecided = true;
+                                else lower_root = true;
+                            }
+                        }
                     };
                     for (int a = t_rp[i]; a < t_rp[i + 1] && !lower_root; ++a) {
                         const int x = t_ci[a];
@@ -410,18 +452,24 @@ __global__ __launch_bounds__(FRONT_THREADS) void k_front(int n, int mode, const 
                         }
                     if (lower_root || !undecided) {
                         longs &= ~(1u << k);
-                        qo[atomicAdd(&s_qn[nxt], 1)] = (unsigned short)(lower_root ? loc : (loc | 0x8000));
+                        if (lower_root) atomicAdd(&s_word[loc], W_ROOT_SEEN);
+                        else atomicAnd(&s_word[loc], ~W_COUNT);
+                        qo[atomicAdd(&s_qn[nxt], 1) & Q_LEN] = (unsigned short)(lower_root ? loc : (loc | 0x8000));
                     } else {
-                        ++pending;
+                        pending = true;
                     }
                 }
             }
-#pragma unroll
-            for (int o = WAVE / 2; o > 0; o >>= 1) pending += __shfl_xor(pending, o, WAVE);
-            if ((t & (WAVE - 1)) == 0 && pending) atomicAdd(&s_pend[nxt], pending);
+            if (__any(pending) && lane == 0) atomicOr(&s_qn[nxt], Q_PENDING);
             __syncthreads();
             ++rounds;
-            if (s_qn[nxt] == 0 && s_pend[nxt] == 0) break;
+            qword = s_qn[nxt];
+            if (qword == 0) break;
+        }
+#pragma unroll
+        for (int k = 0; k < FRONT_ROWS; ++k) {
+            const int loc = t + k * FRONT_THREADS;
+            if (loc < wn) state[lo + loc] = s_word[loc] & W_ROOTS ? 2 : 1;
         }
         __syncthreads();   // LDS reused by the next window, whose staging reads these states
         lo = hi;

@@ -5,7 +5,7 @@
 // block reductions or other summation orders must match to the stated relative tolerance.
 //
 //   parity <case> [level]    case: momentum pressure correction forces indicator mms oss ilu
-//                                  spmv amg sell coupled runs inverse ilutail pcg bicgstab jacobi mixed topology outlet nvb remap reproject
+//                                  spmv amg sell coupled aggregate runs inverse ilutail pcg bicgstab jacobi mixed topology outlet nvb remap reproject
 //                                  all
 //
 // Prints one line per compared quantity and exits 0 when every comparison passes.
@@ -719,6 +719,71 @@ void case_coupled(Fixture& f) {
             if (k < 0) plain_one = down(d_z, f.n);
             else same_bits("one sweep", down(d_z, f.n), plain_one);
         }
+    }
+}
+
+// The greedy aggregation on random graphs (not symmetric, with isolated rows, every 512th row with 200
+// entries so that conflict lists run over their slots) against the row-order loop, whole numbers alike:
+// one row, below, at and past one window of 8192 rows, and several windows.
+void case_aggregate() {
+    std::printf("[aggregation]\n");
+    std::mt19937_64 rng(11);
+    for (int n : {1, 3, 700, 8192, 8193, 30000}) {
+        std::vector<int> rp(n + 1, 0), ci;
+        for (int i = 0; i < n; ++i) {
+            std::vector<int> row{i};
+            const int len = n > 512 && i % 512 == 77 ? 200 : (int)(rng() % 6);
+            for (int k = 0; k < len; ++k) {   // mostly near rows, as on a mesh
+                const int d = (int)(rng() % 61) - 30, j = rng() % 8 ? i + d : (int)(rng() % n);
+                if (j >= 0 && j < n) row.push_back(j);
+            }
+            std::sort(row.begin(), row.end());
+            row.erase(std::unique(row.begin(), row.end()), row.end());
+            ci.insert(ci.end(), row.begin(), row.end());
+            rp[i + 1] = (int)ci.size();
+        }
+        std::vector<int> a1(n, -1), agg;
+        int count = 0;
+        for (int i = 0; i < n; ++i) {
+            bool free_all = a1[i] < 0;
+            for (int k = rp[i]; k < rp[i + 1]; ++k) free_all = free_all && a1[ci[k]] < 0;
+            if (!free_all) continue;
+            for (int k = rp[i]; k < rp[i + 1]; ++k) a1[ci[k]] = count;   // the row itself is in its pattern
+            ++count;
+        }
+        const int phase1 = count;
+        agg = a1;
+        for (int i = 0; i < n; ++i)
+            for (int k = rp[i]; k < rp[i + 1] && agg[i] < 0; ++k)
+                if (ci[k] != i) agg[i] = a1[ci[k]];
+        for (int i = 0; i < n; ++i) {
+            if (agg[i] >= 0) continue;
+            for (int k = rp[i]; k < rp[i + 1]; ++k)
+                if (agg[ci[k]] < 0) agg[ci[k]] = count;
+            ++count;
+        }
+        const int nnz = rp[n];
+        DevArray<int> d_rp, d_ci, d_agg, d_info;
+        DevArray<double> d_v, d_dinv, d_p0;
+        DevArray<char> ws;
+        d_rp.upload(rp);
+        d_ci.upload(ci);
+        d_v.upload(Vec(nnz, 1.0));
+        d_dinv.upload(Vec(n, 1.0));
+        d_agg.reserve(n);
+        d_p0.reserve(n);
+        d_info.reserve(4);
+        const size_t bytes = cfa_amg_aggregate_ws_bytes(n, nnz);
+        ws.reserve(bytes);
+        GPU_CHECK(cfa_amg_aggregate(n, nnz, d_rp, d_ci, d_v, d_dinv, 0.08, ws, bytes, d_agg, d_p0, d_info,
+                                    solver_stream()));
+        std::vector<int> got(n), info(4);
+        GPU_CHECK(cfa_device_sync());
+        d_agg.download(got.data(), n);
+        d_info.download(info.data(), 4);
+        std::printf("  %d rows, %d entries: %d aggregates (%d of phase 1), %d rounds\n", n, nnz, info[0], info[1],
+                    info[3]);
+        expect(got == agg && info[0] == count && info[1] == phase1, "aggregates of the row-order loop");
     }
 }
 
@@ -1756,6 +1821,7 @@ int main(int argc, char** argv) {
         if (all || what == "amg") case_amg(f);
         if (all || what == "sell") case_sell(f);
         if (all || what == "coupled") case_coupled(f);
+        if (all || what == "aggregate") case_aggregate();
         if (all || what == "runs") case_runs();
         if (all || what == "inverse") case_inverse();
         if (all || what == "ilutail") case_ilu_tail();
