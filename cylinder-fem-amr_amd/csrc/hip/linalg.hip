@@ -741,33 +741,54 @@ k_jacobi_from_zero_check(int rows, const int* __restrict__ rp, const int* __rest
     y[row] = x0 + omega * dinv[row] * (b[row] - s);
 }
 
-// Last V-cycle sweep on level 0: y = x + omega dinv (b - A x) written as FP64 (the
-// preconditioned residual z), with the r.z block partials when part is set (rdot = the FP64
-// residual r; b itself in the FP64 cycle). Grid-stride, capped grid.
-template <int TPR, typename T = double>
+// Last V-cycle sweep on a level 0 without coupled transfers: y = x + omega dinv (b - A x) written as
+// FP64 (the preconditioned residual z), with the r.z block partials when part is set (rdot = the FP64
+// residual r; b itself in the FP64 cycle). Row runs through LDS; the grid is capped, so that the
+// consumers' re-summation stays short. On 1.84 M rows 59 us, bound by its 215 MB; with lanes per row, whose
+// loads scatter over the rows of a wavefront, 68 us.
+template <int RB, typename T = double>
 __global__ void __launch_bounds__(BLOCK)
 k_jacobi_dot(int rows, const int* __restrict__ rp, const int* __restrict__ ci, const T* __restrict__ val,
              const T* __restrict__ x, const T* __restrict__ b, const T* __restrict__ dinv, T omega,
              double* __restrict__ y, const double* __restrict__ rdot, double* __restrict__ part,
              const int* __restrict__ st) {
+    constexpr int U = RB / 32, CAP = U * BLOCK;
+    __shared__ T prod[CAP];
     __shared__ double lds[BLOCK / WAVE];
     if (halted(st)) return;   // nothing writes the state while this kernel runs
-    const int groups = gridDim.x * (blockDim.x / TPR);
-    const int lane = threadIdx.x % TPR;
+    const int tid = threadIdx.x;
     double contrib = 0.0;
-    for (int row = (blockIdx.x * blockDim.x + threadIdx.x) / TPR; row < rows; row += groups) {
+    for (int r0 = blockIdx.x * RB; r0 < rows; r0 += gridDim.x * RB) {
+        const int row = r0 + tid, e0 = rp[r0], e1 = rp[min(r0 + RB, rows)];
+        const bool own = tid < RB && row < rows;
+        const int k0 = own ? rp[row] : 0, k1 = own ? rp[row + 1] : 0;
+        const T xi = own ? x[row] : T(0), bi = own ? b[row] : T(0), di = own ? dinv[row] : T(0);
+        const double ri = own && part ? rdot[row] : 0.0;
         T s = 0;
-        row_entries<TPR>(ci, val, rp[row], rp[row + 1], lane, [&](T a, int j) { s += a * x[j]; });
-        s = group_sum<TPR>(s);
-        if (lane == 0) {
-            const double yi = (double)(x[row] + omega * dinv[row] * (b[row] - s));
+        for (int t = e0; t < e1; t += CAP) {
+            int c[U];
+            T v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = t + u * BLOCK + tid;
+                c[u] = k < e1 ? ci[k] : 0;
+                v[u] = k < e1 ? val[k] : T(0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) prod[u * BLOCK + tid] = v[u] * x[c[u]];
+            __syncthreads();
+            for (int k = max(k0, t), end = min(k1, t + CAP); k < end; ++k) s += prod[k - t];
+            __syncthreads();
+        }
+        if (own) {
+            const double yi = (double)(xi + omega * di * (bi - s));
             y[row] = yi;
-            if (part) contrib += rdot[row] * yi;
+            contrib += ri * yi;
         }
     }
     if (part) {
         contrib = block_sum(contrib, lds);
-        if (threadIdx.x == 0) part[blockIdx.x] = contrib;
+        if (tid == 0) part[blockIdx.x] = contrib;
     }
 }
 
@@ -2086,18 +2107,30 @@ struct PrecHooks {
     int h = 0, nb_pq = 0;
 };
 
+// Rows per workgroup of the operator kernels and their workgroups (at most RED_BLOCKS, so that the
+// consumers re-sum at most that many partials; 1536 and 2048 ran the same). 64 rows split a small mesh
+// over the CUs; 128 leave room for six workgroups' LDS on a CU. Stage 1 with 64 / 128 / 256 rows:
+// 6.0 / 6.3 / 8.9 us on 29k nodes; 64 / 128 rows: 11.3 / 11.2 us on 115k, 118 / 107 us on 1.84 M.
+int run_rows(int n) {
+    return n <= 64 * RED_BLOCKS ? 64 : 128;
+}
+int run_blocks(int n) { return std::min(blocks_for(n, run_rows(n)), RED_BLOCKS); }
+template <typename F>
+void run_dispatch(int n, F f) {
+    if (run_rows(n) == 64) f(std::integral_constant<int, 64>{});
+    else f(std::integral_constant<int, 128>{});
+}
+
 // last level-0 sweep into the FP64 output, with the r.z partials when part is set; returns the
 // number of partials
 template <typename T = double>
-int jacobi_dot_launch(int tpr, int rows, const int* rp, const int* ci, const T* val, const T* x, const T* b,
-                      const T* dinv, double omega, double* y, const double* rdot, double* part, const int* st,
-                      hipStream_t s) {
-    int nb = 0;
-    tpr_dispatch(tpr, [&](auto c) {
-        constexpr int TPR = decltype(c)::value;
-        nb = std::min(blocks_for((long long)rows * TPR), RED_BLOCKS);
-        hipLaunchKernelGGL((k_jacobi_dot<TPR, T>), dim3(nb), dim3(BLOCK), 0, s, rows, rp, ci, val, x, b, dinv,
-                           (T)omega, y, rdot, part, st);
+int jacobi_dot_launch(int rows, const int* rp, const int* ci, const T* val, const T* x, const T* b, const T* dinv,
+                      double omega, double* y, const double* rdot, double* part, const int* st, hipStream_t s) {
+    const int nb = run_blocks(rows);
+    run_dispatch(rows, [&](auto rb) {
+        constexpr int RB = decltype(rb)::value;
+        hipLaunchKernelGGL((k_jacobi_dot<RB, T>), dim3(nb), dim3(BLOCK), 0, s, rows, rp, ci, val, x, b, dinv, (T)omega,
+                           y, rdot, part, st);
     });
     return nb;
 }
@@ -2436,7 +2469,7 @@ T* vcycle(const cfa_amg_t* amg, int l, const T* b, double* out, const double* rd
     for (int k = 0; k < ss; ++k) {
         if (out && k == ss - 1) {
             // on the CSR rows: its r.z block partials keep their grouping by rows
-            const int nb = jacobi_dot_launch<T>(L.tpr_a, n, L.a_rp, L.a_ci, Lv<T>::a(L), xa, b, dv, L.omega, out,
+            const int nb = jacobi_dot_launch<T>(n, L.a_rp, L.a_ci, Lv<T>::a(L), xa, b, dv, L.omega, out,
                                                 rdot, hk ? hk->dot_part : nullptr, st, s);
             if (hk && hk->dot_part) hk->dot_blocks = nb;
             return nullptr;   // the result is in out
@@ -2790,20 +2823,6 @@ namespace {
 // PCG with the reductions folded into the consuming kernels (k_fp_*), two iterations per
 // captured graph (the search direction and the r.z partials alternate between two buffers).
 // Same algorithm, guards and stopping rules as the reference (src/cfa/linalg.cuh:183-256).
-// Rows per workgroup of the operator kernels and their workgroups (at most RED_BLOCKS, so that the
-// consumers re-sum at most that many partials; 1536 and 2048 ran the same). 64 rows split a small mesh
-// over the CUs; 128 leave room for six workgroups' LDS on a CU. Stage 1 with 64 / 128 / 256 rows:
-// 6.0 / 6.3 / 8.9 us on 29k nodes; 64 / 128 rows: 11.3 / 11.2 us on 115k, 118 / 107 us on 1.84 M.
-int run_rows(int n) {
-    return n <= 64 * RED_BLOCKS ? 64 : 128;
-}
-int run_blocks(int n) { return std::min(blocks_for(n, run_rows(n)), RED_BLOCKS); }
-template <typename F>
-void run_dispatch(int n, F f) {
-    if (run_rows(n) == 64) f(std::integral_constant<int, 64>{});
-    else f(std::integral_constant<int, 128>{});
-}
-
 void launch_fp_operator(bool oss, hipStream_t s, const PcgArgs& a, int h) {
     run_dispatch(a.n, [&](auto rb) {
         constexpr int RB = decltype(rb)::value;
