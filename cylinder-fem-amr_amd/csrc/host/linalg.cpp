@@ -2,7 +2,7 @@
 // 1276-1431: strength |a_ij| >= theta sqrt(|a_ii a_jj|) with theta 0.08, three-phase greedy
 // aggregation in row order, tentative prolongator 1/sqrt(|aggregate|), one damped Jacobi
 // smoothing step with omega = 4 / (3 * 1.05 * rho(D^-1 A)) from 20 power iterations, Galerkin
-// R A P with R = P^T, stop at <= 300 rows, 15 levels or when P.cols >= 0.85 rows, dense Cholesky
+// R A P with R = P^T, stop at <= 300 rows, 15 levels or when P.cols >= 0.85 rows, dense
 // inverse of the coarsest operator) is sequenced here level by level over the device kernels of
 // amg_setup.hip and aggregate.hip; the host, for remap(), fills the prolongator rows of new nodes
 // layer by layer.

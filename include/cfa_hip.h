@@ -339,7 +339,8 @@ typedef void (*cfa_op_cb)(const double* in, double* out, void* ctx);
 /* Krylov workspace: device vectors of capacity >= n (x 2 for the two-component solver),
  * device scalars, and a pinned status word the kernels update so the host can follow the
  * iteration without a synchronisation per dot product. Layout sizes: vec[12] vectors of
- * 2 * cap doubles, part: 8 * 4096 doubles, scal: 64 doubles, status: 16 ints (host, mapped).
+ * 2 * cap doubles, part: 8 * 4096 doubles, scal: 64 doubles, status: 16 ints (host, mapped;
+ * status_dev may be NULL: the host then waits for the stream instead of following the word).
  * internal: NULL initially; the library keeps its captured iteration graphs there (released by
  * cfa_krylov_ws_release). use_graphs: replay each iteration as a captured HIP graph (set to 0
  * to launch the kernels one by one; solves with host callbacks never use graphs). */
