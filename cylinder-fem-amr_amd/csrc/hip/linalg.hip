@@ -942,7 +942,7 @@ struct CoupledStage {
     RowSet<T, B> mul;      // y = v b, or the dense product
     RowSet<T, B2> step;    // y = x + omega dinv (b - A x)
     const double* dense;   // mul is this dense matrix (rows x rows) times x
-    int sell;              // which of the two level-0 slots runs on the sliced-ELL copy: 0 zero, 2 step
+    int sell;              // which row set runs on the stage's sliced-ELL copy: 0 zero, 2 step, -1 none
     const int* s_sp; const int* s_row; const int* s_ci; const T* s_v;
     const double* prr; int nb_rr; double* sc; int* st; int* status;   // the residual test (prr set)
 };
@@ -970,7 +970,7 @@ __device__ __forceinline__ T lanes_row_sum(const int* __restrict__ ci, const T* 
     return s;
 }
 
-// MAXL, G: the sliced-ELL copy of level 0 (MAXL 0: none in this stage). Every value is computed
+// MAXL, G: the stage's sliced-ELL copy (MAXL 0: none in this stage). Every value is computed
 // before the residual test's barrier, so the test's reduction runs beside the row loads.
 template <int MAXL, int G, typename T, typename B, typename B2>
 __global__ void __launch_bounds__(BLOCK)
@@ -2317,7 +2317,8 @@ void coupled_stage(const cfa_amg_t* amg, int l0, int l, const B0* b0, const int*
         const int sh = log2_of(L.tpr_a), shq = log2_of(L.tpr_q);
         a.zero = {row_blocks(L.rows, sh), L.rows, sh, L.a_rp, L.a_ci, Lv<T>::a(L), nullptr, b, Lv<T>::dinv(L),
                   (T)L.omega, Lv<T>::x(L)};
-        if (L.s_sp) a.zero.blocks = use_sell(L, 0);
+        // one copy per stage: the finer level's, when both have one (the CSR rows give the same bits)
+        if (L.s_sp && !(l > l0 && amg->levels[l - 1].s_sp)) a.zero.blocks = use_sell(L, 0);
         T* cb = l + 1 < bottom ? Lv<T>::b(amg->levels[l + 1]) : bottom_of<T>(amg).b;
         a.mul = {row_blocks(L.cols, shq), L.cols, shq, L.q_rp, L.q_ci, Lv<T>::q(L), nullptr, b, nullptr, T(0), cb};
     }

@@ -5,7 +5,7 @@
 // block reductions or other summation orders must match to the stated relative tolerance.
 //
 //   parity <case> [level]    case: momentum pressure correction forces indicator mms oss ilu
-//                                  spmv amg sell coupled aggregate runs inverse ilutail pcg bicgstab jacobi mixed topology outlet nvb remap reproject
+//                                  spmv amg sell coupled copies aggregate runs inverse ilutail pcg bicgstab jacobi mixed topology outlet nvb remap reproject
 //                                  all
 //
 // Prints one line per compared quantity and exits 0 when every comparison passes.
@@ -720,6 +720,105 @@ void case_coupled(Fixture& f) {
             else same_bits("one sweep", down(d_z, f.n), plain_one);
         }
     }
+}
+
+// Sliced-ELL copies on every level of a caller's hierarchy (the set-up builds one on level 0 only; the
+// descriptor allows one per level), against the same hierarchy with the CSR rows, or with a copy on level 0
+// only: a copy keeps the CSR kernels' sums, so the V-cycle, coupled from level 0, from level 1 and not
+// coupled, FP64 and FP32, and a PCG solve are the same bit for bit. A chain of 3000 rows: three levels of at
+// most five entries per row. Another right-hand side runs in between, so that a row that is not written shows.
+void case_copies() {
+    std::printf("[sliced-ELL copies on several levels]\n");
+    const int n = 3000;
+    std::vector<int> rp(1, 0), ci;
+    Vec val, r(n), other(n);
+    for (int i = 0; i < n; ++i) {
+        for (int j = std::max(i - 1, 0); j <= std::min(i + 1, n - 1); ++j) {
+            ci.push_back(j);
+            val.push_back(j == i ? 2.01 : -1.0);
+        }
+        rp.push_back((int)ci.size());
+    }
+    std::mt19937_64 rng(3);
+    for (Vec* v : {&r, &other})
+        for (double& e : *v) e = std::uniform_real_distribution<double>(-1, 1)(rng);
+    DevArray<int> d_rp, d_ci, d_info;
+    DevArray<double> d_val, d_r, d_other, d_z;
+    d_rp.upload(rp);
+    d_ci.upload(ci);
+    d_val.upload(val);
+    d_r.upload(r);
+    d_other.upload(other);
+    d_z.reserve(n);
+    d_info.reserve(2);
+    AmgPreconditioner amg;
+    amg.fp32 = true;
+    amg.dense_max_rows = 0;
+    amg.setup(n, (int)ci.size(), d_rp, d_ci, d_val);
+    const int nl = amg.view()->n_levels;
+    expect(nl == 3, "three smoothed levels");
+    std::vector<cfa_amg_level_t> csr(amg.view()->levels, amg.view()->levels + nl);
+    for (auto& L : csr) L.s_sp = nullptr;
+    std::vector<cfa_amg_level_t> ell = csr;
+    std::vector<DevArray<int>> s_row(nl), s_sp(nl), s_ci(nl);
+    std::vector<DevArray<double>> s_v(nl);
+    std::vector<DevArray<float>> s_v32(nl);
+    for (int l = 0; l < nl; ++l) {
+        cfa_amg_level_t& L = ell[l];
+        const int slices = (L.rows + 63) / 64;
+        s_row[l].reserve(64 * (size_t)slices);
+        s_sp[l].reserve(slices + 1);
+        DevArray<char> ws;
+        const size_t bytes = cfa_sell_ws_bytes(L.rows);
+        ws.reserve(bytes);
+        GPU_CHECK(cfa_sell_plan(L.rows, L.a_rp, s_row[l], s_sp[l], d_info, ws, bytes, solver_stream()));
+        int info[2];
+        d_info.download(info, 2);
+        s_ci[l].reserve(info[0]);
+        s_v[l].reserve(info[0]);
+        s_v32[l].reserve(info[0]);
+        GPU_CHECK(cfa_sell_fill(L.rows, L.a_rp, L.a_ci, L.a_v, s_row[l], s_sp[l], s_ci[l], s_v[l], solver_stream()));
+        GPU_CHECK(cfa_to_f32(info[0], s_v[l], s_v32[l], solver_stream()));
+        L.s_len = info[1];
+        L.s_sp = s_sp[l]; L.s_row = s_row[l]; L.s_ci = s_ci[l]; L.s_v = s_v[l]; L.s_v32 = s_v32[l];
+    }
+    auto apply = [&](const cfa_amg_t& a) {
+        GPU_CHECK(cfa_amg_apply(&a, d_other, d_z, solver_stream()));
+        GPU_CHECK(cfa_amg_apply(&a, d_r, d_z, solver_stream()));
+        return down(d_z, n);
+    };
+    for (int lanes : {1, 2, 4})
+        for (int couple = 0; couple < 3; ++couple)   // from level 0, from level 1, none
+            for (int f32 = 0; f32 < 2; ++f32) {
+                std::vector<cfa_amg_level_t> a = csr, b = ell;
+                for (auto* lv : {&a, &b})
+                    for (int l = 0; l < nl; ++l) {
+                        (*lv)[l].tpr_a = lanes;
+                        if (l < couple || couple == 2) (*lv)[l].w_rp = nullptr;
+                    }
+                cfa_amg_t va = *amg.view(), vb = va;
+                va.use_f32 = vb.use_f32 = f32;
+                va.levels = a.data();
+                vb.levels = b.data();
+                const Vec want = apply(va);
+                std::printf("  %d lanes, %s, %s\n", lanes,
+                            couple == 0 ? "coupled" : couple == 1 ? "coupled from level 1" : "not coupled",
+                            f32 ? "FP32" : "FP64");
+                same_bits("  V-cycle", apply(vb), want);
+                if (couple) continue;
+                Vec x[2];
+                a[0] = b[0];
+                for (int k = 0; k < 2; ++k) {
+                    KrylovWorkspace kw;
+                    cfa_solve_result_t res{};
+                    dev_zero(d_z, n * sizeof(double));
+                    GPU_CHECK(cfa_pcg(n, d_rp, d_ci, d_val, d_r, d_z, 200, 1e-10, nullptr, nullptr, nullptr,
+                                      k ? &vb : &va, nullptr, nullptr, kw.get(n), &res, solver_stream()));
+                    expect(res.converged[0] == 1, "  PCG converged");
+                    x[k] = down(d_z, n);
+                }
+                same_bits("  PCG", x[1], x[0]);
+            }
 }
 
 // The greedy aggregation on random graphs (not symmetric, with isolated rows, every 512th row with 200
@@ -1821,6 +1920,7 @@ int main(int argc, char** argv) {
         if (all || what == "amg") case_amg(f);
         if (all || what == "sell") case_sell(f);
         if (all || what == "coupled") case_coupled(f);
+        if (all || what == "copies") case_copies();
         if (all || what == "aggregate") case_aggregate();
         if (all || what == "runs") case_runs();
         if (all || what == "inverse") case_inverse();

@@ -1,6 +1,7 @@
 """The coupled V-cycle through the C ABI, on the GPU (tests/native/parity.cpp):
 the cycle against the one with separate residual, restriction and prolongation (uniform levels 1, 3
-and 4: one to four smoothed levels, with the dense bottom at none, the last or the first coarse one);
+and 4: one to four smoothed levels, with the dense bottom at none, the last or the first coarse one),
+and on hierarchies with sliced-ELL copies on several levels;
 the greedy aggregation at the edges of its windows and with conflict lists past their slots;
 the pressure operator's row runs at the edges of their tiles against sums on the host; the dense
 inverse of the coarsest operator at the edges of its blocks; the ILU(0) sweeps where the trailing
@@ -24,7 +25,7 @@ def test_coupled_cycle(level):
     assert r.returncode == 0 and "ALL PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-2000:]
 
 
-@pytest.mark.parametrize("case", ["aggregate", "runs", "inverse", "ilutail"])
+@pytest.mark.parametrize("case", ["copies", "aggregate", "runs", "inverse", "ilutail"])
 def test_tile_edges(case):
     print(f"[case] {case}", flush=True)
     r = subprocess.run([str(BIN), case, "0"], capture_output=True, text=True, timeout=120)
