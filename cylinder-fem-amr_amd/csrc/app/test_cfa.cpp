@@ -610,6 +610,31 @@ void block_pool() {
     std::printf("  block pool: %d synchronisations, %d frees\n", syncs, frees);
 }
 
+// On the device: a refused allocation reports its error and leaves none behind for the next launch's check,
+// and the pool's second attempt after giving its blocks back is usable
+void refused_allocation() {
+    const size_t absurd = (size_t)1 << 60;
+    void *p = nullptr, *q = nullptr;
+    EXPECT(cfa_malloc(&p, 4096) == CFA_OK, "a small block");
+    EXPECT(cfa_malloc(&q, absurd) != CFA_OK && q == nullptr, "2^60 bytes are refused");
+    int rc = cfa_zero(p, 4096, nullptr);
+    EXPECT(rc == CFA_OK, "the next launch reports %d", rc);
+    (void)cfa_free(p);
+    int calls = 0;
+    BlockPool pool;
+    pool.alloc = [&](void** ptr, size_t bytes) { return cfa_malloc(ptr, ++calls == 2 ? absurd : bytes); };
+    pool.free = [](void* ptr) { return cfa_free(ptr); };
+    pool.sync = [] { return cfa_device_sync(); };
+    EXPECT(pool.get(&p, 4096) == 0, "a block");
+    pool.put(p);
+    EXPECT(pool.get(&q, 1 << 20) == 0 && calls == 3 && pool.kept_bytes() == 0, "refused, trimmed, given");
+    rc = cfa_zero(q, 1 << 20, nullptr);
+    EXPECT(rc == CFA_OK, "the next launch reports %d", rc);
+    EXPECT(cfa_device_sync() == CFA_OK, "synchronised");
+    pool.put(q);
+    pool.trim();
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -625,6 +650,7 @@ int main(int argc, char** argv) {
     }
     if (what != "host") {
         GPU_CHECK(cfa_init(0));
+        refused_allocation();
         random_adaptation();
         round_trip();
         min_level();

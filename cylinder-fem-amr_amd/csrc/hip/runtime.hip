@@ -16,6 +16,15 @@ __global__ void k_zero_bytes(unsigned char* __restrict__ p, size_t bytes) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < bytes; i += (size_t)gridDim.x * blockDim.x)
         p[i] = 0;
 }
+
+// Status of a call whose failure the caller may live with (the host layer's block pool gives blocks back
+// and asks again): the runtime keeps a failure as the thread's last error until it is read, and the
+// next launch's check would report it as its own.
+int own_status(hipError_t e) {
+    if (e == hipSuccess) return CFA_OK;
+    (void)hipGetLastError();
+    return (int)e;
+}
 }  // namespace
 
 extern "C" {
@@ -43,14 +52,12 @@ const char* cfa_error_string(int code) {
 int cfa_malloc(void** d_ptr, size_t bytes) {
     if (!d_ptr) return CFA_E_ARG;
     *d_ptr = nullptr;
-    const hipError_t e = hipMalloc(d_ptr, bytes > 0 ? bytes : 8);
-    return e == hipSuccess ? CFA_OK : (int)e;
+    return own_status(hipMalloc(d_ptr, bytes > 0 ? bytes : 8));
 }
 
 int cfa_free(void* d_ptr) {
     if (!d_ptr) return CFA_OK;
-    const hipError_t e = hipFree(d_ptr);
-    return e == hipSuccess ? CFA_OK : (int)e;
+    return own_status(hipFree(d_ptr));
 }
 
 int cfa_host_malloc(void** h_ptr, void** d_alias, size_t bytes) {

@@ -1,8 +1,8 @@
 """The C++ unit tests (cylinder-fem-amr_amd/csrc/app/test_cfa.cpp, the checks of the reference's
 tests/test_cfa.cu) run as one program on the GPU: the device NVB forest's adaptation checks
 (conformity, level cap, angle bound, exact transfer of linear fields, refine/coarsen round trip,
-minimum level, retransfer) and the solver checks. Its host part runs without a device: the
-sliced-ELL layout of the ILU(0) pattern's split rows."""
+minimum level, retransfer), the solver checks and a refused allocation. Its host part runs without a
+device: the sliced-ELL layout of the ILU(0) pattern's split rows and the pool of device blocks."""
 import subprocess
 
 import pytest
