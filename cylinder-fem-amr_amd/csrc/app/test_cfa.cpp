@@ -568,6 +568,25 @@ void block_pool() {
     pool.put(c);
     pool.trim();
     EXPECT(live.empty() && pool.kept_bytes() == 0, "trimmed");
+    // a failed synchronisation (as beside another thread's stream capture): a new block instead, the kept
+    // one stays until a synchronisation succeeds, or goes back when the device has no room for a new one
+    int sync_rc = 1;
+    pool.sync = [&] { ++syncs; return sync_rc; };
+    limit = 200000;
+    const int syncs0 = syncs, frees0 = frees;
+    EXPECT(pool.get(&a, 90000) == 0, "a block");
+    pool.put(a);
+    EXPECT(pool.get(&b, 90000) == 0 && b != a && syncs == syncs0 + 1 && pool.kept_bytes() > 0,
+           "not synchronised: a new block");
+    EXPECT(pool.get(&c, 90000) == 0 && c != a && c != b && pool.kept_bytes() == 0 && frees == frees0 + 1,
+           "not synchronised and no room: the kept block given back");
+    pool.put(c);
+    sync_rc = 0;
+    EXPECT(pool.get(&a, 90000) == 0 && a == c, "synchronised: reuse");
+    pool.put(a);
+    pool.put(b);
+    pool.trim();
+    EXPECT(live.empty(), "every block given back");
     limit = (size_t)-1;
     pool.bound = 1 << 20;
     std::mutex hm;

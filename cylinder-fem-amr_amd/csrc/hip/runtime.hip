@@ -18,8 +18,8 @@ __global__ void k_zero_bytes(unsigned char* __restrict__ p, size_t bytes) {
 }
 
 // Status of a call whose failure the caller may live with (the host layer's block pool gives blocks back
-// and asks again): the runtime keeps a failure as the thread's last error until it is read, and the
-// next launch's check would report it as its own.
+// and asks again, or goes without the synchronisation): the runtime keeps a failure as the thread's last
+// error until it is read, and the next launch's check would report it as its own.
 int own_status(hipError_t e) {
     if (e == hipSuccess) return CFA_OK;
     (void)hipGetLastError();
@@ -122,8 +122,7 @@ int cfa_stream_destroy(cfa_stream_t stream) {
 }
 
 int cfa_device_sync(void) {
-    const hipError_t e = hipDeviceSynchronize();
-    return e == hipSuccess ? CFA_OK : (int)e;
+    return own_status(hipDeviceSynchronize());
 }
 
 int cfa_timer_create(void** timer) {

@@ -19,11 +19,11 @@ int BlockPool::get(void** ptr, size_t bytes) {
         if (it->second.freed <= synced_) { pick = it; break; }   // idle: no wait
         if (pick == kept_.end()) pick = it;
     }
+    if (pick != kept_.end() && pick->second.freed > synced_) {
+        if (sync() == 0) synced_ = clock_++;
+        else pick = kept_.end();   // not known to be idle: it stays kept
+    }
     if (pick != kept_.end()) {
-        if (pick->second.freed > synced_) {
-            if (const int rc = sync()) return rc;
-            synced_ = clock_++;
-        }
         *ptr = pick->second.ptr;
         size_of_[*ptr] = pick->first;
         kept_bytes_ -= pick->first;

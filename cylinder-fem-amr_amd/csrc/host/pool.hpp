@@ -16,7 +16,8 @@ namespace cfa {
 // and given out again for requests they fit within 1.5 times. hipFree returns only when the device has
 // finished everything submitted before; here that wait moves to the reuse: a block given out again was
 // freed before the last full device synchronisation, or one is made first. So a block may be freed while
-// kernels of any stream still use it, as with hipFree. Safe from several threads.
+// kernels of any stream still use it, as with hipFree. When the device cannot be synchronised (another
+// thread may be capturing a stream), a new block is allocated instead. Safe from several threads.
 class BlockPool {
 public:
     std::function<int(void**, size_t)> alloc;   // 0 on success
@@ -45,7 +46,8 @@ private:
     void trim_locked();
 };
 
-// The pool of the host layer's device arrays (cfa_malloc, cfa_free, cfa_device_sync)
+// The pool of the host layer's device arrays (cfa_malloc, cfa_free, cfa_device_sync): one for the process,
+// whose host layer works on device 0 (every entry point selects it)
 BlockPool& device_pool();
 
 }  // namespace cfa
