@@ -50,12 +50,15 @@ void same_ints(const char* what, const std::vector<int>& gpu, const std::vector<
     if (bad) ++failures;
 }
 
+// the larger of two values; a NaN stays (std::max drops it)
+double larger(double m, double v) { return m >= v || std::isnan(m) ? m : v; }
+
 // max |gpu - ref| / max |ref| <= tol
 void close_rel(const char* what, const Vec& gpu, const Vec& ref, double tol) {
     double d = 0.0, s = 0.0;
     for (size_t i = 0; i < ref.size(); ++i) {
-        d = std::max(d, std::fabs(gpu[i] - ref[i]));
-        s = std::max(s, std::fabs(ref[i]));
+        d = larger(d, std::fabs(gpu[i] - ref[i]));
+        s = larger(s, std::fabs(ref[i]));
     }
     const double rel = s > 0.0 ? d / s : d;
     const bool ok = rel <= tol && std::isfinite(rel);
@@ -999,7 +1002,7 @@ void case_inverse() {
                 for (int k = rp[i]; k < rp[i + 1]; ++k)
                     for (int j = 0; j < n; ++j) row[j] += v[k] * inv[(size_t)ci[k] * n + j];
                 row[i] -= 1.0;
-                for (double e : row) worst = std::max(worst, std::fabs(e));
+                for (double e : row) worst = larger(worst, std::fabs(e));
             }
             std::printf("  n %d: max |A inv - I| %.2e\n", n, worst);
             expect(info[0] == 0.0 && worst <= (n <= 300 ? 2e-12 : 1e-11), "inverse");
