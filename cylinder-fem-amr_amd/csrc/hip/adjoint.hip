@@ -733,6 +733,7 @@ constexpr int SHAPE_WAVES = CFA_ADJ_SHAPE_WS / WAVE;
 __global__ void __launch_bounds__(BLOCK)
 k_adj_shape(int n, const double* __restrict__ x0, const double* __restrict__ y0, const double* __restrict__ xb,
             const double* __restrict__ yb, double xc, double yc, double radius, double* __restrict__ part) {
+#pragma clang fp contract(off)   // the cut-off rounds to zero where the displacement's does
     const int k = threadIdx.x % WAVE, w = (blockIdx.x * BLOCK + threadIdx.x) / WAVE;
     constexpr double pi = 3.14159265358979323846;
     const double sigma = 2.0 * pi / WAVE, outer = 3.0 * radius;
@@ -743,7 +744,8 @@ k_adj_shape(int n, const double* __restrict__ x0, const double* __restrict__ y0,
         const double t = fmin(1.0, fmax(0.0, (r - radius) / (outer - radius)));
         const double chi = 1.0 - t * t * (3.0 - 2.0 * t);
         const double d = remainder(atan2(dy, dx) - 2.0 * pi * k / WAVE, 2.0 * pi);
-        acc += radius * exp(-0.5 * (d / sigma) * (d / sigma)) * chi / r * (xb[i] * dx + yb[i] * dy);
+        const double weight = radius * exp(-0.5 * (d / sigma) * (d / sigma)) * chi / r;
+        if (weight != 0.0) acc += weight * (xb[i] * dx + yb[i] * dy);   // a node that does not move adds nothing
     }
     part[(size_t)w * WAVE + k] = acc;
 }

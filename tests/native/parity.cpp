@@ -5,7 +5,7 @@
 // block reductions or other summation orders must match to the stated relative tolerance.
 //
 //   parity <case> [level]    case: momentum pressure correction forces indicator mms oss ilu
-//                                  spmv amg sell coupled copies aggregate runs inverse ilutail pcg bicgstab jacobi mixed topology outlet nvb remap reproject
+//                                  spmv amg sell coupled copies aggregate runs inverse ilutail shape pcg bicgstab jacobi mixed topology outlet nvb remap reproject
 //                                  all
 //
 // Prints one line per compared quantity and exits 0 when every comparison passes.
@@ -1089,6 +1089,58 @@ void case_ilu_tail() {
     }
 }
 
+// The contraction of coordinate sensitivities with the 64 boundary modes against the host loop over the
+// same weights, around the number of wavefronts (1024, a node per turn each); nodes at the centre, on the
+// cylinder, past the outer radius and just inside it, where the weight can round to zero. A weight of zero
+// leaves its node out, also where the sensitivity is not finite. Tolerance: all terms are positive; a term's
+// angle carries 4e-16 of rounding, over the Gaussian's width of 0.098 at up to three widths 1e-14, and a sum
+// adds at most 1024 + n / 1024 roundings of 1e-16: 2e-13.
+void case_shape() {
+    std::printf("[contraction with the boundary modes]\n");
+    const double xc = 0.2, yc = 0.2, R = 0.05, pi = std::acos(-1.0);
+    std::mt19937_64 rng(13);
+    std::uniform_real_distribution<double> U(0.0, 1.0);
+    for (int n : {1, 64, 1023, 1024, 1025, 29152}) {
+        Vec x(n), y(n), xb(n), yb(n), ref(64, 0.0);
+        int zero = 0;
+        for (int i = 0; i < n; ++i) {
+            const double phi = 2.0 * pi * U(rng), r = i % 7 == 5 ? 3.001 * R : i % 7 == 6 ? R : R * (1.0 + 3.0 * U(rng));
+            x[i] = xc + r * std::cos(phi);
+            y[i] = yc + r * std::sin(phi);
+            if (i % 97 == 3) { x[i] = xc; y[i] = yc; }
+            if (i % 97 == 4) { x[i] = xc + 3.0 * R * (1.0 - 1e-9 * (1 + i % 5)); y[i] = yc; }
+            const double dx = x[i] - xc, dy = y[i] - yc, u = 0.5 + 0.5 * U(rng);
+            xb[i] = u * dx;
+            yb[i] = u * dy;
+            bool any = false;
+            for (int k = 0; k < 64; ++k) {
+                const double rr = std::hypot(dx, dy);
+                if (rr >= 3.0 * R || rr <= 0.0) continue;
+                const double t = std::min(1.0, std::max(0.0, (rr - R) / (3.0 * R - R)));
+                const double chi = 1.0 - t * t * (3.0 - 2.0 * t);
+                const double d = std::remainder(std::atan2(dy, dx) - 2.0 * pi * k / 64, 2.0 * pi) / (2.0 * pi / 64);
+                const double w = R * std::exp(-0.5 * d * d) * chi / rr;
+                any = any || w != 0.0;
+                ref[k] += w * (xb[i] * dx + yb[i] * dy);
+            }
+            if (!any) {
+                xb[i] = i % 2 ? INFINITY : NAN;
+                ++zero;
+            }
+        }
+        DevArray<double> d_x, d_y, d_xb, d_yb, d_ws, d_out;
+        d_x.upload(x);
+        d_y.upload(y);
+        d_xb.upload(xb);
+        d_yb.upload(yb);
+        d_ws.reserve(CFA_ADJ_SHAPE_WS);
+        d_out.reserve(64);
+        GPU_CHECK(cfa_adj_shape_modes(n, d_x, d_y, d_xb, d_yb, xc, yc, R, d_ws, d_out, solver_stream()));
+        std::printf("  n %d, %d nodes of weight zero\n", n, zero);
+        close_rel("  mode sums", down(d_out, 64), ref, 2e-13);
+    }
+}
+
 // The scheme-consistent re-projection after a remesh with its two solves (u^{n-1} and u^n) side by
 // side on two streams against the same two solves one after the other, from the same state: the
 // velocities, the vorticity and the last increment bit for bit.
@@ -1928,6 +1980,7 @@ int main(int argc, char** argv) {
         if (all || what == "runs") case_runs();
         if (all || what == "inverse") case_inverse();
         if (all || what == "ilutail") case_ilu_tail();
+        if (all || what == "shape") case_shape();
         if (all || what == "pcg") case_pcg(f);
         if (all || what == "bicgstab") case_bicgstab(f);
         if (all || what == "jacobi") case_jacobi(f);

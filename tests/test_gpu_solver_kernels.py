@@ -5,8 +5,9 @@ and on hierarchies with sliced-ELL copies on several levels;
 the greedy aggregation at the edges of its windows and with conflict lists past their slots;
 the pressure operator's row runs at the edges of their tiles against sums on the host; the dense
 inverse of the coarsest operator at the edges of its blocks; the ILU(0) sweeps where the trailing
-colours change path; and pressure solves in FP64 and with the FP32 cycle against the oracle's on both
-sides of 65,536 rows, up to where the PCG update runs in the cycle's first launch."""
+colours change path; the contraction of the shape gradient with the boundary modes against the host
+loop; and pressure solves in FP64 and with the FP32 cycle against the oracle's on both sides of 65,536
+rows, up to where the PCG update runs in the cycle's first launch."""
 import subprocess
 from pathlib import Path
 
@@ -25,7 +26,7 @@ def test_coupled_cycle(level):
     assert r.returncode == 0 and "ALL PASSED" in r.stdout, r.stdout[-3000:] + r.stderr[-2000:]
 
 
-@pytest.mark.parametrize("case", ["copies", "aggregate", "runs", "inverse", "ilutail"])
+@pytest.mark.parametrize("case", ["copies", "aggregate", "runs", "inverse", "ilutail", "shape"])
 def test_tile_edges(case):
     print(f"[case] {case}", flush=True)
     r = subprocess.run([str(BIN), case, "0"], capture_output=True, text=True, timeout=120)
