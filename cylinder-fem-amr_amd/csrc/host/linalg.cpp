@@ -987,6 +987,40 @@ void AmgPreconditioner::apply(const double* d_r, double* d_z) {
     GPU_CHECK(cfa_amg_apply(&view_, d_r, d_z, solver_stream()));
 }
 
+double AmgPreconditioner::cycle_bytes() const {
+    const double vb = fp32 && !levels.empty() ? 4.0 : 8.0;   // values and vectors of the cycle
+    auto matrix = [&](double rows, double nnz) { return (4.0 + vb) * nnz + 4.0 * (rows + 1.0); };
+    const bool dense = has_dense_ && smooth_steps == 2;
+    const size_t bottom = dense ? (size_t)dense_level_ : levels.size();
+    size_t coupled = bottom;   // first level from which all are coupled
+    if (smooth_steps == 2)
+        while (coupled > 0 && levels[coupled - 1]->has_coupling) --coupled;
+    const double m = dense ? levels[bottom]->A.rows : coarse_n;
+    double b = 8.0 * m * m + 2.0 * vb * m;
+    for (size_t l = 0; l < bottom; ++l) {
+        const Level& L = *levels[l];
+        const double n = L.A.rows, c = L.R.rows, A = matrix(n, L.A.nnz), v = vb * n;
+        // level 0 writes z in FP64; its right-hand side is the FP64 r, in the FP32 cycle of a separate
+        // level 0 a copy of it
+        if (l == 0) b += (8.0 - vb) * n;
+        if (l >= coupled) {
+            const double r = l == 0 ? 8.0 * n : v;   // right-hand side
+            b += A + r + 2.0 * v;                                    // two steps from zero
+            b += matrix(c, L.Q.nnz) + r + vb * c;                    // coarse right-hand side
+            b += A + r + 3.0 * v;                                    // first step
+            b += A + matrix(n, L.W.nnz) + r + 3.0 * v + vb * c;      // second step and correction
+            continue;
+        }
+        if (l == 0 && fp32) b += 12.0 * n;
+        const int sweeps = std::max(2 * smooth_steps - 2, smooth_steps);   // on an iterate
+        b += (smooth_steps >= 2 ? A : 0.0) + 3.0 * v + sweeps * (A + 4.0 * v);
+        b += A + 3.0 * v;                                            // residual
+        b += matrix(c, L.R.nnz) + v + vb * c;                        // restriction
+        b += matrix(n, L.P.nnz) + 2.0 * v + vb * c;                  // correction
+    }
+    return b;
+}
+
 // Carries the level-0 prolongator to a new mesh (src/cfa/linalg.cuh:1074-1157): kept nodes keep
 // their row, a new node gets the mean of the rows of its already-set graph neighbours, pass by
 // pass; coarser levels, omega and the coarse inverse stay.

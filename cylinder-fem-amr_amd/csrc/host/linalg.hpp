@@ -222,6 +222,9 @@ public:
     // A view of the current hierarchy with a second set of work vectors, for a V-cycle running on
     // another stream at the same time as one through view(); valid until the next set-up or remap.
     const cfa_amg_t* second_view();
+    // Algorithmic bytes of one apply(): every array once per launch that reads or writes it (matrices as CSR
+    // rows), for the launches the hierarchy's form runs: coupled levels, the dense bottom, separate levels
+    double cycle_bytes() const;
 
 private:
     // the set-up's second stream: each level's power iteration runs on it beside the aggregation

@@ -93,18 +93,6 @@ double rel_max_diff(const std::vector<double>& a, const std::vector<double>& b) 
     return m > 0.0 ? d / m : d;
 }
 
-// Algorithmic bytes of one V(2,2) cycle: per level three smoother-class passes over A, the
-// residual, restriction and prolongation, plus the dense coarse solve (FP64 values and vectors).
-double vcycle_bytes(const AmgPreconditioner& amg) {
-    double b = 8.0 * amg.coarse_n * (double)amg.coarse_n;
-    for (const auto& L : amg.levels) {
-        const double n = L->A.rows, a = L->A.nnz;
-        b += 3.0 * (12.0 * a + 44.0 * n) + (12.0 * a + 36.0 * n) + (12.0 * L->R.nnz + 28.0 * n) +
-             (12.0 * L->P.nnz + 36.0 * n);
-    }
-    return b;
-}
-
 double synced_ms(Clock::time_point t0) {
     dev_sync();
     return ms_since(t0);
@@ -223,7 +211,7 @@ int cfa_dumped_pressure_solve(const char* path, double tol, int max_iter, int pr
         kernel_timings().push_back({"cfa_spmv, 1 right-hand side", 12.0 * dnnz + 20.0 * dn + 4.0, time_launches(kernel_reps, [&] {
             GPU_CHECK(cfa_spmv(n, rp, ci, val, xd, t_out, 1, solver_stream()));
         }), kernel_reps});
-        kernel_timings().push_back({"V-cycle", vcycle_bytes(amg), time_launches(kernel_reps, [&] { amg.apply(b, t_out); }),
+        kernel_timings().push_back({"V-cycle", amg.cycle_bytes(), time_launches(kernel_reps, [&] { amg.apply(b, t_out); }),
                                     kernel_reps});
     }
     const double v[8] = {(double)n, (double)nnz, (double)amg.num_levels(), setup_ms, solve_ms, (double)iters,

@@ -673,6 +673,36 @@ void case_sell(Fixture& f) {
     }
 }
 
+// Bytes of a V(2,2) cycle from its launches as the descriptor decides them, in FP64: the sizes of the
+// CSR arrays and vectors that each reads and writes.
+double launch_bytes(const cfa_amg_t& a) {
+    auto csr = [](const int* rp, int rows) {
+        int nnz = 0;
+        GPU_CHECK(cfa_memcpy(&nnz, rp + rows, sizeof(int), 1, solver_stream()));
+        return 12.0 * nnz + 4.0 * (rows + 1);
+    };
+    double b = 0.0;
+    const int bottom = a.dense ? a.dense_level : a.n_levels;
+    int from = bottom;
+    while (from > 0 && a.levels[from - 1].w_rp) --from;
+    for (int l = 0; l < bottom; ++l) {
+        const cfa_amg_level_t& L = a.levels[l];
+        const double A = csr(L.a_rp, L.rows), n = 8.0 * L.rows, c = 8.0 * L.cols;
+        b += A + 3 * n;                                                   // b, dinv -> x
+        if (l >= from) {
+            b += csr(L.q_rp, L.cols) + n + c;                             // b -> coarse b
+            b += A + 4 * n;                                               // x, b, dinv -> ax
+            b += A + csr(L.w_rp, L.rows) + 4 * n + c;                     // ax, b, dinv, coarse x -> x
+        } else {
+            b += A + 3 * n;                                               // x, b -> r
+            b += csr(L.r_rp, L.cols) + n + c + csr(L.p_rp, L.rows) + c + 2 * n;   // r -> coarse b; x += P coarse x
+            b += 2 * (A + 4 * n);                                         // x, b, dinv -> ax -> x
+        }
+    }
+    const double m = a.dense ? a.levels[bottom].rows : a.coarse_n;
+    return b + 8.0 * m * m + 16.0 * m;
+}
+
 // The coupled V(2,2) cycle (two launches per level through W = G^2 P, the small levels as one dense
 // matrix) against the cycle with separate residual, restriction and prolongation on the same
 // hierarchy: coupled from level 0, from level 1, with and without the dense matrix, FP64 and FP32.
@@ -715,6 +745,7 @@ void case_coupled(Fixture& f) {
                 expect((amg.view()->dense != nullptr) == (forms[k].dense > 0), "dense bottom");
             }
             if (f32) continue;
+            expect(std::fabs(amg.cycle_bytes() / launch_bytes(*amg.view()) - 1.0) < 1e-12, "bytes of the launches");
             // V(1,1) on the same hierarchy: the dense matrix is V(2,2)'s and stays out of it
             cfa_amg_t one = *amg.view();
             one.smooth_steps = 1;
