@@ -1667,6 +1667,18 @@ void case_pcg(Fixture& f) {
             same_bits(cb ? "solution, host callback" : "solution", x_dev[1], x_dev[0]);
             if (!cb) same_bits("solution of the solver class", x_dev[1], xs);
         }
+        if (warm) continue;
+        // the other form of level 0: coupled past the size rule, or separate below it
+        AmgPreconditioner other;
+        other.couple_max_rows = f.n <= amg.couple_max_rows ? f.n - 1 : 1 << 30;
+        other.setup(f.n, f.nnz, f.g.d_row_ptr, f.g.d_col_ind, f.g.d_Kp_val);
+        expect(other.levels[0]->has_coupling != amg.levels[0]->has_coupling, "the other form of level 0");
+        f.g.d_dp.upload(x0);
+        const int it2 = solver.solve_pcg_fused(f.n, f.g.d_row_ptr, f.g.d_col_ind, f.g.d_Kp_val, f.g.d_rhs_p, f.g.d_dp,
+                                               4000, tol, &op, &other);
+        expect(std::abs(it2 - si.iters) <= 1 && solver.converged, "iterations and convergence");
+        close_rel(other.levels[0]->has_coupling ? "solution, coupled" : "solution, separate", down(f.g.d_dp, f.n), x,
+                  1e-8);
     }
 }
 
@@ -1752,8 +1764,16 @@ void case_bicgstab(Fixture& f) {
                                 f.g.d_v, 150, 1e-10, ilu.view(), 0, ws, &res, solver_stream()));
         ws->status_dev = mapped;
         x_dev[null_dev] = down(f.g.d_u, f.n);
+        std::printf("  iterations (%d, %d), relative residuals (%.3e, %.3e), oracle (%.3e, %.3e)\n", res.iters[0],
+                    res.iters[1], res.rel_residual[0], res.rel_residual[1], bi.rel[0], bi.rel[1]);
+        // the residual is that of the last full iteration: above the tolerance when a half step ended the
+        // solve, so it is held to the oracle's. Rounding of 1e-16 in a residual of 1e-10 is 1e-6 of it; three
+        // decades more for its growth over the iterations.
+        bool same_rel = true;
+        for (int c = 0; c < 2; ++c)
+            if (res.iters[c] == bi.iters[c]) same_rel = same_rel && std::fabs(res.rel_residual[c] / bi.rel[c] - 1.0) < 1e-3;
         expect(std::abs(res.iters[0] - bi.iters[0]) <= 1 && std::abs(res.iters[1] - bi.iters[1]) <= 1 &&
-                   res.converged[0] == 1 && res.converged[1] == 1 && res.rel_residual[1] < 1e-10,
+                   res.converged[0] == 1 && res.converged[1] == 1 && same_rel,
                null_dev ? "outcome without mapped status words" : "outcome through mapped status words");
     }
     same_bits("u", x_dev[1], x_dev[0]);
