@@ -26,7 +26,7 @@ using namespace cfa_dev;
 namespace {
 
 constexpr int RED_BLOCKS = 1024;   // partial sums per reduction (grid-stride kernels)
-constexpr int OP_BLOCKS = 4096;    // grid cap of the fused operator kernels (partials <= workspace)
+constexpr int OP_BLOCKS = 4096;    // partials that one segment of the workspace holds
 constexpr int LOOKAHEAD = 3;       // iterations enqueued ahead of the last one known to have finished
 constexpr int GRAPH_CACHE = 4;     // captured iteration graphs kept per solver kind
 
@@ -744,8 +744,8 @@ k_jacobi_from_zero_check(int rows, const int* __restrict__ rp, const int* __rest
 // Last V-cycle sweep on a level 0 without coupled transfers: y = x + omega dinv (b - A x) written as
 // FP64 (the preconditioned residual z), with the r.z block partials when part is set (rdot = the FP64
 // residual r; b itself in the FP64 cycle). Row runs through LDS; the grid is capped, so that the
-// consumers' re-summation stays short. On 1.84 M rows 59 us, bound by its 215 MB; with lanes per row, whose
-// loads scatter over the rows of a wavefront, 68 us.
+// consumers' re-summation stays short. On 1.84 M rows 59 us for its 215 MB, 3.6 TB/s where a 1 GiB copy
+// reaches 5.2; with lanes per row, whose loads scatter over the rows of a wavefront, 68 us.
 template <int RB, typename T = double>
 __global__ void __launch_bounds__(BLOCK)
 k_jacobi_dot(int rows, const int* __restrict__ rp, const int* __restrict__ ci, const T* __restrict__ val,
@@ -2029,7 +2029,7 @@ __global__ void k_bicg_final_post(int nb, const double* __restrict__ part, doubl
         }
     }
     st[10] = it + 1;
-    if (act[0] || act[1])   // start of the next iteration (bicg_pre_logic)
+    if (act[0] || act[1])   // start of the next iteration
         for (int c = 0; c < 2; ++c) {
             double cb = 0.0, co = 0.0;
             if (act[c] && fabs(rho[c]) < bd[c]) {
@@ -2895,8 +2895,9 @@ int pcg_fused(int n, const int* rp, const int* ci, const double* val, const doub
     a.rbuf[1] = ws->vec[6];
     // The update in the cycle's first launch where a launch costs more than what it adds: both gathers of
     // every level-0 entry of A and W^T, and the residual test's sums in every workgroup of the next stage.
-    // Time steps merged / apart: 2.53 / 2.60 ms on 29k nodes, 4.85 / 4.74 ms on 115k. Its partials (at most
-    // one per 8 rows' lanes, 2048) fit their segment.
+    // Time steps merged / apart: 2.53 / 2.60 ms on 29k nodes, 4.85 / 4.74 ms on 115k; the line between them
+    // is not measured. Its partials, one per workgroup of tpr_a lanes a row, can be up to 16384: the check is
+    // what keeps them in their segment.
     const bool merged = amg && amg->n_levels > 0 && coupled_from(amg, 0) && n <= UPDATE_STAGE_ROWS &&
                         update_blocks(amg->levels[0]) <= OP_BLOCKS;
     // block partials: four segments of OP_BLOCKS doubles, then the prologue's (5 * 4096 of the

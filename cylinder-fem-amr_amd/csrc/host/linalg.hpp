@@ -180,8 +180,9 @@ public:
     int max_levels = 15;
     // Levels up to couple_max_rows carry the coupled transfers: below, a cycle is bound by its launches;
     // beyond, W's 11 entries per row (A has 7, P 2.7) cost more than the launches saved. Two time steps
-    // with limits 60k / 300k / 1M / 3M: level 4 (115k rows) 10.4 / 10.1 / 10.1 / 10.1 ms, level 5 (461k)
-    // 16.2 / 16.0 / 16.8 / 16.8 ms, level 6 (1.84 M) 63.3 / 63.3 / 63.5 / 69.6 ms.
+    // with limits 60k / 300k / 1M / 3M, FP64: level 4 (115k rows) 10.4 / 10.1 / 10.1 / 10.1 ms, level 5 (461k)
+    // 16.2 / 16.0 / 16.8 / 16.8 ms, level 6 (1.84 M) 63.3 / 63.3 / 63.5 / 69.6 ms. So the line lies between
+    // 115k and 461k rows; sizes between them, and the FP32 cycle, are not measured.
     int couple_max_rows = 300000;
     // The first level (from level 1) of at most dense_max_rows rows carries the dense matrix of the rest
     // of the cycle (0: none). 500 / 1000 / 1536 / 2500: level 3 (639 rows) 3.08 / 2.77 / 2.77 / 2.77 ms a

@@ -270,7 +270,8 @@ typedef struct {
      * smoothing steps) and Q = W^T, with w_v32, q_v32 their FP32 copies (use_f32). For a symmetric A
      * the restricted residual after two steps from zero is Q b, and two steps from x + P e are two
      * steps from x plus W e, so a level needs neither the residual nor its coarse correction before
-     * it smooths. NULL w_rp for none. tpr_w, tpr_q: lanes per row (powers of two up to 64). */
+     * it smooths. NULL w_rp for none. tpr_q: lanes per row of Q (a power of two up to 64); the rows of W
+     * take A's tpr_a lanes, and tpr_w is not read. */
     int tpr_w, tpr_q;
     const int* w_rp; const int* w_ci; const double* w_v; const float* w_v32;
     const int* q_rp; const int* q_ci; const double* q_v; const float* q_v32;
